@@ -2860,17 +2860,21 @@ bool narrow_path(int fmt, int64_t tokens, int32_t H, int wide_splits) {
     return H <= 32 || tokens * head_groups(H) * wide_splits < 128;
 }
 
-int auto_splits(int64_t queries, int topk) {
-    int ns = 1;
-    if (queries > 0 && queries < 256) {
-        const int64_t want = (256 + queries - 1) / queries;
-        // keep >= 4 tiles per split (at top-k 2048 and B = 2 or 4: 16 splits
-        // measured 11 % faster than 8 and 6 % faster than 32)
-        const int64_t by_len = (topk + 127) / 128;
-        ns = (int)std::min<int64_t>(want, std::max<int64_t>(1, by_len));
-    }
-    return std::min(ns, DSA_MLA_MAX_SPLITS);
+// Splits of a call whose `wgs` unsplit workgroups would leave CUs idle: as many
+// as fit one round of the 256 CUs (a workgroup takes a whole CU), with at least
+// min_entries list entries each.  A second, mostly empty round costs another
+// workgroup's fixed time (its Q load, first gathers and output) and its share of
+// the list: 2 (F + L / ceil) against F + L / floor, and ceil <= floor + 1 makes
+// the one round shorter for any F > 0.  74 query tokens of 16 heads (656-B rows,
+// 2048 entries): 3 splits 49.9 us against 4 splits (296 workgroups) 73.5 us.
+int one_round_splits(int64_t wgs, int64_t max_list, int64_t min_entries) {
+    if (wgs <= 0 || wgs >= 256) return 1;
+    const int64_t by_len = std::max<int64_t>(1, max_list / min_entries);
+    return (int)std::min<int64_t>(std::min<int64_t>(256 / wgs, by_len), DSA_MLA_MAX_SPLITS);
 }
+// decode: at least 4 tiles per split (at top-k 2048 and B = 2 or 4: 16 splits
+// measured 11 % faster than 8 and 6 % faster than 32)
+int auto_splits(int64_t queries, int topk) { return one_round_splits(queries, (int64_t)topk + 127, 128); }
 
 // Split count and kernel of a top-k decode call: the caller's count, or the
 // automatic one for the kernel narrow_path picks.
@@ -3084,11 +3088,7 @@ size_t mx_ws_bytes(const dsa_mla_decode_mxfp8_args* a, int ns) {
 // max_list entries).
 int prefill_plan(int fmt, int64_t N, int32_t H, int requested, int64_t max_list, bool* narrow);
 int prefill_splits(int requested, int64_t wgs, int64_t max_list) {
-    if (requested > 0) return requested;
-    if (wgs <= 0 || wgs >= 256) return 1;
-    const int64_t want = (256 + wgs - 1) / wgs;
-    const int64_t by_len = std::max<int64_t>(1, max_list / 256);
-    return (int)std::min<int64_t>(std::min<int64_t>(want, by_len), DSA_MLA_MAX_SPLITS);
+    return requested > 0 ? requested : one_round_splits(wgs, max_list, 256);
 }
 int prefill_plan(int fmt, int64_t N, int32_t H, int requested, int64_t max_list, bool* narrow) {
     const int wide = prefill_splits(requested, N * head_groups(H), max_list);
