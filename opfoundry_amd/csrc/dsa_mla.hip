@@ -199,6 +199,10 @@ __host__ __device__ inline int plan_item_slot(int w) { return (w & (PLAN_LAST - 
 // plan header: [0] items, [1] split rows, [2] chunk, then the B, s_q and
 // max_kv_len it was built for
 constexpr int PLAN_HDR_B = 3, PLAN_HDR_SQ = 4, PLAN_HDR_MAXLEN = 5;
+// and [6]: 1 when some row has more items than one wave merges (SMALL_SPLITS)
+constexpr int PLAN_HDR_LONG = 6;
+// splits a wave merges with all its loads in flight at once
+constexpr int SMALL_SPLITS = 16;
 
 // A global-memory pointer from its address (a generic pointer of unknown
 // origin would be accessed with flat loads).
@@ -2470,14 +2474,27 @@ dsa_mla_fwd_narrow_kernel(const FwdParams p_arg) {
 // ---------------------------------------------------------------------------
 constexpr int PLAN_TARGET = 256;     // workgroups a plan aims at: one per CU
 constexpr int PLAN_MIN_CHUNK = 128;  // entries: at least four tiles per item
-constexpr int PLAN_THREADS = 256;
+constexpr int PLAN_THREADS = 512;
+constexpr int PLAN_BLOCK = 256;      // rows laid out at a time
 
+// A call that builds its own plan waits for this kernel, one workgroup on one
+// CU: a chain of dependent steps, so it is the number of them that counts.  The
+// chunk is found by 8 waves testing 8 candidates per step (a bisection by one
+// candidate took 11 steps for a 65536-entry list, two barriers each), and the
+// items of a block of rows are written by all threads (one thread per row wrote
+// them in a loop).  8 lists of 5 to 65536 entries: 7.2 us, before 12.0.
 __global__ void __launch_bounds__(PLAN_THREADS)
 dsa_csr_plan_kernel(const int32_t* __restrict__ indptr, int B, int s_q, int max_len, int4* __restrict__ items,
                     int4* __restrict__ splits, int32_t* __restrict__ hdr) {
     constexpr int NW = PLAN_THREADS / 64;
+    constexpr int RPL = PLAN_BLOCK / 64;      // rows per lane when every wave holds a block
     __shared__ long long s_tot[NW];
-    __shared__ int s_scan[3][NW];
+    __shared__ int s_len[PLAN_BLOCK];         // entries of the block's rows (-1: longer than max_len)
+    __shared__ int s_end[PLAN_BLOCK];         // items up to and with each row of the block
+    __shared__ int s_slot[PLAN_BLOCK];        // first partial slot of each row
+    __shared__ int s_cnt[2][NW];
+    __shared__ int s_scan[3][PLAN_BLOCK / 64];
+    __shared__ int s_long;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int rows = B * s_q;
     // entries of row q; -1 for a row longer than max_len
@@ -2486,11 +2503,11 @@ dsa_csr_plan_kernel(const int32_t* __restrict__ indptr, int B, int s_q, int max_
         const int64_t L = (int64_t)indptr[b + 1] - indptr[b] - (s_q - 1 - t);
         return L > max_len ? -1 : (int)max(L, (int64_t)0);
     };
-    static_assert(PLAN_TARGET <= PLAN_THREADS, "below PLAN_TARGET rows, one row per thread");
-    const bool few = rows < PLAN_TARGET;
-    const int Lr = few && tid < rows ? len_of(tid) : 0;    // this thread's row when few
+    auto items_of = [](int L, int c) -> int { return L <= c ? 1 : (int)((unsigned)L / (unsigned)c + ((unsigned)L % (unsigned)c != 0)); };
+    static_assert(PLAN_TARGET <= PLAN_BLOCK, "below PLAN_TARGET rows, one block holds every row");
     int chunk;
-    if (!few) {
+    if (tid == 0) s_long = 0;
+    if (rows >= PLAN_TARGET) {
         long long tot = 0;
         for (int q = tid; q < rows; q += PLAN_THREADS) tot += max(len_of(q), 0);
 #pragma unroll
@@ -2503,32 +2520,41 @@ dsa_csr_plan_kernel(const int32_t* __restrict__ indptr, int B, int s_q, int max_
         c64 = (c64 + TILE - 1) / TILE * TILE;
         chunk = (int)min(c64, (long long)MAX_LIST);
     } else {
-        // Fewer rows than PLAN_TARGET (one per thread): the smallest chunk, in
-        // tiles and >= PLAN_MIN_CHUNK, whose items fit one round of
-        // PLAN_TARGET workgroups, sum over rows of ceil(L / chunk) <=
-        // PLAN_TARGET (a cut row is one item).  The count falls as chunk
-        // grows, and chunk = the longest list gives rows items: bisection.
-        __shared__ int s_cnt[NW];
-        int lmax = Lr;
+        // Fewer rows than PLAN_TARGET: the smallest chunk, in tiles and >=
+        // PLAN_MIN_CHUNK, whose items fit one round of PLAN_TARGET workgroups,
+        // sum over rows of ceil(L / chunk) <= PLAN_TARGET (a cut row is one
+        // item).  The count falls as chunk grows, and chunk = the longest list
+        // gives rows items.  Every wave holds all rows and tests a candidate of
+        // its own; a step cuts the range to a ninth.
+        if (tid < rows) s_len[tid] = len_of(tid);
+        __syncthreads();
+        int Lr[RPL], lmax = 0;
+#pragma unroll
+        for (int i = 0; i < RPL; ++i) {
+            const int q = 64 * i + lane;
+            Lr[i] = q < rows ? s_len[q] : -2;              // (-2: no row, no item)
+            lmax = max(lmax, Lr[i]);
+        }
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) lmax = max(lmax, __shfl_xor(lmax, off, 64));
-        if (lane == 0) s_cnt[wave] = lmax;
-        __syncthreads();
-        for (int w = 0; w < NW; ++w) lmax = max(lmax, s_cnt[w]);
-        __syncthreads();
         int lo = PLAN_MIN_CHUNK / TILE, hi = max(lo, (lmax + TILE - 1) / TILE);   // in tiles
-        while (lo < hi) {
-            const int mid = (lo + hi) / 2, c = mid * TILE;
-            int n = tid < rows ? (Lr <= c ? 1 : Lr / c + (Lr % c != 0)) : 0;
+        for (int step = 0; lo < hi; step ^= 1) {
+            // candidates lo + ((hi - lo) (w + 1)) / 9 of wave w, below hi, rising with w
+            const int c = (lo + (int)(((int64_t)(hi - lo) * (wave + 1)) / (NW + 1))) * TILE;
+            int n = 0;
+#pragma unroll
+            for (int i = 0; i < RPL; ++i) n += Lr[i] == -2 ? 0 : items_of(Lr[i], c);
 #pragma unroll
             for (int off = 32; off >= 1; off >>= 1) n += __shfl_xor(n, off, 64);
-            if (lane == 0) s_cnt[wave] = n;
+            if (lane == 0) s_cnt[step][wave] = n;
             __syncthreads();
-            int cnt = 0;
-            for (int w = 0; w < NW; ++w) cnt += s_cnt[w];
-            __syncthreads();
-            if (cnt <= PLAN_TARGET) hi = mid;
-            else lo = mid + 1;
+            // the first candidate that fits bounds the chunk from above, the last
+            // that does not from below (the other buffer is written next: no barrier)
+            int first = NW;
+            for (int w = NW - 1; w >= 0; --w) first = s_cnt[step][w] <= PLAN_TARGET ? w : first;
+            const int lo0 = lo, d = hi - lo;
+            if (first < NW) hi = lo0 + (int)(((int64_t)d * (first + 1)) / (NW + 1));
+            if (first > 0) lo = lo0 + (int)(((int64_t)d * first) / (NW + 1)) + 1;
         }
         chunk = lo * TILE;
     }
@@ -2541,40 +2567,50 @@ dsa_csr_plan_kernel(const int32_t* __restrict__ indptr, int B, int s_q, int max_
         return v;
     };
     int item_base = 0, slot_base = 0, split_base = 0;
-    for (int q0 = 0; q0 < rows; q0 += PLAN_THREADS) {
+    for (int q0 = 0; q0 < rows; q0 += PLAN_BLOCK) {
+        // the block's rows, one per thread of the first waves: items, partial
+        // slots and split rows up to each
         const int q = q0 + tid;
-        int L = 0, n = 0;
-        if (q < rows) {
-            L = few ? Lr : len_of(q);
-            n = L <= chunk ? 1 : L / chunk + (L % chunk != 0);
-        }
+        const bool mine = tid < PLAN_BLOCK && q < rows;
+        const int L = mine ? (rows < PLAN_TARGET ? s_len[tid] : len_of(q)) : 0;
+        const int n = mine ? items_of(L, chunk) : 0;
         const int ns = n > 1 ? n : 0, sp = n > 1 ? 1 : 0;
         const int ia = wave_incl(n), ic = wave_incl(ns), id = wave_incl(sp);
-        if (lane == 63) {
+        __syncthreads();    // the last block's items are written
+        if (lane == 63 && tid < PLAN_BLOCK) {
             s_scan[0][wave] = ia;
             s_scan[1][wave] = ic;
             s_scan[2][wave] = id;
         }
         __syncthreads();
         int wa = 0, wc = 0, wd = 0, ta = 0, tc = 0, td = 0;
-        for (int w = 0; w < NW; ++w) {
+        for (int w = 0; w < PLAN_BLOCK / 64; ++w) {
             const int x = s_scan[0][w], y = s_scan[1][w], z = s_scan[2][w];
             if (w < wave) { wa += x; wc += y; wd += z; }
             ta += x; tc += y; td += z;
         }
-        const int ib = item_base + wa + ia - n;
-        const int sb = slot_base + wc + ic - ns;
-        const int pb = split_base + wd + id - sp;
-        for (int j = 0; j < n; ++j) {
-            const int e0 = L < 0 ? 0 : j * chunk;
-            const int e1 = L < 0 ? 0 : (int)min((int64_t)(j + 1) * chunk, (int64_t)L);
-            items[ib + j] = make_int4(q, e0, e1, plan_item_w(n > 1 ? sb + j : -1, j == n - 1));
+        if (tid < PLAN_BLOCK) {
+            s_len[tid] = L;
+            s_end[tid] = wa + ia;
+            s_slot[tid] = slot_base + wc + ic - ns;
+            if (n > 1) splits[split_base + wd + id - sp] = make_int4(q, slot_base + wc + ic - ns, n, 0);
+            if (n > SMALL_SPLITS) s_long = 1;
         }
-        if (n > 1) splits[pb] = make_int4(q, sb, n, 0);
+        __syncthreads();
+        // item i of the block belongs to the first row whose s_end exceeds i
+        for (int i = tid; i < ta; i += PLAN_THREADS) {
+            int r = 0;
+#pragma unroll
+            for (int half = PLAN_BLOCK / 2; half >= 1; half >>= 1)
+                if (s_end[r + half - 1] <= i) r += half;
+            const int rl = s_len[r], rn = items_of(rl, chunk), j = i - (s_end[r] - rn);
+            const int e0 = rl < 0 ? 0 : j * chunk;
+            const int e1 = rl < 0 ? 0 : (int)min((int64_t)(j + 1) * chunk, (int64_t)rl);
+            items[item_base + i] = make_int4(q0 + r, e0, e1, plan_item_w(rn > 1 ? s_slot[r] + j : -1, j == rn - 1));
+        }
         item_base += ta;
         slot_base += tc;
         split_base += td;
-        __syncthreads();    // s_scan is rewritten by the next round
     }
     if (tid == 0) {
         hdr[0] = item_base;
@@ -2583,6 +2619,7 @@ dsa_csr_plan_kernel(const int32_t* __restrict__ indptr, int B, int s_q, int max_
         hdr[PLAN_HDR_B] = B;
         hdr[PLAN_HDR_SQ] = s_q;
         hdr[PLAN_HDR_MAXLEN] = max_len;
+        hdr[PLAN_HDR_LONG] = s_long;           // (written before the last block's barrier)
     }
 }
 
@@ -2593,8 +2630,6 @@ dsa_csr_plan_kernel(const int32_t* __restrict__ indptr, int B, int s_q, int max_
 // m = max(lse_i, sink), den = sum w_i + exp(sink - m), so a sink far above
 // or below every score neither overflows nor underflows.  A row with no
 // attended entry keeps O = 0 and LSE = +inf, as unsplit.
-// splits a wave merges with all its loads in flight at once
-constexpr int SMALL_SPLITS = 16;
 __device__ __forceinline__ void combine_head(const float* __restrict__ part_o, const float* __restrict__ part_lse,
                                              int ns, int64_t first, int64_t step_rows, int row, int head, int H,
                                              int s_q, __bf16* __restrict__ out, int64_t o_sb, int64_t o_st,
@@ -2700,31 +2735,108 @@ dsa_mla_combine_kernel(const float* __restrict__ part_o, const float* __restrict
                      threadIdx.x & 63);
 }
 
+// The same for a row of many splits, one (query row, head) on the four waves of a
+// workgroup: each wave merges a quarter of the splits, all against the row's
+// maximum, and the four sums meet in LDS (red: 4 x 512 floats, then 4
+// denominators).  One wave per head would pay a memory round trip per eight
+// splits, and a plan's few long rows leave too few waves to hide them.
+__device__ __forceinline__ void combine_head_wide(const float* __restrict__ part_o, const float* __restrict__ part_lse,
+                                                  int ns, int64_t first, int row, int head, int H, int s_q,
+                                                  __bf16* __restrict__ out, int64_t o_sb, int64_t o_st, int64_t o_sh,
+                                                  float* __restrict__ lse, LDS_AS float* red) {
+    constexpr int FLIGHT = 8;                  // splits a wave loads at a time
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t base = first * H + head;     // partial index of split 0
+    const int per = (ns + 3) / 4, s0 = wave * per, s1 = min(ns, s0 + per);
+    f32x4 v[FLIGHT][2];
+    float ls[FLIGHT];
+    auto load = [&](int s) {
+#pragma unroll
+        for (int j = 0; j < FLIGHT; ++j) {
+            if (s + j < s1) {
+                const int64_t i = base + (int64_t)(s + j) * H;
+                ls[j] = part_lse[i];
+                const f32x4* src = reinterpret_cast<const f32x4*>(part_o + i * D_VO + 8 * lane);
+                v[j][0] = src[0];
+                v[j][1] = src[1];
+            }
+        }
+    };
+    load(s0);                                  // in flight with the LSEs of every split
+    float m = -FLT_MAX;
+    for (int s = lane; s < ns; s += 64) m = fmaxf(m, part_lse[base + (int64_t)s * H]);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+    f32x4 acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
+    float den = 0.0f;
+    for (int s = s0; s < s1; s += FLIGHT) {
+        if (s > s0) load(s);
+#pragma unroll
+        for (int j = 0; j < FLIGHT; ++j) {
+            if (s + j < s1) {
+                const float w = ls[j] > -FLT_MAX || ls[j] != ls[j] ? __builtin_amdgcn_exp2f((ls[j] - m) * LOG2E) : 0.0f;
+                den += w;
+                acc0 += w * v[j][0];
+                acc1 += w * v[j][1];
+            }
+        }
+    }
+    __syncthreads();                           // the last unit's sums are read
+    LDS_AS f32x4* const dst = (LDS_AS f32x4*)(red + wave * D_VO + 8 * lane);
+    dst[0] = acc0;
+    dst[1] = acc1;
+    if (lane == 0) red[4 * D_VO + wave] = den;
+    __syncthreads();
+    const float all = (red[4 * D_VO] + red[4 * D_VO + 1]) + (red[4 * D_VO + 2] + red[4 * D_VO + 3]);
+    const float inv = all > 0.0f ? 1.0f / all : 0.0f;
+    f32x2 o = {0, 0};                          // outputs 2 tid, 2 tid + 1
+#pragma unroll
+    for (int w = 0; w < 4; ++w) o += *(const LDS_AS f32x2*)(red + w * D_VO + 2 * tid);
+    __bf16* op = out + (int64_t)(row / s_q) * o_sb + (int64_t)(row % s_q) * o_st + (int64_t)head * o_sh + 2 * tid;
+    *reinterpret_cast<bf16x2*>(op) = __builtin_convertvector(o * inv, bf16x2);
+    if (lse && tid == 0)
+        lse[(int64_t)row * H + head] = all > 0.0f || all != all ? m + __builtin_amdgcn_logf(all) * LN2 : INFINITY;
+}
+
 // The split rows of a CSR work plan: map[i] = (query row, first partial row,
-// count), consecutive partial rows, hdr[1] rows listed.  A fixed grid walks
-// the hdr[1] x ceil(H / 4) units of four heads, so a plan without split rows
-// costs one wave of empty workgroups, not a workgroup per possible unit.
+// count), consecutive partial rows, hdr[1] rows listed.  A fixed grid walks them,
+// so a plan without split rows costs one wave of empty workgroups, not a
+// workgroup per possible unit: rows of up to SMALL_SPLITS items in units of four
+// heads, a wave each (one memory round trip), longer rows in units of one head,
+// on the whole workgroup.  8 rows of 33 items, 128 heads: 13.8 us, 67 MB of
+// partials at 4.9 TB/s, against 15.2 with a wave per head; 2 rows of 128 items of
+// 64 heads, where few waves hide their round trips: the whole call 44.5 us
+// against 61.6.
 __global__ void __launch_bounds__(256)
 dsa_mla_combine_plan_kernel(const float* __restrict__ part_o, const float* __restrict__ part_lse, int B, int H,
                             int s_q, int max_len, __bf16* __restrict__ out, int64_t o_sb, int64_t o_st,
                             int64_t o_sh, float* __restrict__ lse, const int4* __restrict__ map,
                             const int32_t* __restrict__ hdr) {
+    __shared__ __attribute__((aligned(16))) float s_red[4 * D_VO + 4];
     // a plan built for other arguments: the forward kernel has written NaN rows
     if (__builtin_amdgcn_readfirstlane(hdr[PLAN_HDR_B]) != B ||
         __builtin_amdgcn_readfirstlane(hdr[PLAN_HDR_SQ]) != s_q ||
         __builtin_amdgcn_readfirstlane(hdr[PLAN_HDR_MAXLEN]) != max_len)
         return;
+    const int rows = __builtin_amdgcn_readfirstlane(hdr[1]);
     const int hq = (H + 3) / 4;
-    const int units = __builtin_amdgcn_readfirstlane(hdr[1]) * hq;
     const int wave = threadIdx.x >> 6;
-    for (int u = blockIdx.x; u < units; u += gridDim.x) {
+    // (fewer than 256 rows, and partial rows that memory holds: rows * H fits int32)
+    for (int u = blockIdx.x; u < rows * hq; u += gridDim.x) {
         const int r = u / hq;
         const int head = (u - r * hq) * 4 + wave;
-        if (head < H) {
-            const int4 m = map[r];
+        const int4 m = map[r];
+        if (head < H && m.z <= SMALL_SPLITS)
             combine_head(part_o, part_lse, m.z, m.y, 1, m.x, head, H, s_q, out, o_sb, o_st, o_sh, lse, nullptr,
                          threadIdx.x & 63);
-        }
+    }
+    if (!__builtin_amdgcn_readfirstlane(hdr[PLAN_HDR_LONG])) return;
+    for (int u = blockIdx.x; u < rows * H; u += gridDim.x) {
+        const int r = u / H;
+        const int4 m = map[r];
+        if (__builtin_amdgcn_readfirstlane(m.z) > SMALL_SPLITS)
+            combine_head_wide(part_o, part_lse, __builtin_amdgcn_readfirstlane(m.z), m.y, m.x,
+                              u - r * H, H, s_q, out, o_sb, o_st, o_sh, lse, (LDS_AS float*)s_red);
     }
 }
 
