@@ -44,19 +44,25 @@ SM_SCALE = 1.0 / math.sqrt(192.0)
 FLOP_PER_PAIR = 2 * H * (D_QK + D_VO)
 
 
+def _fwd_kernel(name, tokens, splits, heads):
+    """The library's rule: 32-head workgroups when heads <= 64 or when the 128-head kernel
+    would run fewer than 128 workgroups, two to a CU (pair) when they outnumber the CUs, else
+    one (narrow); else 128-head workgroups.  (splits: the split count the call runs with.)"""
+    groups = (heads + 31) // 32
+    if heads <= 64 or tokens * ((heads + 127) // 128) * splits < 128:
+        kind = "pair" if tokens * groups * splits > 256 else "narrow"
+        return f"dsa_mla_fwd_{kind}_kernel<{name}>"
+    return f"dsa_mla_fwd_kernel<{name}>"
+
+
 def bf16_fwd_kernel(tokens, splits, heads=H, d512=False):
-    """Name of the forward kernel the library runs for bf16 rows: 32-head workgroups when
-    heads <= 32 or when the 128-head kernel would run fewer than 128 workgroups, else the
-    128-head one.  (splits: the 128-head kernel's split count.)"""
-    narrow = heads <= 32 or tokens * ((heads + 127) // 128) * splits < 128
-    if narrow:
-        return "dsa_mla_fwd_narrow_kernel<" + ("512" if d512 else "576") + ">"
-    return "dsa_mla_fwd_kernel<" + ("bf16_d512" if d512 else "bf16") + ">"
+    """Name of the forward kernel the library runs for bf16 rows."""
+    return _fwd_kernel("bf16_d512" if d512 else "bf16", tokens, splits, heads)
+
 
 def fp8_fwd_kernel(tokens, splits, heads=H):
-    """The same for 656-B fp8 rows (the same selection rule)."""
-    narrow = heads <= 32 or tokens * ((heads + 127) // 128) * splits < 128
-    return "dsa_mla_fwd_narrow_kernel<fp8>" if narrow else "dsa_mla_fwd_kernel<fp8>"
+    """The same for 656-B fp8 rows."""
+    return _fwd_kernel("fp8", tokens, splits, heads)
 
 
 CONFIGS = {
@@ -1400,7 +1406,7 @@ def c5_leg(args, dev, res):
                                    "kernel_avg_us": round(pk_ms * 1e3, 1)}}
     defer_cpu(args, "CPU baseline (oracle) on a c5 sample", res["prefill"],
               lambda: cpu_baseline_prefill(p, args.cpu_prefill_sample, pV))
-    # The c5 lists with fewer heads (the first H heads of c5's Q): H <= 32 runs on 32-head
+    # The c5 lists with fewer heads (the first H heads of c5's Q): H <= 64 runs on 32-head
     # workgroups, H = 64 on 128-head ones; the fraction is of useful flops (H heads).
     import torch
     from opfoundry_amd import dsa

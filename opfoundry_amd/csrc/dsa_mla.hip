@@ -2442,6 +2442,814 @@ dsa_mla_fwd_narrow_kernel(const FwdParams p_arg) {
 }
 
 // ---------------------------------------------------------------------------
+// Pair kernel: 32 heads per workgroup, two workgroups per CU.  For calls of
+// many 32-head workgroups (small head counts at batch, prefill of up to 64
+// heads): the narrow kernel's phases (gather, QK^T, softmax, PV) follow one
+// another on one wave per SIMD, each waiting on LDS or a barrier with nothing
+// else to run; a second workgroup on the CU fills those waits.  That asks for
+// half the LDS (80 KB) and 256 registers per wave:
+//   bf16 rows     two tile slots instead of three
+//   fp8 rows      two raw slots and ONE 16-bit tile buffer: a tile is converted
+//                 once every wave is done with the last one (three barriers per
+//                 tile instead of two); RoPE is read from the raw slot
+//   row list      512 to 2048 entries at a time, as the format leaves room
+// Tile rows are 1040 bytes apart (a 16-byte pad: 16 rows start at 16 distinct
+// 16-byte bank groups), and a row's 16-byte chunk c sits at c ^ 4 (r & 3), so
+// that the transposed V reads (4 rows x 4 chunks) are spread as well.
+// Formats: those of the narrow kernel, MXFP8 split streams and V4 fp8 rows (both
+// converted exactly to bf16); index forms: top-k, CSR with uniform splits or a
+// work plan, V4.  Arithmetic per tile as in dsa_mla_fwd_narrow_kernel.
+// Bound by the LDS and VALU work of both workgroups.  Against the narrow kernel:
+// 4096 queries x 2048 bf16 rows, H = 16, 747 us instead of 1226; 2048 queries of
+// 656-B rows, H = 32, 549 instead of 835.  Against 128-head workgroups (the other
+// 64 or more heads padding): MXFP8, 128 tokens x 2048 rows, H = 16, 67 instead of
+// 86; V4 fp8 rows, 2048 queries x 1152, H = 16, 389 instead of 701.
+// grid = (tokens or plan items x ceil(H / 32), s_q, num_splits), block = 256.
+// ---------------------------------------------------------------------------
+template <int NF>
+struct PairLay {
+    static constexpr bool F16 = NF == DSA_KV_FP8_656;
+    static constexpr bool V4MX = NF == DSA_KV_MXFP8_V4;
+    static constexpr bool MX = NF == DSA_KV_MXFP8 || V4MX;
+    static constexpr bool RAW = F16 || MX;                        // raw slots, converted into one tile buffer
+    static constexpr bool D512 = NF == DSA_KV_BF16_D512 || V4MX;  // K = V = 512 values
+    static constexpr int NKS = (D512 ? D_NOPE : D_QK) / 32;       // 32-deep k-steps of QK^T
+    static constexpr int Q8_KS = V4MX ? DSA_MLA_V4_NOPE / 32 : D_NOPE / 32;   // k-steps from the fp8 stream (MX)
+    static constexpr int STRIDE = 2 * D_NOPE + 16;
+    static constexpr int ROPE = TILE * STRIDE;                    // bf16 576-value rows: RoPE rows behind the NoPE rows
+    static constexpr int SLOT = ROPE + (RAW || D512 ? 0 : TILE * 128);
+    static constexpr int LOADS = V4MX ? 20 : 21;                  // LDS-DMA loads per raw tile; load 20 is half a load
+    static constexpr int RAWB = V4MX ? 20480 : 20992;
+    static constexpr int TILE0 = RAW ? 2 * RAWB : 0;
+    static constexpr int PXO = TILE0 + (RAW ? 1 : 2) * SLOT;
+    static constexpr int REDO = PXO + P_BYTES;
+    static constexpr int MISCO = REDO + 4 * (4 * 2 * NARROW_HEADS + NARROW_HEADS);
+    static constexpr int ROWSO = MISCO + 32;
+    // entries of a chunk (a multiple of the workgroup's threads)
+    static constexpr int MC = V4MX ? 1024 : (D512 ? 2048 : (RAW ? 512 : 768));
+    static constexpr int BYTES = ROWSO + 4 * MC;
+    static_assert(BYTES <= 81920, "two workgroups share a CU's 160 KB of LDS");
+    static_assert(RAWB % 16 == 0 && STRIDE % 16 == 0, "16-byte LDS-DMA destinations");
+    static constexpr float TAU = F16 ? 15.0f : 100.0f;
+};
+
+template <int NF>
+__global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2, 2)))
+dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
+    using L = PairLay<NF>;
+    constexpr bool D512 = L::D512, F16 = L::F16, RAW = L::RAW;
+    __shared__ __attribute__((aligned(1024))) unsigned char s_pool[L::BYTES];
+    const lds_ptr POOL = (lds_ptr)s_pool;
+    const lds_ptr PX = POOL + L::PXO;
+    LDS_AS int32_t* const s_rows = (LDS_AS int32_t*)(POOL + L::ROWSO);
+    LDS_AS float* const s_red = (LDS_AS float*)(POOL + L::REDO);
+    LDS_AS int* const s_misc = (LDS_AS int*)(POOL + L::MISCO);   // [0..3] wave counts, [4] restart, [5] bad scale
+    // the arguments the prologue reads, copied into registers in one batch (see
+    // dsa_mla_fwd_narrow_kernel)
+    FwdParams p = p_arg;
+    unsigned grid_x = gridDim.x, grid_z = gridDim.z;
+    uintptr_t a_q = (uintptr_t)p.q, a_bt = (uintptr_t)p.block_table, a_sl = (uintptr_t)p.seq_lens,
+              a_ix = (uintptr_t)p.indices, a_ip = (uintptr_t)p.kv_indptr, a_ki = (uintptr_t)p.kv_indices,
+              a_pi = (uintptr_t)p.plan_items, a_ph = (uintptr_t)p.plan_hdr;
+    uintptr_t a_o = (uintptr_t)p.out, a_lse = (uintptr_t)p.lse, a_po = (uintptr_t)p.part_o, a_pl = (uintptr_t)p.part_lse;
+    asm volatile(""
+                 : "+s"(grid_x), "+s"(grid_z), "+s"(a_q), "+s"(a_bt), "+s"(a_sl), "+s"(a_ix), "+s"(a_ip), "+s"(a_ki),
+                   "+s"(p.q_sb), "+s"(p.q_st), "+s"(p.q_sh), "+s"(p.kv_total_rows), "+s"(p.kv_batch_stride),
+                   "+s"(p.bt_stride), "+s"(p.block_size), "+s"(p.bs_shift), "+s"(p.seq_len_default), "+s"(p.idx_sb),
+                   "+s"(p.idx_st), "+s"(p.s_q), "+s"(p.topk), "+s"(p.chunk), "+s"(p.H), "+s"(p.hgroups),
+                   "+s"(p.causal), "+s"(p.causal_offset), "+s"(p.reverse), "+s"(a_o), "+s"(p.o_sb), "+s"(p.o_st),
+                   "+s"(p.o_sh), "+s"(a_lse), "+s"(a_po), "+s"(a_pl), "+s"(a_pi), "+s"(a_ph));
+    if constexpr (D512) {
+        uintptr_t a_np = (uintptr_t)p.ind_pre, a_xp = (uintptr_t)p.idx_pre, a_ne = (uintptr_t)p.ind_ext,
+                  a_xe = (uintptr_t)p.idx_ext, a_sk = (uintptr_t)p.attn_sink;
+        asm volatile("" : "+s"(a_np), "+s"(a_xp), "+s"(a_ne), "+s"(a_xe), "+s"(a_sk), "+s"(p.kv2_rows));
+        p.ind_pre = gptr<const int32_t>(a_np);
+        p.idx_pre = gptr<const int32_t>(a_xp);
+        p.ind_ext = gptr<const int32_t>(a_ne);
+        p.idx_ext = gptr<const int32_t>(a_xe);
+        p.attn_sink = gptr<const float>(a_sk);
+    }
+    uintptr_t a_q8 = (uintptr_t)p.q8, a_qs = (uintptr_t)p.qsc;
+    if constexpr (L::MX) {
+        asm volatile("" : "+s"(a_q8), "+s"(a_qs), "+s"(p.q8_sb), "+s"(p.q8_st), "+s"(p.q8_sh), "+s"(p.qsc_sb),
+                          "+s"(p.qsc_st), "+s"(p.qsc_sh));
+        p.q8 = gptr<const unsigned char>(a_q8);
+        p.qsc = gptr<const unsigned char>(a_qs);
+    }
+    p.out = gptr<__bf16>(a_o);
+    p.lse = gptr<float>(a_lse);
+    p.part_o = gptr<float>(a_po);
+    p.part_lse = gptr<float>(a_pl);
+    p.q = gptr<const __bf16>(a_q);
+    p.block_table = gptr<const int32_t>(a_bt);
+    p.seq_lens = gptr<const int32_t>(a_sl);
+    p.indices = gptr<const int32_t>(a_ix);
+    p.kv_indptr = gptr<const int32_t>(a_ip);
+    p.kv_indices = gptr<const int32_t>(a_ki);
+    p.plan_items = gptr<const int4>(a_pi);
+    p.plan_hdr = gptr<const int32_t>(a_ph);
+
+    // Work unit (query token or plan item) and head group.  Workgroups go to the
+    // 8 XCDs in turn: the head groups of a unit are 8 apart, so that they run on
+    // one XCD at about the same time and its L2 fetches the unit's rows once.
+    const int units = (int)(grid_x / (unsigned)p.hgroups);
+    int gx = (int)blockIdx.x, hg = 0;
+    if (p.hgroups > 1) {
+        const int whole = units / 8 * 8 * p.hgroups;       // the last units % 8 are taken group by group
+        if (gx < whole) {
+            const int blk = gx / (8 * p.hgroups), rem = gx - blk * 8 * p.hgroups;
+            hg = rem >> 3;
+            gx = 8 * blk + (rem & 7);
+        } else {
+            const int i = gx - whole;
+            hg = i % p.hgroups;
+            gx = units / 8 * 8 + i / p.hgroups;
+        }
+    }
+    const int hbase = NARROW_HEADS * hg;
+    int b = p.reverse ? units - 1 - gx : gx, t = blockIdx.y;
+    const int split = blockIdx.z;
+    int item_k0 = 0, item_k1 = 0, item_slot = -1;
+    bool item_last = false;
+    if (!D512 && p.plan_items) {
+        // The plan must be the one built for this call's kv_indptr, B, s_q and
+        // max_kv_len, else every query row's outputs are NaN and nothing else is
+        // read or written (as in dsa_mla_fwd_kernel).
+        const int32_t hdr_items = sload(p.plan_hdr), hdr_b = sload(p.plan_hdr + PLAN_HDR_B),
+                      hdr_sq = sload(p.plan_hdr + PLAN_HDR_SQ), hdr_len = sload(p.plan_hdr + PLAN_HDR_MAXLEN);
+        if ((hdr_b != p.B) | (hdr_sq != p.s_q) | (hdr_len != p.chunk)) {
+            // (the grid holds at least B * s_q units)
+            if (gx < p.B * p.s_q) {
+                const int bq = gx / p.s_q, tq = gx - bq * p.s_q;
+                __bf16* const orow = p.out + (int64_t)bq * p.o_sb + (int64_t)tq * p.o_st;
+                const unsigned nan2 = 0x7FC07FC0u;    // two bf16 NaNs
+                for (int i = (int)threadIdx.x; i < NARROW_HEADS * (D_VO / 4); i += NTHR) {
+                    const int hh = hbase + i / (D_VO / 4);
+                    if (hh < p.H)
+                        reinterpret_cast<u32x2*>(orow + (int64_t)hh * p.o_sh)[i % (D_VO / 4)] = u32x2{nan2, nan2};
+                }
+                for (int hh = (int)threadIdx.x; hh < NARROW_HEADS; hh += NTHR)
+                    if (p.lse && hbase + hh < p.H) p.lse[(int64_t)gx * p.H + hbase + hh] = __builtin_nanf("");
+            }
+            return;
+        }
+        // the s_q rows of a batch (one list) on one XCD: unit 8 s_q j + r takes
+        // item 8 s_q j + s_q (r mod 8) + r / 8, as in dsa_mla_fwd_kernel
+        const int G = 8 * p.s_q, j = gx / G, rem = gx - j * G;
+        const int item = G * j + p.s_q * (rem & 7) + (rem >> 3);
+        if (item >= hdr_items) return;                 // the whole workgroup, before any barrier
+        const int4 w = p.plan_items[item];
+        const int qrow_i = __builtin_amdgcn_readfirstlane(w.x);
+        if ((unsigned)qrow_i >= (unsigned)(p.B * p.s_q)) return;
+        b = qrow_i / p.s_q;
+        t = qrow_i - b * p.s_q;
+        item_k0 = __builtin_amdgcn_readfirstlane(w.y);
+        item_k1 = __builtin_amdgcn_readfirstlane(w.z);
+        const int ww = __builtin_amdgcn_readfirstlane(w.w);
+        item_slot = plan_item_slot(ww);
+        item_last = (ww & PLAN_LAST) != 0;
+    }
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rb = wave & 1, hb = wave >> 1;      // QK^T: row half, head half
+    const int c16 = lane & 15, g4 = lane >> 4;    // 16x16 operand lanes
+    const int hi = lane >> 5, r32 = lane & 31;    // PV and epilogue lanes: head r32
+    const int hq = 16 * hb + c16;                 // this lane's head in QK^T and the softmax
+    const int head_g = hbase + r32;               // heads past H: a copy of head H-1, never stored
+    if (tid == 0) {
+        s_misc[NWAVE] = 0;
+        s_misc[NWAVE + 1] = 0;
+    }
+
+    // ---- this split's entries, by the rules of dsa_mla_fwd_kernel ----
+    int k0 = !D512 && p.plan_items ? item_k0 : split * p.chunk;
+    int k1;
+    const int32_t* idx;
+    bool truncated = false;
+    int64_t v4_np = 0, v4_eb = 0;
+    if constexpr (D512) {
+        const int64_t pb = sload(p.ind_pre + b);
+        v4_np = max((int64_t)sload(p.ind_pre + b + 1) - pb, (int64_t)0);
+        v4_eb = sload(p.ind_ext + b);
+        const int64_t ne = max((int64_t)sload(p.ind_ext + b + 1) - v4_eb, (int64_t)0);
+        const int64_t n_b = min(v4_np + ne, (int64_t)p.topk);
+        truncated = v4_np + ne > p.topk;
+        const int64_t per = (n_b + grid_z - 1) / grid_z;
+        const int64_t cb = (per + TILE - 1) / TILE * TILE;
+        k0 = (int)min((int64_t)split * cb, n_b);
+        k1 = (int)min((int64_t)k0 + cb, n_b);
+        idx = p.idx_pre + pb;
+    } else if (p.kv_indptr) {
+        const int64_t kb = sload(p.kv_indptr + b);
+        const int64_t count = (int64_t)sload(p.kv_indptr + b + 1) - kb - (p.s_q - 1 - t);
+        k1 = (int)min(p.plan_items ? (int64_t)item_k1 : (int64_t)k0 + p.chunk, count);
+        // a list longer than the splits cover (max_kv_len) is cut: NaN; so is a
+        // row whose last item no longer ends at its list's length
+        truncated = count > (int64_t)grid_z * p.chunk;
+        if (item_last && (int64_t)item_k1 != max(count, (int64_t)0)) truncated = true;
+        idx = p.kv_indices + kb;
+    } else {
+        k1 = (int)min((int64_t)k0 + p.chunk, (int64_t)p.topk);
+        idx = p.indices + (int64_t)b * p.idx_sb + (int64_t)t * p.idx_st;
+    }
+    constexpr int MC = L::MC, PER_T = MC / NTHR;
+    const int nchunks = k1 > k0 ? (k1 - k0 + MC - 1) / MC : 1;
+    // the entries of chunk c (-1 past the split's end); V4: entry k is an
+    // extend entry from k = v4_np on
+    auto load_entries = [&](int c, int32_t (&jv)[PER_T]) {
+        const int kc0 = k0 + c * MC;
+        const int kc1 = min(kc0 + MC, k1);
+#pragma unroll
+        for (int e = 0; e < PER_T; ++e) {
+            const int k = kc0 + tid * PER_T + e;
+            if (D512 && k >= v4_np) jv[e] = k < kc1 ? p.idx_ext[v4_eb + (k - v4_np)] : -1;
+            else jv[e] = k < kc1 ? idx[k] : -1;
+        }
+    };
+    // chunk 0's entries, and a paged list's block-table reads for them, before Q:
+    // vmcnt counts in order, so waiting for them does not wait for Q
+    int32_t jv0[PER_T], ent0[PER_T];
+    load_entries(0, jv0);
+    int64_t jmax = 0;
+    const bool topk_form = !D512 && !p.kv_indptr;
+    if (topk_form) {
+        const int64_t Lq = p.seq_lens ? (int64_t)sload(p.seq_lens + b) : p.seq_len_default;
+        jmax = Lq;
+        if (p.causal == 1) jmax = min(Lq, Lq - p.s_q + t + 1);
+        else if (p.causal == 2) jmax = min(Lq, (int64_t)b + p.causal_offset + 1);
+    }
+    const bool topk_paged = topk_form && p.block_table;
+    if (topk_paged) topk_ents(p, b, jmax, jv0, ent0);
+
+    // ---- Q fragments (B operand of S^T = K Q^T): head hq, dims 32 ks + 8 g4 .. +7 ----
+    u32x4 qf[L::NKS];
+    u32x4 q_scales = {0, 0, 0, 0};                // MX: the E8M0 scales of the head's Q, block ks in k-step ks
+    {
+        const int64_t head_q = min(hbase + hq, p.H - 1);
+        if constexpr (L::MX) {
+            const unsigned char* q8p = p.q8 + (int64_t)b * p.q8_sb + (int64_t)t * p.q8_st + head_q * p.q8_sh + 8 * g4;
+#pragma unroll
+            for (int ks = 0; ks < L::Q8_KS; ++ks) {
+                const u32x2 c = *reinterpret_cast<const u32x2*>(q8p + 32 * ks);
+                qf[ks] = u32x4{c[0], c[1], 0u, 0u};
+            }
+            q_scales = *reinterpret_cast<const u32x4*>(p.qsc + (int64_t)b * p.qsc_sb + (int64_t)t * p.qsc_st +
+                                                       head_q * p.qsc_sh);
+        }
+        constexpr int K0 = L::MX ? L::Q8_KS : 0;  // first k-step of the bf16 part
+        const __bf16* qp = p.q + (int64_t)b * p.q_sb + (int64_t)t * p.q_st + head_q * p.q_sh + 8 * g4;
+#pragma unroll
+        for (int ks = K0; ks < L::NKS; ++ks) qf[ks] = *reinterpret_cast<const u32x4*>(qp + 32 * (ks - K0));
+    }
+    float c_s = p.scale_log2;                     // softmax scale (log2 units) of head hq
+    // Q once it has landed: MX codes to bf16 (exact); 656-B rows: NoPE to fp16
+    // with the head's power-of-two prescale (see dsa_mla_fwd_narrow_kernel)
+    auto convert_q = [&]() {
+        if constexpr (L::MX) {
+#pragma unroll
+            for (int ks = 0; ks < L::Q8_KS; ++ks)
+                qf[ks] = mx_to_bf16(qf[ks][0], qf[ks][1], (q_scales[ks >> 2] >> (8 * (ks & 3))) & 0xFFu);
+        } else if constexpr (F16) {
+            typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+            u16x2 amax = {0, 0};
+#pragma unroll
+            for (int ks = 0; ks < KS_NOPE / 2; ++ks)
+#pragma unroll
+                for (int w = 0; w < 4; ++w)
+                    amax = __builtin_elementwise_max(amax, __builtin_bit_cast(u16x2, qf[ks][w] & 0x7FFF7FFFu));
+            int eb = max((int)amax[0], (int)amax[1]) >> 7;   // biased exponent of the head's largest |q|
+            eb = max(eb, __shfl_xor(eb, 16, 64));
+            eb = max(eb, __shfl_xor(eb, 32, 64));
+            const int k = max(eb - 141, 0);                  // 141 = 127 + 14
+            const float s = __uint_as_float((unsigned)(127 - k) << 23);
+            c_s = p.scale_log2 * __uint_as_float((unsigned)(127 + k) << 23);
+#pragma unroll
+            for (int ks = 0; ks < KS_NOPE / 2; ++ks)
+#pragma unroll
+                for (int w = 0; w < 4; ++w) qf[ks][w] = bf16x2_to_f16x2(qf[ks][w], s);
+#pragma unroll
+            for (int ks = KS_NOPE / 2; ks < L::NKS; ++ks)
+#pragma unroll
+                for (int w = 0; w < 4; ++w) qf[ks][w] = bf16x2_scale(qf[ks][w], s);
+        }
+    };
+
+    // entries of chunk c -> the compacted row list, the last tile padded with
+    // copies of the first valid row (ends with a barrier)
+    int n_valid = 0, ntiles = 0;
+    bool any_rows = false;
+    auto resolve_chunk = [&](int c, bool preloaded) {
+        int32_t rows_local[PER_T];
+        int cnt = 0;
+        {
+            int32_t jv[PER_T];
+            if (preloaded) {
+#pragma unroll
+                for (int e = 0; e < PER_T; ++e) jv[e] = jv0[e];
+            } else {
+                load_entries(c, jv);
+            }
+            if constexpr (D512) {
+                const int kc0 = k0 + c * MC;
+#pragma unroll
+                for (int e = 0; e < PER_T; ++e)
+                    rows_local[e] = kc0 + tid * PER_T + e >= v4_np ? dsa_rows::v4_extend_row(jv[e], p.kv2_rows)
+                                                                   : dsa_rows::v4_prefix_row(jv[e], p.kv_total_rows);
+            } else if (p.kv_indptr) {
+#pragma unroll
+                for (int e = 0; e < PER_T; ++e) rows_local[e] = dsa_rows::csr_row(jv[e], p.kv_total_rows);
+            } else {
+                int32_t ent[PER_T];
+                if (preloaded && topk_paged) {
+#pragma unroll
+                    for (int e = 0; e < PER_T; ++e) ent[e] = ent0[e];
+                } else {
+                    topk_ents(p, b, jmax, jv, ent);
+                }
+                topk_rows_of(p, b, jv, ent, rows_local);
+            }
+#pragma unroll
+            for (int e = 0; e < PER_T; ++e) cnt += rows_local[e] >= 0 ? 1 : 0;
+        }
+        const int incl = wave_incl_sum16(cnt);
+        // (the barrier also ends every wave's use of the previous chunk's row
+        // list, tile buffers and P)
+        if (lane == 63) s_misc[wave] = incl;
+        __syncthreads();
+        int wbase = 0, nv = 0;
+#pragma unroll
+        for (int w = 0; w < NWAVE; ++w) {
+            const int s = s_misc[w];
+            wbase += w < wave ? s : 0;
+            nv += s;
+        }
+        {
+            int pos = wbase + incl - cnt;
+#pragma unroll
+            for (int e = 0; e < PER_T; ++e)
+                if (rows_local[e] >= 0) s_rows[pos++] = rows_local[e];
+        }
+        n_valid = __builtin_amdgcn_readfirstlane(nv);
+        ntiles = (n_valid + TILE - 1) / TILE;
+        any_rows = any_rows || nv > 0;
+        __syncthreads();
+        if (tid < TILE && nv > 0 && nv + tid < ntiles * TILE) s_rows[nv + tid] = s_rows[0];
+        __syncthreads();
+    };
+
+    // ---- gather ----
+    // bf16 rows: wave w loads NoPE rows 8w .. 8w+7 (one 1 KB load each; chunk c of
+    // row r at c ^ 4 (r & 3)) and their RoPE blocks in one more load.  fp8 rows:
+    // the raw tile in 21 (20) loads, wave w taking loads w, w+4, ...; the last
+    // load of 21 is half one (32 lanes), so that it ends with the slot.  656-B
+    // rows lie back to back, lane chunk 64 k + lane in row chunk / 41; the MXFP8
+    // streams have a region each (NoPE at 512 r, RoPE at 16384 + 128 r with its
+    // pieces at c ^ (r & 7), the scales at 20480 + 16 r).
+    struct GatherRows {
+        int32_t r[RAW ? FP8_LPW : TILE / NWAVE];
+        int32_t rope;              // bf16 576-value rows: row of this lane's RoPE chunk
+    };
+    uint32_t f_rc[FP8_LPW] = {};
+    if constexpr (F16) {
+#pragma unroll
+        for (int i = 0; i < FP8_LPW; ++i) {
+            const unsigned ch = 64 * (wave + NWAVE * i) + lane;
+            const unsigned rt = ch / 41u;
+            f_rc[i] = 4u * (rt < TILE - 1 ? rt : TILE - 1) | (16u * (ch - 41u * rt)) << 16;
+        }
+    }
+    const int my_loads = RAW ? (wave < L::LOADS - NWAVE * (FP8_LPW - 1) ? FP8_LPW : FP8_LPW - 1)
+                             : TILE / NWAVE + (D512 ? 0 : 1);
+    auto load_rows = [&](int ti) -> GatherRows {
+        const LDS_AS int32_t* rows = s_rows + ti * TILE;
+        const int ln = opaque(lane);
+        GatherRows g;
+        g.rope = 0;
+        if constexpr (RAW) {
+#pragma unroll
+            for (int i = 0; i < FP8_LPW; ++i) {
+                const int k = wave + NWAVE * i;
+                if constexpr (F16) g.r[i] = lds_ld<int32_t>((lds_cptr)rows + ((unsigned)opaque((int)f_rc[i]) & 0xFFFFu));
+                else g.r[i] = rows[k < 16 ? 2 * k + (ln >> 5) : (k < 20 ? 8 * (k - 16) + (ln >> 3) : (ln & 31))];
+            }
+        } else {
+            const u32x4 ra = lds_ld<u32x4>((lds_cptr)(rows + 8 * wave));
+            const u32x4 rv = lds_ld<u32x4>((lds_cptr)(rows + 8 * wave + 4));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                g.r[i] = __builtin_amdgcn_readfirstlane((int)ra[i]);
+                g.r[4 + i] = __builtin_amdgcn_readfirstlane((int)rv[i]);
+            }
+            if constexpr (!D512) g.rope = rows[8 * wave + (ln >> 3)];
+        }
+        return g;
+    };
+    auto issue_rows = [&](const GatherRows& g, lds_ptr tb) {
+        const int ln = opaque(lane);
+        if constexpr (RAW) {
+            // (pool and stream pointers through registers the compiler cannot
+            // trace to the argument block: see dsa_mla_fwd_kernel)
+            const unsigned char* n0 = p.kv;
+            const unsigned char* n1 = p.kv2;
+            const unsigned char* o0 = p.kv_ro;
+            const unsigned char* o1 = p.kv2_ro;
+            const unsigned char* sc = p.kv_sc;
+            asm("" : "+s"(n0), "+s"(n1), "+s"(o0), "+s"(o1), "+s"(sc));
+#pragma unroll
+            for (int i = 0; i < FP8_LPW; ++i)
+                if (i < my_loads) {
+                    const int k = wave + NWAVE * i;
+                    const uint64_t row = (uint32_t)dsa_rows::row_index(g.r[i]);
+                    const bool e2 = L::V4MX && dsa_rows::row_in_pool2(g.r[i]);
+                    const unsigned char* src;
+                    if constexpr (F16)
+                        src = n0 + ((uint64_t)(uint32_t)g.r[i] * (uint32_t)p.row_bytes + ((unsigned)opaque((int)f_rc[i]) >> 16));
+                    else if constexpr (L::V4MX)
+                        src = k < 16 ? (e2 ? n1 : n0) + row * p.kvn_st + 16 * (ln & 31)
+                                     : (e2 ? o1 : o0) + row * p.kvr_st + 16 * (ln & 7);
+                    else
+                        src = k < 16 ? n0 + (uint64_t)(uint32_t)g.r[i] * p.kvn_st + 16 * (ln & 31)
+                                     : (k < 20 ? o0 + (uint64_t)(uint32_t)g.r[i] * p.kvr_st + 16 * ((ln & 7) ^ ((ln >> 3) & 7))
+                                               : sc + (uint64_t)(uint32_t)g.r[i] * p.kvs_st);
+                    if (k < 20) lds_dma16(src, tb + 1024 * k);
+                    else if (ln < 32) lds_dma16(src, tb + 1024 * k);
+                }
+        } else {
+#pragma unroll
+            for (int i = 0; i < TILE / NWAVE; ++i) {
+                const int r = 8 * wave + i;
+                const int32_t id = __builtin_amdgcn_readfirstlane(g.r[i]);
+                const unsigned char* base;
+                if constexpr (D512)
+                    base = (dsa_rows::row_in_pool2(id) ? p.kv2 : p.kv) +
+                           (uint64_t)(uint32_t)dsa_rows::row_index(id) * (uint32_t)p.row_bytes;
+                else
+                    base = p.kv + (uint64_t)(uint32_t)id * (uint32_t)p.row_bytes;
+                lds_dma16_s(base, 16u * (unsigned)(ln ^ (4 * (i & 3))), tb + r * L::STRIDE);
+            }
+            if constexpr (!D512) {
+                const int r = 8 * wave + (ln >> 3);
+                lds_dma16(p.kv + (uint64_t)(uint32_t)g.rope * (uint32_t)p.row_bytes + 2 * D_NOPE +
+                              16 * ((ln & 7) ^ rope_sw(r)),
+                          tb + L::ROPE + 8 * wave * 128);
+            }
+        }
+    };
+    // wait until this wave's loads of all but the newest tile landed
+    auto wait_but_one = [&]() {
+        if constexpr (RAW) {
+            if (my_loads == FP8_LPW) wait_vm<FP8_LPW>();
+            else wait_vm<FP8_LPW - 1>();
+        } else {
+            wait_vm<TILE / NWAVE + (D512 ? 0 : 1)>();
+        }
+    };
+    // fp8: raw slot rw -> the 16-bit tile buffer.  Wave w converts rows w + 4j,
+    // lane l the codes 8l .. 8l+7 (V4: lanes 56..63 copy the row's RoPE values).
+    // All loads are issued before any store.
+    bool range_bad = false;
+    auto dequant_tile = [&](lds_cptr rw, lds_ptr tb) {
+        const int ln = opaque(lane);
+        u32x2 codes[TILE / NWAVE], extra[TILE / NWAVE];      // extra: scale bits, scale byte(s), or RoPE
+#pragma unroll
+        for (int j = 0; j < TILE / NWAVE; ++j) {
+            const int r = wave + NWAVE * j;
+            if constexpr (F16) {
+                const lds_cptr rr = rw + r * FP8_ROW;
+                codes[j] = lds_ld<u32x2>(rr + 8 * ln);
+                extra[j][0] = lds_ld<unsigned>(rr + FP8_SCALE_OFF + 4 * (ln >> 4));
+            } else if constexpr (L::V4MX) {
+                const lds_cptr rr = rw + r * D_NOPE;
+                const lds_cptr ra = rw + MX_ROPE_OFF + 128 * r + 16 * (ln & 7);
+                const bool rp = ln >= 56;
+                codes[j] = lds_ld<u32x2>(rp ? ra : rr + 8 * ln);
+                extra[j] = lds_ld<u32x2>(rp ? ra + 8 : rr + DSA_MLA_V4_NOPE + 8 * (ln >> 5));
+            } else {
+                codes[j] = lds_ld<u32x2>(rw + r * D_NOPE + 8 * ln);
+                extra[j][0] = lds_ld<unsigned char>(rw + MX_SC_OFF + 16 * r + (ln >> 2));
+            }
+        }
+        bool bad = false;
+#pragma unroll
+        for (int j = 0; j < TILE / NWAVE; ++j) {
+            const int r = wave + NWAVE * j;
+            u32x4 out;
+            if constexpr (F16) {
+                const unsigned sb = extra[j][0];
+                const float sc = __uint_as_float(sb);
+                bad |= sb >= FP8_SCALE_LIMIT_BITS;
+                const _Float16 m16 = (_Float16)__uint_as_float((sb & 0x007FFFFFu) | 0x3F800000u);
+                const f16x2 mm = {m16, m16};
+                const f16x2 h0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)codes[j][0], sc, false) * mm;
+                const f16x2 h1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)codes[j][0], sc, true) * mm;
+                const f16x2 h2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)codes[j][1], sc, false) * mm;
+                const f16x2 h3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)codes[j][1], sc, true) * mm;
+                out = u32x4{__builtin_bit_cast(unsigned, h0), __builtin_bit_cast(unsigned, h1),
+                            __builtin_bit_cast(unsigned, h2), __builtin_bit_cast(unsigned, h3)};
+            } else if constexpr (L::V4MX) {
+                const uint64_t sc8 = ((uint64_t)extra[j][1] << 32) | extra[j][0];
+                const unsigned e = (unsigned)(sc8 >> (8 * ((ln >> 2) & 7))) & 0xFFu;
+                const u32x4 cv = mx_to_bf16(codes[j][0], codes[j][1], e);
+                out = ln >= 56 ? u32x4{codes[j][0], codes[j][1], extra[j][0], extra[j][1]} : cv;
+            } else {
+                out = mx_to_bf16(codes[j][0], codes[j][1], extra[j][0]);
+            }
+            // (r & 3 is the wave)
+            lds_st<u32x4>(tb + r * L::STRIDE + 16 * (ln ^ (4 * wave)), out);
+        }
+        range_bad |= bad;
+    };
+
+    // ---- S^T[16 rows x 16 heads] = K Q^T (A operand: row 16 rb + c16, dims 32 ks
+    // + 8 g4 .. +7: chunk 4 ks + g4); kt: the tile, rt: its RoPE rows' base ----
+    auto qk16 = [&](lds_cptr kt, lds_cptr rt) -> f32x4 {
+        const int ln = opaque(lane);
+        const int row = 16 * rb + (ln & 15), lg = ln >> 4;
+        const lds_cptr kn = kt + row * L::STRIDE + 16 * lg;
+        const int x = 64 * (ln & 3);              // 64 (row & 3)
+        auto k_addr = [&](int ks) -> lds_cptr {
+            if (ks < KS_NOPE / 2) return kn + ((64 * (ks & 3)) ^ x) + 256 * (ks >> 2);
+            const int c = 4 * (ks - KS_NOPE / 2) + lg;
+            if constexpr (F16) return rt + row * FP8_ROW + FP8_ROPE_OFF + 16 * c;
+            else if constexpr (L::MX) return rt + MX_ROPE_OFF + 128 * row + 16 * (c ^ (row & 7));
+            else return rt + L::ROPE + 128 * row + 16 * (c ^ rope_sw(row));
+        };
+        constexpr int KPF = 6;
+        u32x4 kb[KPF];
+#pragma unroll
+        for (int i = 0; i < KPF; ++i) kb[i] = lds_ld<u32x4>(k_addr(i));
+        // two accumulator chains (a single 16x16x32 chain is latency-bound)
+        f32x4 acc[2] = {};
+#pragma unroll
+        for (int ks = 0; ks < L::NKS; ++ks) {
+            __builtin_amdgcn_sched_barrier(0);
+            // (656-B rows: the NoPE k-steps on fp16 operands, RoPE on bf16)
+            if (F16 && ks < KS_NOPE / 2) acc[ks & 1] = mfma16_f16(kb[ks % KPF], qf[ks], acc[ks & 1]);
+            else acc[ks & 1] = mfma16_bf16(kb[ks % KPF], qf[ks], acc[ks & 1]);
+            if (ks + KPF < L::NKS) kb[ks % KPF] = lds_ld<u32x4>(k_addr(ks + KPF));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        return acc[0] + acc[1];
+    };
+
+    // softmax state of head hq over this wave's rows: lane (g4, c16), value i
+    // of the 16x16 tile is row 16 rb + 4 g4 + i of the tile
+    float m_ref = 0.0f, l_lane = 0.0f, s_max = -INFINITY;
+    bool first_tile = true;
+    auto red4_max = [&](float v) {
+        v = fmaxf(v, __shfl_xor(v, 16, 64));
+        return fmaxf(v, __shfl_xor(v, 32, 64));
+    };
+    auto red4_sum = [&](float v) {
+        v += __shfl_xor(v, 16, 64);
+        return v + __shfl_xor(v, 32, 64);
+    };
+    // per-head value of both row halves through LDS slot k (a barrier between)
+    auto put_half = [&](int k, float v) {
+        if (g4 == 0) s_red[(2 * k + rb) * NARROW_HEADS + hq] = v;
+    };
+    auto get_max = [&](int k) { return fmaxf(s_red[2 * k * NARROW_HEADS + hq], s_red[(2 * k + 1) * NARROW_HEADS + hq]); };
+
+    // O^T accumulators: dims 128 wave + 32 m + (0..31) of the 32 heads: o[m]
+    f32x16 o[4];
+    auto raw_slot = [&](int i) -> lds_ptr { return POOL + (i & 1) * L::RAWB; };
+    auto tile_slot = [&](int i) -> lds_ptr { return RAW ? POOL + L::TILE0 : POOL + (i & 1) * L::SLOT; };
+    resolve_chunk(0, true);
+    for (int pass = 0;; ++pass) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m) o[m] = f32x16{};
+        l_lane = 0.0f;
+        s_max = -INFINITY;
+        first_tile = pass == 0;
+        for (int c = 0; c < nchunks; ++c) {
+            // a one-chunk list keeps its row list for the second pass
+            if ((pass == 0 && c > 0) || (pass > 0 && nchunks > 1)) resolve_chunk(c, false);
+            // Tiles (raw tiles) 0 and 1 go out before the loop, with Q possibly still
+            // in flight (older: the in-order waits for a tile cover it).
+#pragma unroll
+            for (int s0 = 0; s0 < 2; ++s0)
+                if (s0 < ntiles) issue_rows(load_rows(s0), RAW ? raw_slot(s0) : tile_slot(s0));
+            GatherRows gnext;
+            if (2 < ntiles) gnext = load_rows(2);
+            if (pass == 0 && c == 0) convert_q();
+            // Q's last fragment, and so all of it, is waited for here, on every path to
+            // the tile loop: left to its first use, the wait fell into the loop and
+            // drained the gathers on every tile (V4 fp8 rows)
+            asm volatile("" ::"v"(qf[L::NKS - 1][3]));
+            for (int it = 0; it < ntiles; ++it) {
+                const lds_ptr kt = tile_slot(it);
+                const lds_cptr rt = RAW ? raw_slot(it) : kt;
+                if constexpr (RAW) {
+                    // raw tile it landed (it+1 may be in flight); after the barrier
+                    // every wave is done with tile it-1's buffer and P
+                    if (it + 1 < ntiles) wait_but_one();
+                    else wait_vm<0>();
+                    tile_barrier();
+                    dequant_tile(rt, kt);
+                    tile_barrier();
+                } else {
+                    // tile it landed (tile 1 may be in flight behind tile 0); after the
+                    // barrier every wave is done with tile it-1, whose slot receives it+1
+                    if (it == 0 && ntiles > 1) wait_but_one();
+                    else wait_vm<0>();
+                    tile_barrier();
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (it >= 1 && it + 1 < ntiles) {
+                        issue_rows(gnext, tile_slot(it + 1));
+                        if (it + 2 < ntiles) gnext = load_rows(it + 2);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                f32x4 s = qk16(kt, rt);
+                const int rows_left = n_valid - it * TILE;
+                const int row0 = 16 * rb + 4 * g4;
+                if (first_tile) {
+                    // the reference: the largest score of the list's first tile
+                    float mx = -INFINITY;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) mx = fmaxf(mx, row0 + i < rows_left ? s[i] : -INFINITY);
+                    put_half(0, red4_max(mx));
+                    tile_barrier();
+                    m_ref = get_max(0) * c_s;
+                    first_tile = false;
+                }
+                if (rows_left < TILE) {
+                    asm volatile("");
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) s[i] = row0 + i < rows_left ? s[i] : -INFINITY;
+                }
+                s_max = fmaxf(s_max, fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])));
+                if (nchunks == 1 && ntiles == 1) {
+                    // single-tile list: the exact sum folded into the reference,
+                    // so that P is normalised when it is rounded
+                    // (opus_attn/dsa_v32/common/host.cc:448-451)
+                    float lt = 0.0f;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) lt += __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], c_s, -m_ref));
+                    put_half(1, red4_sum(lt));
+                    tile_barrier();
+                    float l1 = s_red[2 * NARROW_HEADS + hq] + s_red[3 * NARROW_HEADS + hq], m_fold = m_ref;
+                    // (an attention sink joins the sum: mla_v4_host.cc:469-472)
+                    if (D512 && p.attn_sink)
+                        add_sink(l1, m_ref, p.attn_sink[min(hbase + hq, p.H - 1)] * LOG2E, l1, m_fold);
+                    m_ref = m_fold + __builtin_amdgcn_logf(l1);
+                }
+                f32x4 e;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) e[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], c_s, -m_ref));
+                l_lane += (e[0] + e[1]) + (e[2] + e[3]);
+                // P of rows 16 rb + 4 g4 + i: PV k-step u = rb, lane half g4 & 1,
+                // positions 4 (g4 >> 1) + i (the rows the V reads pair with them)
+                u32x2 pw;
+                if constexpr (F16) {
+                    // fp16 P for the fp16 PV MFMAs (finite below 2^16: TAU = 15)
+                    const f16x2 p01 = {(_Float16)e[0], (_Float16)e[1]}, p23 = {(_Float16)e[2], (_Float16)e[3]};
+                    pw = u32x2{__builtin_bit_cast(unsigned, p01), __builtin_bit_cast(unsigned, p23)};
+                } else {
+                    pw = __builtin_bit_cast(u32x2, __builtin_convertvector(e, bf16x4));
+                }
+                lds_st<u32x2>(PX + ((2 * rb + (g4 & 1)) * NARROW_HEADS + hq) * 16 + 8 * (g4 >> 1), pw);
+                tile_barrier();
+                if constexpr (RAW) {
+                    // every wave is done with this raw slot: tile it+2 into it
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (it + 2 < ntiles) {
+                        issue_rows(gnext, raw_slot(it));
+                        if (it + 3 < ntiles) gnext = load_rows(it + 3);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                // ---- O^T[128 dims of this wave x 32 heads] += V^T P^T.  Transposed
+                // reads: 16-lane group g16 reads rows R..R+3 (lane 4rr+pp: row R+rr,
+                // dims d0+4pp..+3) with R = 16u + 4hi and R + 8 ----
+                const int vln = opaque(lane);
+                const int vhi = vln >> 5;
+                const int g16 = vln >> 4, i16 = vln & 15, vrr = i16 >> 2, vpp = i16 & 3;
+                const lds_cptr v0 = kt + (4 * vhi + vrr) * L::STRIDE + 16 * (2 * (g16 & 1) + (vpp >> 1)) +
+                                    8 * (vpp & 1) + 256 * wave;
+                auto v_frag = [&](int u, int m) -> u32x4 {
+                    const lds_cptr v = v0 + 64 * (m ^ vrr) + 16 * u * L::STRIDE;
+                    const s16x4 va = lds_read_tr16(v);
+                    const s16x4 vb = lds_read_tr16(v + 8 * L::STRIDE);
+                    return __builtin_bit_cast(u32x4, __builtin_shufflevector(va, vb, 0, 1, 2, 3, 4, 5, 6, 7));
+                };
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const u32x4 pb = lds_ld<u32x4>(PX + ((2 * u + vhi) * NARROW_HEADS + (vln & 31)) * 16);
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) {
+                        if constexpr (F16) o[m] = mfma_f16(v_frag(u, m), pb, o[m]);
+                        else o[m] = mfma_bf16(v_frag(u, m), pb, o[m]);
+                    }
+                }
+            }
+            // drain in-flight gathers before the slots can be reused or left
+            wait_vm<0>();
+        }
+        // per head: the largest score of the pass over both row halves (log2
+        // units); NaN compares false.  A head past the reference by more than
+        // TAU restarts the workgroup once, with the exact maximum.
+        put_half(2, red4_max(s_max));
+        // (the barrier also ends every wave's use of the tile buffers: a
+        // restart refills them, the epilogue stages O in them)
+        tile_barrier();
+        const float top = get_max(2) * c_s;
+        if (pass == 0 && __builtin_amdgcn_ballot_w64(top - m_ref > L::TAU) != 0 && lane == 0) s_misc[NWAVE] = 1;
+        tile_barrier();
+        if (pass != 0 || s_misc[NWAVE] == 0) break;
+        m_ref = fmaxf(m_ref, top);
+    }
+
+    // ---- epilogue: O / l and LSE, final (bf16) or a split's partial (fp32) ----
+    put_half(3, red4_sum(l_lane));
+    if (rb == 0 && g4 == 0) s_red[8 * NARROW_HEADS + hq] = m_ref;
+    if (F16 && range_bad) s_misc[NWAVE + 1] = 1;
+    tile_barrier();
+    // A list cut short, or (656-B rows) a scale outside the fp16 path's range:
+    // NaN outputs, never a silently truncated or wrong attention.
+    const bool nan_out = truncated || (F16 && s_misc[NWAVE + 1] != 0);
+    const float l_rows = s_red[6 * NARROW_HEADS + r32] + s_red[7 * NARROW_HEADS + r32];
+    const float m_head = s_red[8 * NARROW_HEADS + r32];
+    const bool has = any_rows;
+    float l = l_rows, m_fin = m_head, o_scale = 1.0f;
+    if constexpr (D512)
+        if (p.attn_sink) {
+            add_sink(l_rows, m_head, p.attn_sink[min(head_g, p.H - 1)] * LOG2E, l, m_fin);
+            o_scale = __builtin_amdgcn_exp2f(m_head - m_fin);
+        }
+    const float inv =
+        nan_out ? __builtin_nanf("") : (has ? (nchunks == 1 && ntiles == 1 ? 1.0f : o_scale / l) : 0.0f);
+    const int64_t qrow = (int64_t)b * p.s_q + t;
+    const bool planned = !D512 && p.plan_items;
+    const bool to_part = p.part_o != nullptr && (!planned || item_slot >= 0);
+    const int64_t part_row = planned ? (int64_t)item_slot : (int64_t)split * p.B * p.s_q + qrow;
+    if (wave == 0 && hi == 0 && head_g < p.H) {
+        const float lse_v = nan_out ? __builtin_nanf("") : (m_fin + __builtin_amdgcn_logf(l)) * LN2;
+        if (!to_part) {
+            if (p.lse) p.lse[qrow * p.H + head_g] = has || nan_out ? lse_v : INFINITY;
+        } else {
+            p.part_lse[part_row * p.H + head_g] = has || nan_out ? lse_v : -FLT_MAX;
+        }
+    }
+    // lane (hi, r32), reg 4g + i of o[m]: dim 128 wave + 32 m + 8 g + 4 hi + i of head r32.
+    // Staged through LDS (each wave its own region) so that the global stores
+    // write whole row pieces of the wave's 128 dims.
+    const int ln = opaque(lane);
+    if (!to_part) {
+        constexpr int OST = 2 * 128 + 16;               // staged head row: 128 bf16 + pad
+        static_assert(NWAVE * 32 * OST <= L::REDO, "O stage fits the buffers");
+        const lds_ptr stg = POOL + wave * 32 * OST;
+        const int st_w = opaque(r32 * OST + 8 * hi);
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const f32x4 v4 = {o[m][4 * g] * inv, o[m][4 * g + 1] * inv, o[m][4 * g + 2] * inv,
+                                  o[m][4 * g + 3] * inv};
+                lds_st<u32x2>(stg + st_w + 2 * (32 * m + 8 * g), __builtin_bit_cast(u32x2, __builtin_convertvector(v4, bf16x4)));
+            }
+        __bf16* const orow = p.out + (int64_t)b * p.o_sb + (int64_t)t * p.o_st;
+        const bool o16 = ((p.o_sb | p.o_st | p.o_sh) & 7) == 0 && ((uintptr_t)p.out & 15) == 0;
+        // lane (k, c): head row 4k + c / 16 of the group, dims 8 (c % 16) .. +7 of the wave's 128
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int r = 4 * k + (ln >> 4);
+            if (hbase + r >= p.H) break;
+            const u32x4 v = lds_ld<u32x4>(stg + r * OST + 16 * (ln & 15));
+            __bf16* const dst = orow + (int64_t)(hbase + r) * p.o_sh + 128 * wave + 8 * (ln & 15);
+            if (o16) {
+                *reinterpret_cast<u32x4*>(dst) = v;
+            } else {
+                reinterpret_cast<u32x2*>(dst)[0] = u32x2{v[0], v[1]};
+                reinterpret_cast<u32x2*>(dst)[1] = u32x2{v[2], v[3]};
+            }
+        }
+    } else {
+        constexpr int PST = 4 * 128 + 16;               // staged head row: 128 floats + pad
+        static_assert(NWAVE * 32 * PST <= L::REDO, "partial stage fits the buffers");
+        const lds_ptr stg = POOL + wave * 32 * PST;
+        const int st_w = opaque(r32 * PST + 16 * hi);
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const f32x4 v4 = {o[m][4 * g] * inv, o[m][4 * g + 1] * inv, o[m][4 * g + 2] * inv,
+                                  o[m][4 * g + 3] * inv};
+                lds_st<f32x4>(stg + st_w + 4 * (32 * m + 8 * g), v4);
+            }
+        const int64_t prow0 = part_row * p.H + hbase;
+        // lane (j, c): head row 2k + j of the group, floats 4c..4c+3 of the wave's 128
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const int r = 2 * k + (ln >> 5);
+            const f32x4 v = lds_ld<f32x4>(stg + r * PST + 16 * (ln & 31));
+            if (hbase + r < p.H)
+                *reinterpret_cast<f32x4*>(p.part_o + (prow0 + r) * D_VO + 128 * wave + 4 * (ln & 31)) = v;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Split combine: one wave per (row, head); lane holds 8 of the 512 outputs.
 // Math of mla_reduce (opus_attn/dsa_v32/common/mla_reduce.hpp:6-156):
 // m = max lse_i, w_i = exp(lse_i - m) (0 for an empty split),
@@ -2956,21 +3764,28 @@ bool heads_ok(int32_t H, int64_t tokens) {
     return H >= 1 && tokens * head_groups(H) <= INT32_MAX;
 }
 
-// Forward kernel for bf16 rows (576-value rows in the top-k or uniform-split
-// CSR form, V4 512-value rows) and 656-B fp8 rows (the same forms):
-// 32-head workgroups (dsa_mla_fwd_narrow_kernel) when the 128-head kernel
-// would compute at least 4x padding heads (H <= 32), or could not occupy half
-// the GPU even with its splits (fewer than 128 workgroups at wide_splits
-// splits).  Per head and row the 32-head kernel costs about 2.3x the cycles,
-// so it pays only where the 128-head kernel leaves CUs idle or computes
-// mostly padding.
+// Forward kernel of a call of `tokens` query tokens (work items) and H heads.
+//   WIDE    128 heads per workgroup, one per CU (dsa_mla_fwd_kernel)
+//   NARROW  32 heads, one workgroup per CU (dsa_mla_fwd_narrow_kernel)
+//   PAIR    32 heads, two workgroups per CU (dsa_mla_fwd_pair_kernel)
+// 32-head workgroups where the 128-head kernel would compute at least 2x padding
+// heads (H <= 64; V4 fp8 rows H <= 32: two groups convert every row twice, 763
+// against 711 us at H = 64, 2048 queries of 1152 rows), or could not occupy half
+// the GPU even with its splits (fewer than 128 workgroups at wide_splits splits).
+// PAIR when there are more of them than CUs, so that a second one on a CU has
+// something to fill: 4096 queries x 2048 rows at H = 16 in bf16 747 us, NARROW
+// 1226; at H = 64 (2048 queries) 759, WIDE 945.
+enum Kern { WIDE, NARROW, PAIR };
 int narrow_groups(int32_t H) { return (H + NARROW_HEADS - 1) / NARROW_HEADS; }
+int groups_of(Kern k, int32_t H) { return k == WIDE ? head_groups(H) : narrow_groups(H); }
+bool has_narrow(int fmt) { return fmt == DSA_KV_BF16 || fmt == DSA_KV_BF16_D512 || fmt == DSA_KV_FP8_656; }
 bool narrow_path(int fmt, int64_t tokens, int32_t H, int wide_splits) {
-    if ((fmt != DSA_KV_BF16 && fmt != DSA_KV_BF16_D512 && fmt != DSA_KV_FP8_656) || H < 1 ||
-        tokens * narrow_groups(H) > INT32_MAX)
-        return false;
-    return H <= 32 || tokens * head_groups(H) * wide_splits < 128;
+    if (H < 1 || tokens * narrow_groups(H) > INT32_MAX) return false;
+    if (H <= (fmt == DSA_KV_MXFP8_V4 ? 32 : 64)) return true;
+    return has_narrow(fmt) && tokens * head_groups(H) * wide_splits < 128;
 }
+// NARROW or PAIR for `wgs` 32-head workgroups
+Kern narrow_kern(int fmt, int64_t wgs) { return !has_narrow(fmt) || wgs > 256 ? PAIR : NARROW; }
 
 // Splits of a call whose `wgs` unsplit workgroups would leave CUs idle: as many
 // as fit one round of the 256 CUs (a workgroup takes a whole CU), with at least
@@ -2979,26 +3794,43 @@ bool narrow_path(int fmt, int64_t tokens, int32_t H, int wide_splits) {
 // the list: 2 (F + L / ceil) against F + L / floor, and ceil <= floor + 1 makes
 // the one round shorter for any F > 0.  74 query tokens of 16 heads (656-B rows,
 // 2048 entries): 3 splits 49.9 us against 4 splits (296 workgroups) 73.5 us.
-int one_round_splits(int64_t wgs, int64_t max_list, int64_t min_entries) {
+int one_round_splits(int64_t wgs, int64_t max_list, int64_t min_entries, int round = 256) {
     if (wgs <= 0 || wgs >= 256) return 1;
     const int64_t by_len = std::max<int64_t>(1, max_list / min_entries);
-    return (int)std::min<int64_t>(std::min<int64_t>(256 / wgs, by_len), DSA_MLA_MAX_SPLITS);
+    return (int)std::min<int64_t>(std::min<int64_t>(round / wgs, by_len), DSA_MLA_MAX_SPLITS);
+}
+// The same for 32-head workgroups, of which two fit a CU.  656-B rows fill both
+// places (a workgroup waits through its conversions): 130 tokens of 16 heads 68
+// us in 3 splits, 108 unsplit; 74 tokens 42 against 50 in 3.  bf16 rows gain
+// less from a second workgroup than its partials cost (40 tokens of 32 heads 34
+// us in 6 splits, 42 in 12), except where one round of CUs would leave the call
+// unsplit and a third of them idle (130 tokens of 16 heads 73 us in 3 splits, 84
+// unsplit; 200 tokens 104 in 2, 91 unsplit).
+int narrow_splits(int fmt, int64_t wgs, int64_t max_list, int64_t min_entries, bool one_per_cu = false) {
+    const bool two = one_per_cu ? false : fmt == DSA_KV_FP8_656 || fmt == DSA_KV_MXFP8_V4 || (wgs > 128 && wgs <= 512 / 3);
+    return one_round_splits(wgs, max_list, min_entries, two ? 512 : 256);
 }
 // decode: at least 4 tiles per split (at top-k 2048 and B = 2 or 4: 16 splits
 // measured 11 % faster than 8 and 6 % faster than 32)
-int auto_splits(int64_t queries, int topk) { return one_round_splits(queries, (int64_t)topk + 127, 128); }
+constexpr int DECODE_MIN = 128;
+int auto_splits(int64_t wgs, int topk) { return one_round_splits(wgs, (int64_t)topk + DECODE_MIN - 1, DECODE_MIN); }
 
 // Split count and kernel of a top-k decode call: the caller's count, or the
 // automatic one for the kernel narrow_path picks.
-int decode_splits(const dsa_mla_decode_args* a, bool* narrow) {
-    const int64_t tokens = (int64_t)a->B * a->s_q;
+// one_per_cu: no more splits than one workgroup per CU asks for (fewer partials).
+int decode_splits(const dsa_mla_decode_args* a, Kern* kern, bool one_per_cu = false) {
+    const int64_t tokens = (int64_t)a->B * a->s_q, groups = narrow_groups(a->H);
     const int wide = a->num_splits ? a->num_splits : auto_splits(tokens * head_groups(a->H), a->topk);
-    *narrow = narrow_path(a->kv_format, tokens, a->H, wide);
-    if (a->num_splits || !*narrow) return wide;
-    return auto_splits(tokens * narrow_groups(a->H), a->topk);
+    *kern = WIDE;
+    if (!narrow_path(a->kv_format, tokens, a->H, wide)) return wide;
+    const int ns = a->num_splits ? a->num_splits
+                                 : narrow_splits(a->kv_format, tokens * groups, (int64_t)a->topk + DECODE_MIN - 1, DECODE_MIN,
+                                               one_per_cu);
+    *kern = narrow_kern(a->kv_format, tokens * groups * ns);
+    return ns;
 }
 
-int validate_decode(const dsa_mla_decode_args* a, int* ns_out, int* chunk_out) {
+int validate_decode(const dsa_mla_decode_args* a, int* ns_out, int* chunk_out, bool one_per_cu = false) {
     if (!a) return DSA_ERR_NULL_POINTER;
     if (a->B < 0 || a->s_q <= 0 || a->topk < 0 || a->topk > MAX_LIST) return DSA_ERR_BAD_SHAPE;
     if (!heads_ok(a->H, a->B)) return DSA_ERR_BAD_SHAPE;
@@ -3007,8 +3839,8 @@ int validate_decode(const dsa_mla_decode_args* a, int* ns_out, int* chunk_out) {
     if (a->block_table && a->block_size <= 0) return DSA_ERR_BAD_SHAPE;
     if (row_stride_bytes(a->kv_format, a->kv_stride_row) < 0) return DSA_ERR_BAD_STRIDE;
     if (a->num_splits < 0 || a->num_splits > DSA_MLA_MAX_SPLITS) return DSA_ERR_BAD_SPLITS;
-    bool narrow;
-    const int ns = decode_splits(a, &narrow);
+    Kern kern;
+    const int ns = decode_splits(a, &kern, one_per_cu);
     const int chunk = a->topk == 0 ? 0 : (a->topk + ns - 1) / ns;
     if (a->B > 0 && a->topk > 0) {
         if (!a->q || !a->kv_cache || !a->seq_lens || !a->indices || !a->out) return DSA_ERR_NULL_POINTER;
@@ -3032,18 +3864,28 @@ size_t decode_ws_bytes(const dsa_mla_decode_args* a, int ns) {
     return (size_t)ns * rows * (D_VO + 1) * sizeof(float) + 256;
 }
 
-int launch_fwd(const FwdParams& fp, int fmt, int B, int s_q, int ns, hipStream_t st, bool narrow = false) {
+int launch_fwd(const FwdParams& fp, int fmt, int B, int s_q, int ns, hipStream_t st, Kern kern = WIDE) {
     dim3 grid((unsigned)((int64_t)B * fp.hgroups), s_q, ns), block(NTHR);
-    if (narrow && fmt == DSA_KV_BF16_D512)
-        hipLaunchKernelGGL(dsa_mla_fwd_narrow_kernel<DSA_KV_BF16_D512>, grid, block, 0, st, fp);
-    else if (narrow && fmt == DSA_KV_FP8_656)
-        hipLaunchKernelGGL(dsa_mla_fwd_narrow_kernel<DSA_KV_FP8_656>, grid, block, 0, st, fp);
-    else if (narrow) hipLaunchKernelGGL(dsa_mla_fwd_narrow_kernel<DSA_KV_BF16>, grid, block, 0, st, fp);
-    else if (fmt == DSA_KV_BF16) hipLaunchKernelGGL(dsa_mla_fwd_kernel<DSA_KV_BF16>, grid, block, 0, st, fp);
-    else if (fmt == DSA_KV_FP8_656) hipLaunchKernelGGL(dsa_mla_fwd_kernel<DSA_KV_FP8_656>, grid, block, 0, st, fp);
-    else if (fmt == DSA_KV_MXFP8) hipLaunchKernelGGL(dsa_mla_fwd_kernel<DSA_KV_MXFP8>, grid, block, 0, st, fp);
-    else if (fmt == DSA_KV_MXFP8_V4) hipLaunchKernelGGL(dsa_mla_fwd_kernel<DSA_KV_MXFP8_V4>, grid, block, 0, st, fp);
-    else hipLaunchKernelGGL(dsa_mla_fwd_kernel<DSA_KV_BF16_D512>, grid, block, 0, st, fp);
+    if (kern == PAIR) {
+        auto fn = fmt == DSA_KV_BF16 ? dsa_mla_fwd_pair_kernel<DSA_KV_BF16>
+                  : fmt == DSA_KV_FP8_656 ? dsa_mla_fwd_pair_kernel<DSA_KV_FP8_656>
+                  : fmt == DSA_KV_MXFP8 ? dsa_mla_fwd_pair_kernel<DSA_KV_MXFP8>
+                  : fmt == DSA_KV_MXFP8_V4 ? dsa_mla_fwd_pair_kernel<DSA_KV_MXFP8_V4>
+                                           : dsa_mla_fwd_pair_kernel<DSA_KV_BF16_D512>;
+        hipLaunchKernelGGL(fn, grid, block, 0, st, fp);
+    } else if (kern == NARROW) {
+        auto fn = fmt == DSA_KV_BF16 ? dsa_mla_fwd_narrow_kernel<DSA_KV_BF16>
+                  : fmt == DSA_KV_FP8_656 ? dsa_mla_fwd_narrow_kernel<DSA_KV_FP8_656>
+                                          : dsa_mla_fwd_narrow_kernel<DSA_KV_BF16_D512>;
+        hipLaunchKernelGGL(fn, grid, block, 0, st, fp);
+    } else {
+        auto fn = fmt == DSA_KV_BF16 ? dsa_mla_fwd_kernel<DSA_KV_BF16>
+                  : fmt == DSA_KV_FP8_656 ? dsa_mla_fwd_kernel<DSA_KV_FP8_656>
+                  : fmt == DSA_KV_MXFP8 ? dsa_mla_fwd_kernel<DSA_KV_MXFP8>
+                  : fmt == DSA_KV_MXFP8_V4 ? dsa_mla_fwd_kernel<DSA_KV_MXFP8_V4>
+                                           : dsa_mla_fwd_kernel<DSA_KV_BF16_D512>;
+        hipLaunchKernelGGL(fn, grid, block, 0, st, fp);
+    }
     return hipGetLastError() == hipSuccess ? DSA_OK : DSA_ERR_HIP;
 }
 
@@ -3093,6 +3935,10 @@ int csr_plan_build(const int32_t* kv_indptr, int B, int s_q, int H, int max_len,
 // (plan kernel,) forward kernel over the plan's items, combine of the split rows;
 // build = false: the workspace already holds the plan of these lists
 int csr_plan_launch(FwdParams& fp, int fmt, int max_len, void* ws, bool build, hipStream_t st) {
+    // 32-head workgroups for up to 64 heads (the plan's rows are a device matter:
+    // its items number about 256 or more, so PAIR)
+    const Kern kern = narrow_path(fmt, (int64_t)fp.B * fp.s_q + PLAN_TARGET, fp.H, PLAN_TARGET) ? PAIR : WIDE;
+    fp.hgroups = groups_of(kern, fp.H);
     const CsrPlanLayout L = csr_plan_layout(fp.B, fp.s_q, fp.H, max_len);
     char* w = (char*)ws;
     int32_t* hdr = (int32_t*)w;
@@ -3111,7 +3957,7 @@ int csr_plan_launch(FwdParams& fp, int fmt, int max_len, void* ws, bool build, h
     }
     // (a multiple of 8 s_q workgroups: the item order the kernel maps them to)
     const int G = 8 * fp.s_q;
-    const int r = launch_fwd(fp, fmt, (L.items_max + G - 1) / G * G, 1, 1, st);
+    const int r = launch_fwd(fp, fmt, (L.items_max + G - 1) / G * G, 1, 1, st, kern);
     if (r || !L.slots_max) return r;
     hipLaunchKernelGGL(dsa_mla_combine_plan_kernel, dim3(4 * PLAN_TARGET), dim3(256), 0, st, (const float*)fp.part_o,
                        (const float*)fp.part_lse, fp.B, fp.H, fp.s_q, max_len, fp.out, fp.o_sb, fp.o_st, fp.o_sh,
@@ -3198,14 +4044,14 @@ size_t mx_ws_bytes(const dsa_mla_decode_mxfp8_args* a, int ns) {
 // the combine kernel (with the attention sink, V4).
 // Split count and kernel of a prefill call (N query tokens, lists of at most
 // max_list entries).
-int prefill_plan(int fmt, int64_t N, int32_t H, int requested, int64_t max_list, bool* narrow);
-int prefill_splits(int requested, int64_t wgs, int64_t max_list) {
-    return requested > 0 ? requested : one_round_splits(wgs, max_list, 256);
-}
-int prefill_plan(int fmt, int64_t N, int32_t H, int requested, int64_t max_list, bool* narrow) {
-    const int wide = prefill_splits(requested, N * head_groups(H), max_list);
-    *narrow = narrow_path(fmt, N, H, wide);
-    return *narrow ? prefill_splits(requested, N * narrow_groups(H), max_list) : wide;
+constexpr int PREFILL_MIN = 256;
+int prefill_plan(int fmt, int64_t N, int32_t H, int requested, int64_t max_list, Kern* kern) {
+    const int wide = requested > 0 ? requested : one_round_splits(N * head_groups(H), max_list, PREFILL_MIN);
+    *kern = WIDE;
+    if (!narrow_path(fmt, N, H, wide)) return wide;
+    const int ns = requested > 0 ? requested : narrow_splits(fmt, N * narrow_groups(H), max_list, PREFILL_MIN);
+    *kern = narrow_kern(fmt, N * narrow_groups(H) * ns);
+    return ns;
 }
 size_t prefill_ws_bytes(int ns, int64_t N, int H) {
     return ns <= 1 || N == 0 ? 0 : (size_t)ns * N * H * (D_VO + 1) * sizeof(float) + 256;
@@ -3213,7 +4059,7 @@ size_t prefill_ws_bytes(int ns, int64_t N, int H) {
 // Forward kernel over ns splits of N query tokens, then (ns > 1) the combine of
 // their partials, with the attention sink folded in once by the combine.
 int prefill_launch(FwdParams& fp, int fmt, int ns, const float* sink, void* ws, hipStream_t st,
-                   bool narrow = false) {
+                   Kern kern) {
     const int64_t N = fp.B;
     if (ns > 1) {
         fp.part_o = (float*)ws;
@@ -3222,7 +4068,7 @@ int prefill_launch(FwdParams& fp, int fmt, int ns, const float* sink, void* ws, 
     } else {
         fp.attn_sink = sink;
     }
-    const int r = launch_fwd(fp, fmt, (int)N, 1, ns, st, narrow);
+    const int r = launch_fwd(fp, fmt, (int)N, 1, ns, st, kern);
     if (r || ns == 1) return r;
     return launch_combine(fp.part_o, fp.part_lse, ns, (int)N, fp.H, 1, fp.out, fp.o_sb, 0, fp.o_sh, fp.lse, st,
                           sink);
@@ -3236,8 +4082,8 @@ int validate_prefill(const dsa_mla_prefill_args* a, int* ns_out) {
     if (row_stride_bytes(a->kv_format, a->kv_stride_row) < 0) return DSA_ERR_BAD_STRIDE;
     if (a->topk > MAX_LIST) return DSA_ERR_BAD_SHAPE;
     if (a->num_splits < 0 || a->num_splits > DSA_MLA_MAX_SPLITS) return DSA_ERR_BAD_SPLITS;
-    bool narrow;
-    *ns_out = prefill_plan(a->kv_format, a->N, a->H, a->num_splits, a->topk, &narrow);
+    Kern kern;
+    *ns_out = prefill_plan(a->kv_format, a->N, a->H, a->num_splits, a->topk, &kern);
     if (a->N == 0) return DSA_OK;
     if (!a->q || !a->out || (a->topk > 0 && (!a->kv || !a->indices))) return DSA_ERR_NULL_POINTER;
     if ((a->q_stride_n % 8) || (a->q_stride_h % 8) || (a->o_stride_n % 4) || (a->o_stride_h % 4))
@@ -3256,8 +4102,8 @@ int validate_v4(const dsa_mla_prefill_v4_args* a, int* ns_out) {
     if (!heads_ok(a->H, a->N)) return DSA_ERR_BAD_SHAPE;
     if (a->D != DSA_MLA_D_V4) return DSA_ERR_UNSUPPORTED;
     if (a->num_splits < 0 || a->num_splits > DSA_MLA_MAX_SPLITS) return DSA_ERR_BAD_SPLITS;
-    bool narrow;
-    *ns_out = prefill_plan(DSA_KV_BF16_D512, a->N, a->H, a->num_splits, a->max_rows, &narrow);
+    Kern kern;
+    *ns_out = prefill_plan(DSA_KV_BF16_D512, a->N, a->H, a->num_splits, a->max_rows, &kern);
     if (a->N == 0) return DSA_OK;
     if (!a->q || !a->out || !a->kv_indptr_prefix || !a->kv_indices_prefix || !a->kv_indptr_extend ||
         !a->kv_indices_extend)
@@ -3280,7 +4126,8 @@ int validate_v4fp8(const dsa_mla_prefill_v4_fp8_args* a, int* ns_out) {
     if (a->max_rows > MAX_LIST) return DSA_ERR_BAD_SHAPE;
     if (!heads_ok(a->H, a->N)) return DSA_ERR_BAD_SHAPE;
     if (a->num_splits < 0 || a->num_splits > DSA_MLA_MAX_SPLITS) return DSA_ERR_BAD_SPLITS;
-    *ns_out = prefill_splits(a->num_splits, (int64_t)a->N * head_groups(a->H), a->max_rows);
+    Kern kern;
+    *ns_out = prefill_plan(DSA_KV_MXFP8_V4, a->N, a->H, a->num_splits, a->max_rows, &kern);
     if (a->N == 0) return DSA_OK;
     if (!a->q_nope || !a->q_rope || !a->out || !a->kv_indptr_prefix || !a->kv_indices_prefix ||
         !a->kv_indptr_extend || !a->kv_indices_extend)
@@ -3359,7 +4206,12 @@ int dsa_mla_decode_noalloc(const dsa_mla_decode_args* a, void* stream) {
     int ns, chunk;
     const int rc = validate_decode(a, &ns, &chunk);
     if (rc) return rc;
-    const size_t need = decode_ws_bytes(a, ns);
+    size_t need = decode_ws_bytes(a, ns);
+    if (need > DSA_MLA_NOALLOC_SCRATCH_BYTES) {
+        // fewer splits, where the automatic count can do with fewer
+        validate_decode(a, &ns, &chunk, true);
+        need = decode_ws_bytes(a, ns);
+    }
     if (need > DSA_MLA_NOALLOC_SCRATCH_BYTES) return DSA_ERR_SCRATCH_LIMIT;
     if (a->B == 0) return DSA_OK;
     void* ws = nullptr;
@@ -3375,11 +4227,12 @@ int dsa_mla_decode_noalloc(const dsa_mla_decode_args* a, void* stream) {
 namespace {
 
 int decode_launch(const dsa_mla_decode_args* a, int ns, int chunk, void* ws, hipStream_t st) {
-    bool narrow;
-    decode_splits(a, &narrow);
+    // the kernel of this split count (the automatic one, or fewer)
+    Kern kern;
+    if (decode_splits(a, &kern) != ns) decode_splits(a, &kern, true);
     FwdParams fp{};
     fp.H = a->H;
-    fp.hgroups = narrow ? narrow_groups(a->H) : head_groups(a->H);
+    fp.hgroups = groups_of(kern, a->H);
     fp.q = (const __bf16*)a->q;
     fp.q_sb = a->q_stride_b; fp.q_st = a->q_stride_t; fp.q_sh = a->q_stride_h;
     fp.kv = (const unsigned char*)a->kv_cache;
@@ -3406,7 +4259,7 @@ int decode_launch(const dsa_mla_decode_args* a, int ns, int chunk, void* ws, hip
         fp.part_o = (float*)ws;
         fp.part_lse = (float*)((char*)ws + (size_t)ns * rows * D_VO * sizeof(float));
     }
-    int r = launch_fwd(fp, a->kv_format, a->B, a->s_q, ns, st, narrow);
+    int r = launch_fwd(fp, a->kv_format, a->B, a->s_q, ns, st, kern);
     if (r || ns == 1) return r;
     return launch_combine(fp.part_o, fp.part_lse, ns, a->B * a->s_q, a->H, a->s_q, a->out, a->o_stride_b,
                           a->o_stride_t, a->o_stride_h, a->lse, st);
@@ -3444,10 +4297,12 @@ int dsa_mla_decode_csr(const dsa_mla_decode_csr_args* a, void* ws, size_t ws_byt
     if (a->B == 0) return DSA_OK;
     hipStream_t st = (hipStream_t)stream;
     // uniform splits (no work plan) of few query rows or few heads: 32-head workgroups
-    const bool narrow = ns >= 1 && narrow_path(a->kv_format, (int64_t)a->B * a->s_q, a->H, ns);
+    const int64_t rows_q = (int64_t)a->B * a->s_q;
+    const Kern kern = ns >= 1 && narrow_path(a->kv_format, rows_q, a->H, ns)
+                          ? narrow_kern(a->kv_format, rows_q * narrow_groups(a->H) * ns) : WIDE;
     FwdParams fp{};
     fp.H = a->H;
-    fp.hgroups = narrow ? narrow_groups(a->H) : head_groups(a->H);
+    fp.hgroups = groups_of(kern, a->H);
     fp.q = (const __bf16*)a->q;
     fp.q_sb = (int64_t)a->s_q * a->stride_q_b; fp.q_st = a->stride_q_b; fp.q_sh = a->stride_q_h;
     fp.kv = (const unsigned char*)a->kv;
@@ -3468,7 +4323,7 @@ int dsa_mla_decode_csr(const dsa_mla_decode_csr_args* a, void* ws, size_t ws_byt
         fp.part_o = (float*)ws;
         fp.part_lse = (float*)((char*)ws + (size_t)ns * rows * D_VO * sizeof(float));
     }
-    int r = launch_fwd(fp, a->kv_format, a->B, a->s_q, ns, st, narrow);
+    int r = launch_fwd(fp, a->kv_format, a->B, a->s_q, ns, st, kern);
     if (r || ns == 1) return r;
     return launch_combine(fp.part_o, fp.part_lse, ns, a->B * a->s_q, a->H, a->s_q, a->out, fp.o_sb, fp.o_st,
                           fp.o_sh, a->lse, st);
@@ -3489,9 +4344,10 @@ int dsa_mla_decode_mxfp8(const dsa_mla_decode_mxfp8_args* a, void* ws, size_t ws
     if (need && (!ws || ws_bytes < need || ((uintptr_t)ws & 15))) return DSA_ERR_WORKSPACE;
     if (a->B == 0) return DSA_OK;
     hipStream_t st = (hipStream_t)stream;
+    const Kern kern = ns >= 1 && narrow_path(DSA_KV_MXFP8, (int64_t)a->B * a->s_q, a->H, ns) ? PAIR : WIDE;
     FwdParams fp{};
     fp.H = a->H;
-    fp.hgroups = head_groups(a->H);
+    fp.hgroups = groups_of(kern, a->H);
     const int64_t sq = a->s_q;
     fp.q = (const __bf16*)a->q_rope;
     fp.q_sb = sq * a->stride_q_rope_b; fp.q_st = a->stride_q_rope_b; fp.q_sh = a->stride_q_rope_h;
@@ -3521,7 +4377,7 @@ int dsa_mla_decode_mxfp8(const dsa_mla_decode_mxfp8_args* a, void* ws, size_t ws
         fp.part_o = (float*)ws;
         fp.part_lse = (float*)((char*)ws + (size_t)ns * rows * D_VO * sizeof(float));
     }
-    int r = launch_fwd(fp, DSA_KV_MXFP8, a->B, a->s_q, ns, st);
+    int r = launch_fwd(fp, DSA_KV_MXFP8, a->B, a->s_q, ns, st, kern);
     if (r || ns == 1) return r;
     return launch_combine(fp.part_o, fp.part_lse, ns, a->B * a->s_q, a->H, a->s_q, a->out, fp.o_sb, fp.o_st,
                           fp.o_sh, a->lse, st);
@@ -3552,11 +4408,11 @@ int dsa_mla_prefill(const dsa_mla_prefill_args* a, void* ws, size_t ws_bytes, vo
     const size_t need = prefill_ws_bytes(ns, a->N, a->H);
     if (need && (!ws || ws_bytes < need || ((uintptr_t)ws & 15))) return DSA_ERR_WORKSPACE;
     if (a->N == 0) return DSA_OK;
-    bool narrow;
-    prefill_plan(a->kv_format, a->N, a->H, a->num_splits, a->topk, &narrow);
+    Kern kern;
+    prefill_plan(a->kv_format, a->N, a->H, a->num_splits, a->topk, &kern);
     FwdParams fp{};
     fp.H = a->H;
-    fp.hgroups = narrow ? narrow_groups(a->H) : head_groups(a->H);
+    fp.hgroups = groups_of(kern, a->H);
     fp.q = (const __bf16*)a->q;
     fp.q_sb = a->q_stride_n; fp.q_st = 0; fp.q_sh = a->q_stride_h;
     fp.kv = (const unsigned char*)a->kv;
@@ -3579,7 +4435,7 @@ int dsa_mla_prefill(const dsa_mla_prefill_args* a, void* ws, size_t ws_bytes, vo
     fp.causal_offset = a->causal_offset;
     fp.reverse = 1;
     fp.scale_log2 = a->sm_scale * LOG2E;
-    return prefill_launch(fp, a->kv_format, ns, nullptr, ws, (hipStream_t)stream, narrow);
+    return prefill_launch(fp, a->kv_format, ns, nullptr, ws, (hipStream_t)stream, kern);
 }
 
 int dsa_mla_prefill_v4_workspace_size(const dsa_mla_prefill_v4_args* a, size_t* bytes) {
@@ -3598,11 +4454,11 @@ int dsa_mla_prefill_v4(const dsa_mla_prefill_v4_args* a, void* ws, size_t ws_byt
     const size_t need = prefill_ws_bytes(ns, a->N, a->H);
     if (need && (!ws || ws_bytes < need || ((uintptr_t)ws & 15))) return DSA_ERR_WORKSPACE;
     if (a->N == 0) return DSA_OK;
-    bool narrow;
-    prefill_plan(DSA_KV_BF16_D512, a->N, a->H, a->num_splits, a->max_rows, &narrow);
+    Kern kern;
+    prefill_plan(DSA_KV_BF16_D512, a->N, a->H, a->num_splits, a->max_rows, &kern);
     FwdParams fp{};
     fp.H = a->H;
-    fp.hgroups = narrow ? narrow_groups(a->H) : head_groups(a->H);
+    fp.hgroups = groups_of(kern, a->H);
     fp.q = (const __bf16*)a->q;
     fp.q_sb = a->stride_qo_n; fp.q_st = 0; fp.q_sh = a->stride_qo_h;
     fp.kv = (const unsigned char*)a->unified_kv;
@@ -3618,7 +4474,7 @@ int dsa_mla_prefill_v4(const dsa_mla_prefill_v4_args* a, void* ws, size_t ws_byt
     fp.lse = a->lse;
     fp.B = a->N; fp.s_q = 1; fp.topk = a->max_rows; fp.chunk = a->max_rows;
     fp.scale_log2 = a->softmax_scale * LOG2E;
-    return prefill_launch(fp, DSA_KV_BF16_D512, ns, a->attn_sink, ws, (hipStream_t)stream, narrow);
+    return prefill_launch(fp, DSA_KV_BF16_D512, ns, a->attn_sink, ws, (hipStream_t)stream, kern);
 }
 
 int dsa_mla_prefill_v4_fp8_workspace_size(const dsa_mla_prefill_v4_fp8_args* a, size_t* bytes) {
@@ -3637,9 +4493,11 @@ int dsa_mla_prefill_v4_fp8(const dsa_mla_prefill_v4_fp8_args* a, void* ws, size_
     const size_t need = prefill_ws_bytes(ns, a->N, a->H);
     if (need && (!ws || ws_bytes < need || ((uintptr_t)ws & 15))) return DSA_ERR_WORKSPACE;
     if (a->N == 0) return DSA_OK;
+    Kern kern;
+    prefill_plan(DSA_KV_MXFP8_V4, a->N, a->H, a->num_splits, a->max_rows, &kern);
     FwdParams fp{};
     fp.H = a->H;
-    fp.hgroups = head_groups(a->H);
+    fp.hgroups = groups_of(kern, a->H);
     fp.q = (const __bf16*)a->q_rope;
     fp.q_sb = a->stride_q_rope_n; fp.q_st = 0; fp.q_sh = a->stride_q_rope_h;
     fp.q8 = (const unsigned char*)a->q_nope;
@@ -3663,7 +4521,7 @@ int dsa_mla_prefill_v4_fp8(const dsa_mla_prefill_v4_fp8_args* a, void* ws, size_
     fp.lse = a->lse;
     fp.B = a->N; fp.s_q = 1; fp.topk = a->max_rows; fp.chunk = a->max_rows;
     fp.scale_log2 = a->softmax_scale * LOG2E;
-    return prefill_launch(fp, DSA_KV_MXFP8_V4, ns, a->attn_sink, ws, (hipStream_t)stream);
+    return prefill_launch(fp, DSA_KV_MXFP8_V4, ns, a->attn_sink, ws, (hipStream_t)stream, kern);
 }
 int dsa_kv_quantize_fp8(const void* src, int64_t src_stride, int64_t n_rows, void* dst, int64_t dst_total,
                         const int64_t* dst_rows, void* stream) {

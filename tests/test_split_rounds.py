@@ -1,4 +1,5 @@
-"""Automatic split counts: the workgroups of a split call fit one round of the 256 CUs."""
+"""Automatic split counts: the workgroups of a split call fit one round of the GPU (256 CUs,
+each holding one 128-head workgroup or up to two 32-head ones)."""
 import ctypes
 
 import pytest
@@ -6,20 +7,26 @@ import pytest
 from opfoundry_amd import abi
 
 
+@pytest.mark.parametrize("fmt", [abi.KV_BF16, abi.KV_FP8_656])
 @pytest.mark.parametrize("B,H,topk", [(1, 128, 2048), (3, 16, 2048), (37, 16, 2048), (74, 16, 2048), (86, 128, 2048),
-                                      (127, 128, 512), (128, 128, 2048), (129, 32, 2048), (255, 128, 4096),
-                                      (256, 128, 4096), (300, 16, 100)])
-def test_splits_fit_one_round(B, H, topk):
+                                      (127, 128, 512), (128, 128, 2048), (129, 32, 2048), (130, 64, 2048),
+                                      (170, 16, 2048), (171, 16, 2048), (255, 128, 4096), (255, 32, 4096),
+                                      (256, 128, 4096), (256, 16, 4096), (300, 16, 100)])
+def test_splits_fit_one_round(fmt, B, H, topk):
     a = abi.DecodeArgs()
     for f in ("q", "kv_cache", "block_table", "seq_lens", "indices", "out", "lse"):
         setattr(a, f, 0x1000)
-    a.kv_format, a.kv_total_rows, a.block_size, a.block_table_stride = abi.KV_BF16, 1 << 20, 64, 1024
+    a.kv_format, a.kv_total_rows, a.block_size, a.block_table_stride = fmt, 1 << 20, 64, 1024
     a.B, a.s_q, a.H, a.topk, a.sm_scale = B, 1, H, topk, 0.07
     ns = ctypes.c_int32(0)
     assert abi.load_library().dsa_mla_decode_num_splits(ctypes.byref(a), ctypes.byref(ns)) == 0
-    # 32-head workgroups for H <= 32 or a call whose 128-head ones would fill under half the GPU
     cap = max(1, (topk + 127) // 128)
-    wide = max(1, min(256 // B, cap))
-    wgs = B * ((H + 31) // 32 if H <= 32 or B * ((H + 127) // 128) * wide < 128 else (H + 127) // 128)
-    assert ns.value == max(1, min(256 // wgs, cap, 64))
-    assert wgs >= 256 or wgs * ns.value <= 256
+    wide_wgs = B * ((H + 127) // 128)
+    wide = 1 if wide_wgs >= 256 else min(256 // wide_wgs, cap, 64)
+    if H <= 64 or wide_wgs * wide < 128:       # 32-head workgroups
+        wgs = B * ((H + 31) // 32)
+        round_ = 512 if fmt == abi.KV_FP8_656 or 128 < wgs <= 170 else 256
+    else:
+        wgs, round_ = wide_wgs, 256
+    assert ns.value == (1 if wgs >= 256 else max(1, min(round_ // wgs, cap, 64)))
+    assert wgs >= 256 or wgs * ns.value <= round_
