@@ -45,13 +45,16 @@ FLOP_PER_PAIR = 2 * H * (D_QK + D_VO)
 
 
 def _fwd_kernel(name, tokens, splits, heads):
-    """The library's rule: 32-head workgroups when heads <= 64 or when the 128-head kernel
-    would run fewer than 128 workgroups, two to a CU (pair) when they outnumber the CUs, else
-    one (narrow); else 128-head workgroups.  (splits: the split count the call runs with.)"""
+    """The library's rule: workgroups of 32 heads (of 64 for 33 to 64 heads of more tokens x
+    splits than CUs) when heads <= 64 or when the 128-head kernel would run fewer than 128
+    workgroups, two to a CU (pair) when they outnumber the CUs, else one (narrow); else
+    128-head workgroups.  (splits: the split count the call runs with.)"""
     groups = (heads + 31) // 32
     if heads <= 64 or tokens * ((heads + 127) // 128) * splits < 128:
-        kind = "pair" if tokens * groups * splits > 256 else "narrow"
-        return f"dsa_mla_fwd_{kind}_kernel<{name}>"
+        if 32 < heads <= 64 and tokens * splits > 256:
+            return f"dsa_mla_fwd_pair_kernel<{name}, 64>"
+        return (f"dsa_mla_fwd_pair_kernel<{name}, 32>" if tokens * groups * splits > 256
+                else f"dsa_mla_fwd_narrow_kernel<{name}>")
     return f"dsa_mla_fwd_kernel<{name}>"
 
 

@@ -37,11 +37,11 @@
  *
  * Heads.  Every entry takes any head count H >= 1 (H <= 0 is
  * DSA_ERR_BAD_SHAPE).  A query token runs in ceil(H / 128) workgroups of 128
- * heads, or in ceil(H / 32) workgroups of 32 heads at H <= 64 (V4 fp8 rows:
- * H <= 32) and, for bf16 and 656-B fp8 rows, when 128-head workgroups would be
- * too few to occupy the GPU (the summation order of the scores then differs,
- * within the same bounds); the last group computes its heads past H on a copy of head H-1 and stores
- * nothing for them, so outputs, LSEs and partials are written for heads
+ * heads, or in workgroups of 32 or 64 heads at H <= 64 and, of 32, for bf16 and
+ * 656-B fp8 rows when 128-head workgroups would be too few to occupy the GPU
+ * (the summation order of the scores then differs, within the same bounds); the
+ * last group computes its heads past H on a copy of head H-1 and stores nothing
+ * for them, so outputs, LSEs and partials are written for heads
  * 0..H-1 only.  The kernel choice changes dsa_mla_decode_num_splits and the
  * workspace sizes, which report the split count of the kernel that runs.
  *

@@ -2442,9 +2442,9 @@ dsa_mla_fwd_narrow_kernel(const FwdParams p_arg) {
 }
 
 // ---------------------------------------------------------------------------
-// Pair kernel: 32 heads per workgroup, two workgroups per CU.  For calls of
-// many 32-head workgroups (small head counts at batch, prefill of up to 64
-// heads): the narrow kernel's phases (gather, QK^T, softmax, PV) follow one
+// Pair kernel: HG = 32 or 64 heads per workgroup, two workgroups per CU.  For
+// calls of many 32-head workgroups (small head counts at batch, prefill of up
+// to 64 heads): the narrow kernel's phases (gather, QK^T, softmax, PV) follow one
 // another on one wave per SIMD, each waiting on LDS or a barrier with nothing
 // else to run; a second workgroup on the CU fills those waits.  That asks for
 // half the LDS (80 KB) and 256 registers per wave:
@@ -2459,14 +2459,23 @@ dsa_mla_fwd_narrow_kernel(const FwdParams p_arg) {
 // Formats: those of the narrow kernel, MXFP8 split streams and V4 fp8 rows (both
 // converted exactly to bf16); index forms: top-k, CSR with uniform splits or a
 // work plan, V4.  Arithmetic per tile as in dsa_mla_fwd_narrow_kernel.
-// Bound by the LDS and VALU work of both workgroups.  Against the narrow kernel:
+// 64 heads: a wave scores 16 heads x all 32 rows (two row blocks; no maxima or
+// sums cross waves) and its PV accumulates 128 dims x 64 heads, 128 registers,
+// which leaves few for reads ahead: row ids are read when they are needed, K
+// two k-steps ahead instead of six, fp8 rows converted four at a time.  Rows are
+// gathered, converted and read for PV once instead of once per 32 heads.
+// Bound by the LDS and VALU work of both workgroups.  HG = 32 against the narrow
+// kernel:
 // 4096 queries x 2048 bf16 rows, H = 16, 747 us instead of 1226; 2048 queries of
 // 656-B rows, H = 32, 549 instead of 835.  Against 128-head workgroups (the other
 // 64 or more heads padding): MXFP8, 128 tokens x 2048 rows, H = 16, 67 instead of
-// 86; V4 fp8 rows, 2048 queries x 1152, H = 16, 389 instead of 701.
-// grid = (tokens or plan items x ceil(H / 32), s_q, num_splits), block = 256.
+// 86; V4 fp8 rows, 2048 queries x 1152, H = 16, 389 instead of 701.  H = 64, 2048
+// queries, 128-head workgroups / two of HG = 32 / HG = 64: bf16 rows x 2048
+// 939 / 759 / 585 us, 656-B rows 1136 / 1089 / 755, V4 bf16 x 1152 561 / 473 /
+// 368, V4 fp8 714 / 763 / 484.
+// grid = (tokens or plan items x ceil(H / HG), s_q, num_splits), block = 256.
 // ---------------------------------------------------------------------------
-template <int NF>
+template <int NF, int HG>
 struct PairLay {
     static constexpr bool F16 = NF == DSA_KV_FP8_656;
     static constexpr bool V4MX = NF == DSA_KV_MXFP8_V4;
@@ -2482,21 +2491,26 @@ struct PairLay {
     static constexpr int RAWB = V4MX ? 20480 : 20992;
     static constexpr int TILE0 = RAW ? 2 * RAWB : 0;
     static constexpr int PXO = TILE0 + (RAW ? 1 : 2) * SLOT;
-    static constexpr int REDO = PXO + P_BYTES;
-    static constexpr int MISCO = REDO + 4 * (4 * 2 * NARROW_HEADS + NARROW_HEADS);
+    static constexpr int PB = 2 * 2 * HG * 16;                    // P of a tile: [u][hi][head] x 8 values
+    // per-head exchanges: 32 heads 4 x 2 x 32 + 32 floats; 64 heads only the sums
+    // and references after the last tile, in P's place
+    static constexpr int REDO = HG == 64 ? PXO : PXO + PB;
+    static constexpr int MISCO = PXO + PB + (HG == 64 ? 0 : 4 * (4 * 2 * HG + HG));
     static constexpr int ROWSO = MISCO + 32;
+    static constexpr int STAGE = PXO;                             // the epilogue's stage ends below P
     // entries of a chunk (a multiple of the workgroup's threads)
-    static constexpr int MC = V4MX ? 1024 : (D512 ? 2048 : (RAW ? 512 : 768));
+    static constexpr int MC = V4MX ? (HG == 64 ? 768 : 1024) : (D512 ? 2048 : (RAW || HG == 64 ? 512 : 768));
     static constexpr int BYTES = ROWSO + 4 * MC;
     static_assert(BYTES <= 81920, "two workgroups share a CU's 160 KB of LDS");
     static_assert(RAWB % 16 == 0 && STRIDE % 16 == 0, "16-byte LDS-DMA destinations");
     static constexpr float TAU = F16 ? 15.0f : 100.0f;
 };
 
-template <int NF>
+template <int NF, int HG>
 __global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2, 2)))
 dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
-    using L = PairLay<NF>;
+    using L = PairLay<NF, HG>;
+    constexpr int QB = HG / 32;                   // 16-row blocks of a wave's QK^T, 32-head blocks of its PV
     constexpr bool D512 = L::D512, F16 = L::F16, RAW = L::RAW;
     __shared__ __attribute__((aligned(1024))) unsigned char s_pool[L::BYTES];
     const lds_ptr POOL = (lds_ptr)s_pool;
@@ -2566,7 +2580,7 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
             gx = units / 8 * 8 + i / p.hgroups;
         }
     }
-    const int hbase = NARROW_HEADS * hg;
+    const int hbase = HG * hg;
     int b = p.reverse ? units - 1 - gx : gx, t = blockIdx.y;
     const int split = blockIdx.z;
     int item_k0 = 0, item_k1 = 0, item_slot = -1;
@@ -2583,12 +2597,12 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
                 const int bq = gx / p.s_q, tq = gx - bq * p.s_q;
                 __bf16* const orow = p.out + (int64_t)bq * p.o_sb + (int64_t)tq * p.o_st;
                 const unsigned nan2 = 0x7FC07FC0u;    // two bf16 NaNs
-                for (int i = (int)threadIdx.x; i < NARROW_HEADS * (D_VO / 4); i += NTHR) {
+                for (int i = (int)threadIdx.x; i < HG * (D_VO / 4); i += NTHR) {
                     const int hh = hbase + i / (D_VO / 4);
                     if (hh < p.H)
                         reinterpret_cast<u32x2*>(orow + (int64_t)hh * p.o_sh)[i % (D_VO / 4)] = u32x2{nan2, nan2};
                 }
-                for (int hh = (int)threadIdx.x; hh < NARROW_HEADS; hh += NTHR)
+                for (int hh = (int)threadIdx.x; hh < HG; hh += NTHR)
                     if (p.lse && hbase + hh < p.H) p.lse[(int64_t)gx * p.H + hbase + hh] = __builtin_nanf("");
             }
             return;
@@ -2611,11 +2625,12 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
     }
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int rb = wave & 1, hb = wave >> 1;      // QK^T: row half, head half
+    // QK^T: 32 heads: row half and head half; 64 heads: both row halves, head quarter
+    const int rb = HG == 64 ? 0 : wave & 1, hb = HG == 64 ? wave : wave >> 1;
     const int c16 = lane & 15, g4 = lane >> 4;    // 16x16 operand lanes
     const int hi = lane >> 5, r32 = lane & 31;    // PV and epilogue lanes: head r32
     const int hq = 16 * hb + c16;                 // this lane's head in QK^T and the softmax
-    const int head_g = hbase + r32;               // heads past H: a copy of head H-1, never stored
+    // (heads past H: a copy of head H-1, never stored)
     if (tid == 0) {
         s_misc[NWAVE] = 0;
         s_misc[NWAVE + 1] = 0;
@@ -2809,15 +2824,22 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
         int32_t r[RAW ? FP8_LPW : TILE / NWAVE];
         int32_t rope;              // bf16 576-value rows: row of this lane's RoPE chunk
     };
+    // (656-B rows: bits 0..15 the offset of the row's id in the row list, 16..31 the
+    // chunk's byte offset in the row; 64 heads: worked out where it is used)
+    auto rc_of = [&](int i, int ln) -> uint32_t {
+        const unsigned ch = 64 * (wave + NWAVE * i) + ln;
+        const unsigned rt = ch / 41u;
+        return 4u * (rt < TILE - 1 ? rt : TILE - 1) | (16u * (ch - 41u * rt)) << 16;
+    };
     uint32_t f_rc[FP8_LPW] = {};
-    if constexpr (F16) {
+    if constexpr (F16 && HG != 64) {
 #pragma unroll
-        for (int i = 0; i < FP8_LPW; ++i) {
-            const unsigned ch = 64 * (wave + NWAVE * i) + lane;
-            const unsigned rt = ch / 41u;
-            f_rc[i] = 4u * (rt < TILE - 1 ? rt : TILE - 1) | (16u * (ch - 41u * rt)) << 16;
-        }
+        for (int i = 0; i < FP8_LPW; ++i) f_rc[i] = rc_of(i, lane);
     }
+    auto f_at = [&](int i, int ln) -> uint32_t {
+        if constexpr (HG == 64) return rc_of(i, ln);
+        else return (uint32_t)opaque((int)f_rc[i]);
+    };
     const int my_loads = RAW ? (wave < L::LOADS - NWAVE * (FP8_LPW - 1) ? FP8_LPW : FP8_LPW - 1)
                              : TILE / NWAVE + (D512 ? 0 : 1);
     auto load_rows = [&](int ti) -> GatherRows {
@@ -2829,7 +2851,7 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
 #pragma unroll
             for (int i = 0; i < FP8_LPW; ++i) {
                 const int k = wave + NWAVE * i;
-                if constexpr (F16) g.r[i] = lds_ld<int32_t>((lds_cptr)rows + ((unsigned)opaque((int)f_rc[i]) & 0xFFFFu));
+                if constexpr (F16) g.r[i] = lds_ld<int32_t>((lds_cptr)rows + (f_at(i, ln) & 0xFFFFu));
                 else g.r[i] = rows[k < 16 ? 2 * k + (ln >> 5) : (k < 20 ? 8 * (k - 16) + (ln >> 3) : (ln & 31))];
             }
         } else {
@@ -2863,7 +2885,7 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
                     const bool e2 = L::V4MX && dsa_rows::row_in_pool2(g.r[i]);
                     const unsigned char* src;
                     if constexpr (F16)
-                        src = n0 + ((uint64_t)(uint32_t)g.r[i] * (uint32_t)p.row_bytes + ((unsigned)opaque((int)f_rc[i]) >> 16));
+                        src = n0 + ((uint64_t)(uint32_t)g.r[i] * (uint32_t)p.row_bytes + (f_at(i, ln) >> 16));
                     else if constexpr (L::V4MX)
                         src = k < 16 ? (e2 ? n1 : n0) + row * p.kvn_st + 16 * (ln & 31)
                                      : (e2 ? o1 : o0) + row * p.kvr_st + 16 * (ln & 7);
@@ -2906,90 +2928,108 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
     };
     // fp8: raw slot rw -> the 16-bit tile buffer.  Wave w converts rows w + 4j,
     // lane l the codes 8l .. 8l+7 (V4: lanes 56..63 copy the row's RoPE values).
-    // All loads are issued before any store.
+    // A batch's loads are issued before any of its stores.
     bool range_bad = false;
     auto dequant_tile = [&](lds_cptr rw, lds_ptr tb) {
         const int ln = opaque(lane);
-        u32x2 codes[TILE / NWAVE], extra[TILE / NWAVE];      // extra: scale bits, scale byte(s), or RoPE
-#pragma unroll
-        for (int j = 0; j < TILE / NWAVE; ++j) {
-            const int r = wave + NWAVE * j;
-            if constexpr (F16) {
-                const lds_cptr rr = rw + r * FP8_ROW;
-                codes[j] = lds_ld<u32x2>(rr + 8 * ln);
-                extra[j][0] = lds_ld<unsigned>(rr + FP8_SCALE_OFF + 4 * (ln >> 4));
-            } else if constexpr (L::V4MX) {
-                const lds_cptr rr = rw + r * D_NOPE;
-                const lds_cptr ra = rw + MX_ROPE_OFF + 128 * r + 16 * (ln & 7);
-                const bool rp = ln >= 56;
-                codes[j] = lds_ld<u32x2>(rp ? ra : rr + 8 * ln);
-                extra[j] = lds_ld<u32x2>(rp ? ra + 8 : rr + DSA_MLA_V4_NOPE + 8 * (ln >> 5));
-            } else {
-                codes[j] = lds_ld<u32x2>(rw + r * D_NOPE + 8 * ln);
-                extra[j][0] = lds_ld<unsigned char>(rw + MX_SC_OFF + 16 * r + (ln >> 2));
-            }
-        }
+        constexpr int DB = HG == 64 ? 4 : 8;       // rows of a batch (64 heads: few registers are left)
         bool bad = false;
 #pragma unroll
-        for (int j = 0; j < TILE / NWAVE; ++j) {
-            const int r = wave + NWAVE * j;
-            u32x4 out;
-            if constexpr (F16) {
-                const unsigned sb = extra[j][0];
-                const float sc = __uint_as_float(sb);
-                bad |= sb >= FP8_SCALE_LIMIT_BITS;
-                const _Float16 m16 = (_Float16)__uint_as_float((sb & 0x007FFFFFu) | 0x3F800000u);
-                const f16x2 mm = {m16, m16};
-                const f16x2 h0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)codes[j][0], sc, false) * mm;
-                const f16x2 h1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)codes[j][0], sc, true) * mm;
-                const f16x2 h2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)codes[j][1], sc, false) * mm;
-                const f16x2 h3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)codes[j][1], sc, true) * mm;
-                out = u32x4{__builtin_bit_cast(unsigned, h0), __builtin_bit_cast(unsigned, h1),
-                            __builtin_bit_cast(unsigned, h2), __builtin_bit_cast(unsigned, h3)};
-            } else if constexpr (L::V4MX) {
-                const uint64_t sc8 = ((uint64_t)extra[j][1] << 32) | extra[j][0];
-                const unsigned e = (unsigned)(sc8 >> (8 * ((ln >> 2) & 7))) & 0xFFu;
-                const u32x4 cv = mx_to_bf16(codes[j][0], codes[j][1], e);
-                out = ln >= 56 ? u32x4{codes[j][0], codes[j][1], extra[j][0], extra[j][1]} : cv;
-            } else {
-                out = mx_to_bf16(codes[j][0], codes[j][1], extra[j][0]);
+        for (int j0 = 0; j0 < TILE / NWAVE; j0 += DB) {
+            u32x2 codes[DB], extra[DB];                // extra: scale bits, scale byte(s), or RoPE
+#pragma unroll
+            for (int j = 0; j < DB; ++j) {
+                const int r = wave + NWAVE * (j0 + j);
+                if constexpr (F16) {
+                    const lds_cptr rr = rw + r * FP8_ROW;
+                    codes[j] = lds_ld<u32x2>(rr + 8 * ln);
+                    extra[j][0] = lds_ld<unsigned>(rr + FP8_SCALE_OFF + 4 * (ln >> 4));
+                } else if constexpr (L::V4MX) {
+                    const lds_cptr rr = rw + r * D_NOPE;
+                    const lds_cptr ra = rw + MX_ROPE_OFF + 128 * r + 16 * (ln & 7);
+                    const bool rp = ln >= 56;
+                    codes[j] = lds_ld<u32x2>(rp ? ra : rr + 8 * ln);
+                    extra[j] = lds_ld<u32x2>(rp ? ra + 8 : rr + DSA_MLA_V4_NOPE + 8 * (ln >> 5));
+                } else {
+                    codes[j] = lds_ld<u32x2>(rw + r * D_NOPE + 8 * ln);
+                    extra[j][0] = lds_ld<unsigned char>(rw + MX_SC_OFF + 16 * r + (ln >> 2));
+                }
             }
-            // (r & 3 is the wave)
-            lds_st<u32x4>(tb + r * L::STRIDE + 16 * (ln ^ (4 * wave)), out);
+#pragma unroll
+            for (int j = 0; j < DB; ++j) {
+                const int r = wave + NWAVE * (j0 + j);
+                u32x4 out;
+                if constexpr (F16) {
+                    const unsigned sb = extra[j][0];
+                    const float sc = __uint_as_float(sb);
+                    bad |= sb >= FP8_SCALE_LIMIT_BITS;
+                    const _Float16 m16 = (_Float16)__uint_as_float((sb & 0x007FFFFFu) | 0x3F800000u);
+                    const f16x2 mm = {m16, m16};
+                    const f16x2 h0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)codes[j][0], sc, false) * mm;
+                    const f16x2 h1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)codes[j][0], sc, true) * mm;
+                    const f16x2 h2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)codes[j][1], sc, false) * mm;
+                    const f16x2 h3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((int)codes[j][1], sc, true) * mm;
+                    out = u32x4{__builtin_bit_cast(unsigned, h0), __builtin_bit_cast(unsigned, h1),
+                                __builtin_bit_cast(unsigned, h2), __builtin_bit_cast(unsigned, h3)};
+                } else if constexpr (L::V4MX) {
+                    const uint64_t sc8 = ((uint64_t)extra[j][1] << 32) | extra[j][0];
+                    const unsigned e = (unsigned)(sc8 >> (8 * ((ln >> 2) & 7))) & 0xFFu;
+                    const u32x4 cv = mx_to_bf16(codes[j][0], codes[j][1], e);
+                    out = ln >= 56 ? u32x4{codes[j][0], codes[j][1], extra[j][0], extra[j][1]} : cv;
+                } else {
+                    out = mx_to_bf16(codes[j][0], codes[j][1], extra[j][0]);
+                }
+                // (r & 3 is the wave)
+                lds_st<u32x4>(tb + r * L::STRIDE + 16 * (ln ^ (4 * wave)), out);
+            }
+            if constexpr (DB < TILE / NWAVE) __builtin_amdgcn_sched_barrier(0);
         }
         range_bad |= bad;
     };
 
     // ---- S^T[16 rows x 16 heads] = K Q^T (A operand: row 16 rb + c16, dims 32 ks
     // + 8 g4 .. +7: chunk 4 ks + g4); kt: the tile, rt: its RoPE rows' base ----
-    auto qk16 = [&](lds_cptr kt, lds_cptr rt) -> f32x4 {
+    auto qk16 = [&](lds_cptr kt, lds_cptr rt, f32x4 (&s)[QB]) {
         const int ln = opaque(lane);
         const int row = 16 * rb + (ln & 15), lg = ln >> 4;
         const lds_cptr kn = kt + row * L::STRIDE + 16 * lg;
         const int x = 64 * (ln & 3);              // 64 (row & 3)
-        auto k_addr = [&](int ks) -> lds_cptr {
-            if (ks < KS_NOPE / 2) return kn + ((64 * (ks & 3)) ^ x) + 256 * (ks >> 2);
+        // (row + 16: the same swizzles)
+        auto k_addr = [&](int ks, int blk) -> lds_cptr {
+            if (ks < KS_NOPE / 2) return kn + ((64 * (ks & 3)) ^ x) + 256 * (ks >> 2) + 16 * blk * L::STRIDE;
             const int c = 4 * (ks - KS_NOPE / 2) + lg;
-            if constexpr (F16) return rt + row * FP8_ROW + FP8_ROPE_OFF + 16 * c;
-            else if constexpr (L::MX) return rt + MX_ROPE_OFF + 128 * row + 16 * (c ^ (row & 7));
-            else return rt + L::ROPE + 128 * row + 16 * (c ^ rope_sw(row));
+            if constexpr (F16) return rt + row * FP8_ROW + FP8_ROPE_OFF + 16 * c + 16 * blk * FP8_ROW;
+            else if constexpr (L::MX) return rt + MX_ROPE_OFF + 128 * row + 16 * (c ^ (row & 7)) + 2048 * blk;
+            else return rt + L::ROPE + 128 * row + 16 * (c ^ rope_sw(row)) + 2048 * blk;
         };
-        constexpr int KPF = 6;
-        u32x4 kb[KPF];
+        constexpr int KPF = HG == 64 ? (NF == DSA_KV_BF16_D512 ? 3 : 2) : 6;      // (deeper spills)
+        u32x4 kb[KPF][QB];
 #pragma unroll
-        for (int i = 0; i < KPF; ++i) kb[i] = lds_ld<u32x4>(k_addr(i));
-        // two accumulator chains (a single 16x16x32 chain is latency-bound)
+        for (int i = 0; i < KPF; ++i)
+#pragma unroll
+            for (int k = 0; k < QB; ++k) kb[i][k] = lds_ld<u32x4>(k_addr(i, k));
+        // two accumulator chains (a single 16x16x32 chain is latency-bound): the
+        // row blocks, or the even and odd k-steps
         f32x4 acc[2] = {};
 #pragma unroll
         for (int ks = 0; ks < L::NKS; ++ks) {
             __builtin_amdgcn_sched_barrier(0);
-            // (656-B rows: the NoPE k-steps on fp16 operands, RoPE on bf16)
-            if (F16 && ks < KS_NOPE / 2) acc[ks & 1] = mfma16_f16(kb[ks % KPF], qf[ks], acc[ks & 1]);
-            else acc[ks & 1] = mfma16_bf16(kb[ks % KPF], qf[ks], acc[ks & 1]);
-            if (ks + KPF < L::NKS) kb[ks % KPF] = lds_ld<u32x4>(k_addr(ks + KPF));
+#pragma unroll
+            for (int k = 0; k < QB; ++k) {
+                f32x4& a = acc[QB == 2 ? k : ks & 1];
+                // (656-B rows: the NoPE k-steps on fp16 operands, RoPE on bf16)
+                if (F16 && ks < KS_NOPE / 2) a = mfma16_f16(kb[ks % KPF][k], qf[ks], a);
+                else a = mfma16_bf16(kb[ks % KPF][k], qf[ks], a);
+                if (ks + KPF < L::NKS) kb[ks % KPF][k] = lds_ld<u32x4>(k_addr(ks + KPF, k));
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
-        return acc[0] + acc[1];
+        if constexpr (QB == 2) {
+            s[0] = acc[0];
+            s[1] = acc[1];
+        } else {
+            s[0] = acc[0] + acc[1];
+        }
     };
 
     // softmax state of head hq over this wave's rows: lane (g4, c16), value i
@@ -3010,14 +3050,16 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
     };
     auto get_max = [&](int k) { return fmaxf(s_red[2 * k * NARROW_HEADS + hq], s_red[(2 * k + 1) * NARROW_HEADS + hq]); };
 
-    // O^T accumulators: dims 128 wave + 32 m + (0..31) of the 32 heads: o[m]
-    f32x16 o[4];
+    // O^T accumulators: dims 128 wave + 32 m + (0..31) of heads 32 h + (0..31): o[h][m]
+    f32x16 o[QB][4];
     auto raw_slot = [&](int i) -> lds_ptr { return POOL + (i & 1) * L::RAWB; };
     auto tile_slot = [&](int i) -> lds_ptr { return RAW ? POOL + L::TILE0 : POOL + (i & 1) * L::SLOT; };
     resolve_chunk(0, true);
     for (int pass = 0;; ++pass) {
 #pragma unroll
-        for (int m = 0; m < 4; ++m) o[m] = f32x16{};
+        for (int h = 0; h < QB; ++h)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) o[h][m] = f32x16{};
         l_lane = 0.0f;
         s_max = -INFINITY;
         first_tile = pass == 0;
@@ -3029,8 +3071,11 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
 #pragma unroll
             for (int s0 = 0; s0 < 2; ++s0)
                 if (s0 < ntiles) issue_rows(load_rows(s0), RAW ? raw_slot(s0) : tile_slot(s0));
+            // row ids of the next tile to go out, read a step ahead (64 heads: when they
+            // are needed, to keep no registers for them)
             GatherRows gnext;
-            if (2 < ntiles) gnext = load_rows(2);
+            if constexpr (HG != 64)
+                if (2 < ntiles) gnext = load_rows(2);
             if (pass == 0 && c == 0) convert_q();
             // Q's last fragment, and so all of it, is waited for here, on every path to
             // the tile loop: left to its first use, the wait fell into the loop and
@@ -3055,67 +3100,91 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
                     tile_barrier();
                     __builtin_amdgcn_sched_barrier(0);
                     if (it >= 1 && it + 1 < ntiles) {
+                        if constexpr (HG == 64) gnext = load_rows(it + 1);
                         issue_rows(gnext, tile_slot(it + 1));
-                        if (it + 2 < ntiles) gnext = load_rows(it + 2);
+                        if constexpr (HG != 64)
+                            if (it + 2 < ntiles) gnext = load_rows(it + 2);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                f32x4 s = qk16(kt, rt);
+                f32x4 s[QB];
+                qk16(kt, rt, s);
                 const int rows_left = n_valid - it * TILE;
-                const int row0 = 16 * rb + 4 * g4;
+                const int row0 = 16 * rb + 4 * g4;         // block k: rows row0 + 16 k + i
                 if (first_tile) {
                     // the reference: the largest score of the list's first tile
                     float mx = -INFINITY;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) mx = fmaxf(mx, row0 + i < rows_left ? s[i] : -INFINITY);
-                    put_half(0, red4_max(mx));
-                    tile_barrier();
-                    m_ref = get_max(0) * c_s;
+                    for (int k = 0; k < QB; ++k)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            mx = fmaxf(mx, row0 + 16 * k + i < rows_left ? s[k][i] : -INFINITY);
+                    mx = red4_max(mx);
+                    if constexpr (QB == 1) {
+                        put_half(0, mx);
+                        tile_barrier();
+                        mx = get_max(0);
+                    }
+                    m_ref = mx * c_s;
                     first_tile = false;
                 }
                 if (rows_left < TILE) {
                     asm volatile("");
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) s[i] = row0 + i < rows_left ? s[i] : -INFINITY;
+                    for (int k = 0; k < QB; ++k)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) s[k][i] = row0 + 16 * k + i < rows_left ? s[k][i] : -INFINITY;
                 }
-                s_max = fmaxf(s_max, fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])));
+#pragma unroll
+                for (int k = 0; k < QB; ++k)
+                    s_max = fmaxf(s_max, fmaxf(fmaxf(s[k][0], s[k][1]), fmaxf(s[k][2], s[k][3])));
                 if (nchunks == 1 && ntiles == 1) {
                     // single-tile list: the exact sum folded into the reference,
                     // so that P is normalised when it is rounded
                     // (opus_attn/dsa_v32/common/host.cc:448-451)
-                    float lt = 0.0f;
+                    float l1 = 0.0f, m_fold = m_ref;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) lt += __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], c_s, -m_ref));
-                    put_half(1, red4_sum(lt));
-                    tile_barrier();
-                    float l1 = s_red[2 * NARROW_HEADS + hq] + s_red[3 * NARROW_HEADS + hq], m_fold = m_ref;
+                    for (int k = 0; k < QB; ++k)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) l1 += __builtin_amdgcn_exp2f(__builtin_fmaf(s[k][i], c_s, -m_ref));
+                    l1 = red4_sum(l1);
+                    if constexpr (QB == 1) {
+                        put_half(1, l1);
+                        tile_barrier();
+                        l1 = s_red[2 * NARROW_HEADS + hq] + s_red[3 * NARROW_HEADS + hq];
+                    }
                     // (an attention sink joins the sum: mla_v4_host.cc:469-472)
                     if (D512 && p.attn_sink)
                         add_sink(l1, m_ref, p.attn_sink[min(hbase + hq, p.H - 1)] * LOG2E, l1, m_fold);
                     m_ref = m_fold + __builtin_amdgcn_logf(l1);
                 }
-                f32x4 e;
+                // P of rows row0 + 16 k + i: PV k-step u (the 16-row block), lane half
+                // g4 & 1, positions 4 (g4 >> 1) + i (the rows the V reads pair with them)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) e[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], c_s, -m_ref));
-                l_lane += (e[0] + e[1]) + (e[2] + e[3]);
-                // P of rows 16 rb + 4 g4 + i: PV k-step u = rb, lane half g4 & 1,
-                // positions 4 (g4 >> 1) + i (the rows the V reads pair with them)
-                u32x2 pw;
-                if constexpr (F16) {
-                    // fp16 P for the fp16 PV MFMAs (finite below 2^16: TAU = 15)
-                    const f16x2 p01 = {(_Float16)e[0], (_Float16)e[1]}, p23 = {(_Float16)e[2], (_Float16)e[3]};
-                    pw = u32x2{__builtin_bit_cast(unsigned, p01), __builtin_bit_cast(unsigned, p23)};
-                } else {
-                    pw = __builtin_bit_cast(u32x2, __builtin_convertvector(e, bf16x4));
+                for (int k = 0; k < QB; ++k) {
+                    f32x4 e;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) e[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[k][i], c_s, -m_ref));
+                    l_lane += (e[0] + e[1]) + (e[2] + e[3]);
+                    u32x2 pw;
+                    if constexpr (F16) {
+                        // fp16 P for the fp16 PV MFMAs (finite below 2^16: TAU = 15)
+                        const f16x2 p01 = {(_Float16)e[0], (_Float16)e[1]}, p23 = {(_Float16)e[2], (_Float16)e[3]};
+                        pw = u32x2{__builtin_bit_cast(unsigned, p01), __builtin_bit_cast(unsigned, p23)};
+                    } else {
+                        pw = __builtin_bit_cast(u32x2, __builtin_convertvector(e, bf16x4));
+                    }
+                    lds_st<u32x2>(PX + ((2 * (rb + k) + (g4 & 1)) * HG + hq) * 16 + 8 * (g4 >> 1), pw);
                 }
-                lds_st<u32x2>(PX + ((2 * rb + (g4 & 1)) * NARROW_HEADS + hq) * 16 + 8 * (g4 >> 1), pw);
                 tile_barrier();
                 if constexpr (RAW) {
                     // every wave is done with this raw slot: tile it+2 into it
                     __builtin_amdgcn_sched_barrier(0);
                     if (it + 2 < ntiles) {
+                        if constexpr (HG == 64) gnext = load_rows(it + 2);
                         issue_rows(gnext, raw_slot(it));
-                        if (it + 3 < ntiles) gnext = load_rows(it + 3);
+                        if constexpr (HG != 64)
+                            if (it + 3 < ntiles) gnext = load_rows(it + 3);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -3135,11 +3204,18 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
                 };
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
-                    const u32x4 pb = lds_ld<u32x4>(PX + ((2 * u + vhi) * NARROW_HEADS + (vln & 31)) * 16);
+                    u32x4 pb[QB];
+#pragma unroll
+                    for (int h = 0; h < QB; ++h)
+                        pb[h] = lds_ld<u32x4>(PX + ((2 * u + vhi) * HG + 32 * h + (vln & 31)) * 16);
 #pragma unroll
                     for (int m = 0; m < 4; ++m) {
-                        if constexpr (F16) o[m] = mfma_f16(v_frag(u, m), pb, o[m]);
-                        else o[m] = mfma_bf16(v_frag(u, m), pb, o[m]);
+                        const u32x4 v = v_frag(u, m);
+#pragma unroll
+                        for (int h = 0; h < QB; ++h) {
+                            if constexpr (F16) o[h][m] = mfma_f16(v, pb[h], o[h][m]);
+                            else o[h][m] = mfma_bf16(v, pb[h], o[h][m]);
+                        }
                     }
                 }
             }
@@ -3149,11 +3225,13 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
         // per head: the largest score of the pass over both row halves (log2
         // units); NaN compares false.  A head past the reference by more than
         // TAU restarts the workgroup once, with the exact maximum.
-        put_half(2, red4_max(s_max));
+        float top = red4_max(s_max);
+        if constexpr (QB == 1) put_half(2, top);
         // (the barrier also ends every wave's use of the tile buffers: a
         // restart refills them, the epilogue stages O in them)
         tile_barrier();
-        const float top = get_max(2) * c_s;
+        if constexpr (QB == 1) top = get_max(2);
+        top *= c_s;
         if (pass == 0 && __builtin_amdgcn_ballot_w64(top - m_ref > L::TAU) != 0 && lane == 0) s_misc[NWAVE] = 1;
         tile_barrier();
         if (pass != 0 || s_misc[NWAVE] == 0) break;
@@ -3161,90 +3239,118 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
     }
 
     // ---- epilogue: O / l and LSE, final (bf16) or a split's partial (fp32) ----
-    put_half(3, red4_sum(l_lane));
-    if (rb == 0 && g4 == 0) s_red[8 * NARROW_HEADS + hq] = m_ref;
+    if constexpr (QB == 1) {
+        put_half(3, red4_sum(l_lane));
+        if (rb == 0 && g4 == 0) s_red[8 * NARROW_HEADS + hq] = m_ref;
+    } else {
+        const float l_all = red4_sum(l_lane);
+        if (g4 == 0) {
+            s_red[hq] = l_all;
+            s_red[HG + hq] = m_ref;
+        }
+    }
     if (F16 && range_bad) s_misc[NWAVE + 1] = 1;
     tile_barrier();
     // A list cut short, or (656-B rows) a scale outside the fp16 path's range:
     // NaN outputs, never a silently truncated or wrong attention.
     const bool nan_out = truncated || (F16 && s_misc[NWAVE + 1] != 0);
-    const float l_rows = s_red[6 * NARROW_HEADS + r32] + s_red[7 * NARROW_HEADS + r32];
-    const float m_head = s_red[8 * NARROW_HEADS + r32];
     const bool has = any_rows;
-    float l = l_rows, m_fin = m_head, o_scale = 1.0f;
-    if constexpr (D512)
-        if (p.attn_sink) {
-            add_sink(l_rows, m_head, p.attn_sink[min(head_g, p.H - 1)] * LOG2E, l, m_fin);
-            o_scale = __builtin_amdgcn_exp2f(m_head - m_fin);
-        }
-    const float inv =
-        nan_out ? __builtin_nanf("") : (has ? (nchunks == 1 && ntiles == 1 ? 1.0f : o_scale / l) : 0.0f);
+    float inv[QB], lse_v[QB];                     // of heads hbase + 32 h + r32
+#pragma unroll
+    for (int h = 0; h < QB; ++h) {
+        const int hh = 32 * h + r32;
+        const float l_rows =
+            QB == 1 ? s_red[6 * NARROW_HEADS + hh] + s_red[7 * NARROW_HEADS + hh] : s_red[hh];
+        const float m_head = s_red[(QB == 1 ? 8 * NARROW_HEADS : HG) + hh];
+        float l = l_rows, m_fin = m_head, o_scale = 1.0f;
+        if constexpr (D512)
+            if (p.attn_sink) {
+                add_sink(l_rows, m_head, p.attn_sink[min(hbase + hh, p.H - 1)] * LOG2E, l, m_fin);
+                o_scale = __builtin_amdgcn_exp2f(m_head - m_fin);
+            }
+        inv[h] = nan_out ? __builtin_nanf("") : (has ? (nchunks == 1 && ntiles == 1 ? 1.0f : o_scale / l) : 0.0f);
+        lse_v[h] = nan_out ? __builtin_nanf("") : (m_fin + __builtin_amdgcn_logf(l)) * LN2;
+    }
     const int64_t qrow = (int64_t)b * p.s_q + t;
     const bool planned = !D512 && p.plan_items;
     const bool to_part = p.part_o != nullptr && (!planned || item_slot >= 0);
     const int64_t part_row = planned ? (int64_t)item_slot : (int64_t)split * p.B * p.s_q + qrow;
-    if (wave == 0 && hi == 0 && head_g < p.H) {
-        const float lse_v = nan_out ? __builtin_nanf("") : (m_fin + __builtin_amdgcn_logf(l)) * LN2;
-        if (!to_part) {
-            if (p.lse) p.lse[qrow * p.H + head_g] = has || nan_out ? lse_v : INFINITY;
-        } else {
-            p.part_lse[part_row * p.H + head_g] = has || nan_out ? lse_v : -FLT_MAX;
+    if (wave == 0 && hi == 0) {
+#pragma unroll
+        for (int h = 0; h < QB; ++h) {
+            const int head_g = hbase + 32 * h + r32;
+            if (head_g >= p.H) continue;
+            if (!to_part) {
+                if (p.lse) p.lse[qrow * p.H + head_g] = has || nan_out ? lse_v[h] : INFINITY;
+            } else {
+                p.part_lse[part_row * p.H + head_g] = has || nan_out ? lse_v[h] : -FLT_MAX;
+            }
         }
     }
-    // lane (hi, r32), reg 4g + i of o[m]: dim 128 wave + 32 m + 8 g + 4 hi + i of head r32.
-    // Staged through LDS (each wave its own region) so that the global stores
-    // write whole row pieces of the wave's 128 dims.
+    // lane (hi, r32), reg 4g + i of o[h][m]: dim 128 wave + 32 m + 8 g + 4 hi + i of head
+    // 32 h + r32.  Staged through LDS, 32 heads at a time, each wave in its own region
+    // (its LDS accesses run in order: no barrier), so that the global stores write
+    // whole row pieces of the wave's 128 dims.
     const int ln = opaque(lane);
-    if (!to_part) {
-        constexpr int OST = 2 * 128 + 16;               // staged head row: 128 bf16 + pad
-        static_assert(NWAVE * 32 * OST <= L::REDO, "O stage fits the buffers");
-        const lds_ptr stg = POOL + wave * 32 * OST;
-        const int st_w = opaque(r32 * OST + 8 * hi);
+    constexpr int OST = 2 * 128 + 16;               // staged head row: 128 bf16 + pad
+    constexpr int PST = 4 * 128 + 16;               // 128 floats + pad
+    static_assert(NWAVE * 32 * OST <= L::STAGE, "O stage fits below P");
+    static_assert(NWAVE * 32 * PST <= L::STAGE + L::PB && (HG != 64 || NWAVE * 32 * PST <= L::MISCO),
+                  "partial stage fits the buffers");
+    const bool o16 = ((p.o_sb | p.o_st | p.o_sh) & 7) == 0 && ((uintptr_t)p.out & 15) == 0;
+    // (64 heads: the stage of 512-value rows' partials reaches into P, where the
+    // sums were: every wave has read them)
+    if constexpr (HG == 64 && NWAVE * 32 * PST > L::STAGE) tile_barrier();
 #pragma unroll
-        for (int m = 0; m < 4; ++m)
+    for (int h = 0; h < QB; ++h) {
+        const int h0 = hbase + 32 * h;
+        if (!to_part) {
+            const lds_ptr stg = POOL + wave * 32 * OST;
+            const int st_w = opaque(r32 * OST + 8 * hi);
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const f32x4 v4 = {o[m][4 * g] * inv, o[m][4 * g + 1] * inv, o[m][4 * g + 2] * inv,
-                                  o[m][4 * g + 3] * inv};
-                lds_st<u32x2>(stg + st_w + 2 * (32 * m + 8 * g), __builtin_bit_cast(u32x2, __builtin_convertvector(v4, bf16x4)));
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const f32x16& a = o[h][m];
+                    const f32x4 v4 = {a[4 * g] * inv[h], a[4 * g + 1] * inv[h], a[4 * g + 2] * inv[h], a[4 * g + 3] * inv[h]};
+                    lds_st<u32x2>(stg + st_w + 2 * (32 * m + 8 * g),
+                                  __builtin_bit_cast(u32x2, __builtin_convertvector(v4, bf16x4)));
+                }
+            __bf16* const orow = p.out + (int64_t)b * p.o_sb + (int64_t)t * p.o_st;
+            // lane (k, c): head row 4k + c / 16 of the block, dims 8 (c % 16) .. +7 of the wave's 128
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int r = 4 * k + (ln >> 4);
+                if (h0 + r >= p.H) break;
+                const u32x4 v = lds_ld<u32x4>(stg + r * OST + 16 * (ln & 15));
+                __bf16* const dst = orow + (int64_t)(h0 + r) * p.o_sh + 128 * wave + 8 * (ln & 15);
+                if (o16) {
+                    *reinterpret_cast<u32x4*>(dst) = v;
+                } else {
+                    reinterpret_cast<u32x2*>(dst)[0] = u32x2{v[0], v[1]};
+                    reinterpret_cast<u32x2*>(dst)[1] = u32x2{v[2], v[3]};
+                }
             }
-        __bf16* const orow = p.out + (int64_t)b * p.o_sb + (int64_t)t * p.o_st;
-        const bool o16 = ((p.o_sb | p.o_st | p.o_sh) & 7) == 0 && ((uintptr_t)p.out & 15) == 0;
-        // lane (k, c): head row 4k + c / 16 of the group, dims 8 (c % 16) .. +7 of the wave's 128
+        } else {
+            const lds_ptr stg = POOL + wave * 32 * PST;
+            const int st_w = opaque(r32 * PST + 16 * hi);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int r = 4 * k + (ln >> 4);
-            if (hbase + r >= p.H) break;
-            const u32x4 v = lds_ld<u32x4>(stg + r * OST + 16 * (ln & 15));
-            __bf16* const dst = orow + (int64_t)(hbase + r) * p.o_sh + 128 * wave + 8 * (ln & 15);
-            if (o16) {
-                *reinterpret_cast<u32x4*>(dst) = v;
-            } else {
-                reinterpret_cast<u32x2*>(dst)[0] = u32x2{v[0], v[1]};
-                reinterpret_cast<u32x2*>(dst)[1] = u32x2{v[2], v[3]};
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const f32x16& a = o[h][m];
+                    const f32x4 v4 = {a[4 * g] * inv[h], a[4 * g + 1] * inv[h], a[4 * g + 2] * inv[h], a[4 * g + 3] * inv[h]};
+                    lds_st<f32x4>(stg + st_w + 4 * (32 * m + 8 * g), v4);
+                }
+            const int64_t prow0 = part_row * p.H + h0;
+            // lane (j, c): head row 2k + j of the block, floats 4c..4c+3 of the wave's 128
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const int r = 2 * k + (ln >> 5);
+                const f32x4 v = lds_ld<f32x4>(stg + r * PST + 16 * (ln & 31));
+                if (h0 + r < p.H)
+                    *reinterpret_cast<f32x4*>(p.part_o + (prow0 + r) * D_VO + 128 * wave + 4 * (ln & 31)) = v;
             }
-        }
-    } else {
-        constexpr int PST = 4 * 128 + 16;               // staged head row: 128 floats + pad
-        static_assert(NWAVE * 32 * PST <= L::REDO, "partial stage fits the buffers");
-        const lds_ptr stg = POOL + wave * 32 * PST;
-        const int st_w = opaque(r32 * PST + 16 * hi);
-#pragma unroll
-        for (int m = 0; m < 4; ++m)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const f32x4 v4 = {o[m][4 * g] * inv, o[m][4 * g + 1] * inv, o[m][4 * g + 2] * inv,
-                                  o[m][4 * g + 3] * inv};
-                lds_st<f32x4>(stg + st_w + 4 * (32 * m + 8 * g), v4);
-            }
-        const int64_t prow0 = part_row * p.H + hbase;
-        // lane (j, c): head row 2k + j of the group, floats 4c..4c+3 of the wave's 128
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const int r = 2 * k + (ln >> 5);
-            const f32x4 v = lds_ld<f32x4>(stg + r * PST + 16 * (ln & 31));
-            if (hbase + r < p.H)
-                *reinterpret_cast<f32x4*>(p.part_o + (prow0 + r) * D_VO + 128 * wave + 4 * (ln & 31)) = v;
         }
     }
 }
@@ -3767,25 +3873,39 @@ bool heads_ok(int32_t H, int64_t tokens) {
 // Forward kernel of a call of `tokens` query tokens (work items) and H heads.
 //   WIDE    128 heads per workgroup, one per CU (dsa_mla_fwd_kernel)
 //   NARROW  32 heads, one workgroup per CU (dsa_mla_fwd_narrow_kernel)
-//   PAIR    32 heads, two workgroups per CU (dsa_mla_fwd_pair_kernel)
-// 32-head workgroups where the 128-head kernel would compute at least 2x padding
-// heads (H <= 64; V4 fp8 rows H <= 32: two groups convert every row twice, 763
-// against 711 us at H = 64, 2048 queries of 1152 rows), or could not occupy half
-// the GPU even with its splits (fewer than 128 workgroups at wide_splits splits).
-// PAIR when there are more of them than CUs, so that a second one on a CU has
-// something to fill: 4096 queries x 2048 rows at H = 16 in bf16 747 us, NARROW
-// 1226; at H = 64 (2048 queries) 759, WIDE 945.
-enum Kern { WIDE, NARROW, PAIR };
+//   PAIR    32 heads, two workgroups per CU (dsa_mla_fwd_pair_kernel<., 32>)
+//   PAIR64  64 heads, two workgroups per CU (dsa_mla_fwd_pair_kernel<., 64>)
+// The three small ones where the 128-head kernel would compute at least 2x padding
+// heads (H <= 64), or could not occupy half the GPU even with its splits (fewer
+// than 128 workgroups at wide_splits splits).  Splits are counted for 32-head
+// workgroups (narrow_splits); given them, `units` query tokens (or plan items)
+// x splits run
+//   PAIR64  at 33..64 heads when the units alone outnumber the CUs: below that
+//           each would have a CU to itself, and twice as many workgroups of 32
+//           heads are faster (MXFP8, 256 units, 92.3 against 93.3 us, 100 tokens
+//           with their plan 41.8 against 43.3; above, 300 units at H = 64 136 us
+//           against 226 on WIDE)
+//   PAIR    when 32-head workgroups outnumber the CUs, so that a second one on a
+//           CU has something to fill (4096 queries x 2048 rows, H = 16, bf16:
+//           747 us, NARROW 1226), and for the formats without a narrow kernel
+//   NARROW  otherwise
+enum Kern { WIDE, NARROW, PAIR, PAIR64 };
 int narrow_groups(int32_t H) { return (H + NARROW_HEADS - 1) / NARROW_HEADS; }
-int groups_of(Kern k, int32_t H) { return k == WIDE ? head_groups(H) : narrow_groups(H); }
+int groups_of(Kern k, int32_t H) {
+    return k == WIDE ? head_groups(H) : (k == PAIR64 ? (H + 63) / 64 : narrow_groups(H));
+}
 bool has_narrow(int fmt) { return fmt == DSA_KV_BF16 || fmt == DSA_KV_BF16_D512 || fmt == DSA_KV_FP8_656; }
 bool narrow_path(int fmt, int64_t tokens, int32_t H, int wide_splits) {
     if (H < 1 || tokens * narrow_groups(H) > INT32_MAX) return false;
-    if (H <= (fmt == DSA_KV_MXFP8_V4 ? 32 : 64)) return true;
+    if (H <= 64) return true;
     return has_narrow(fmt) && tokens * head_groups(H) * wide_splits < 128;
 }
-// NARROW or PAIR for `wgs` 32-head workgroups
-Kern narrow_kern(int fmt, int64_t wgs) { return !has_narrow(fmt) || wgs > 256 ? PAIR : NARROW; }
+Kern pair_kern(int64_t units, int32_t H) {
+    return H > 32 && H <= 64 && units > 256 ? PAIR64 : PAIR;
+}
+Kern narrow_kern(int fmt, int64_t units, int32_t H) {
+    return !has_narrow(fmt) || units * narrow_groups(H) > 256 ? pair_kern(units, H) : NARROW;
+}
 
 // Splits of a call whose `wgs` unsplit workgroups would leave CUs idle: as many
 // as fit one round of the 256 CUs (a workgroup takes a whole CU), with at least
@@ -3826,7 +3946,7 @@ int decode_splits(const dsa_mla_decode_args* a, Kern* kern, bool one_per_cu = fa
     const int ns = a->num_splits ? a->num_splits
                                  : narrow_splits(a->kv_format, tokens * groups, (int64_t)a->topk + DECODE_MIN - 1, DECODE_MIN,
                                                one_per_cu);
-    *kern = narrow_kern(a->kv_format, tokens * groups * ns);
+    *kern = narrow_kern(a->kv_format, tokens * ns, a->H);
     return ns;
 }
 
@@ -3866,12 +3986,16 @@ size_t decode_ws_bytes(const dsa_mla_decode_args* a, int ns) {
 
 int launch_fwd(const FwdParams& fp, int fmt, int B, int s_q, int ns, hipStream_t st, Kern kern = WIDE) {
     dim3 grid((unsigned)((int64_t)B * fp.hgroups), s_q, ns), block(NTHR);
-    if (kern == PAIR) {
-        auto fn = fmt == DSA_KV_BF16 ? dsa_mla_fwd_pair_kernel<DSA_KV_BF16>
-                  : fmt == DSA_KV_FP8_656 ? dsa_mla_fwd_pair_kernel<DSA_KV_FP8_656>
-                  : fmt == DSA_KV_MXFP8 ? dsa_mla_fwd_pair_kernel<DSA_KV_MXFP8>
-                  : fmt == DSA_KV_MXFP8_V4 ? dsa_mla_fwd_pair_kernel<DSA_KV_MXFP8_V4>
-                                           : dsa_mla_fwd_pair_kernel<DSA_KV_BF16_D512>;
+    if (kern == PAIR || kern == PAIR64) {
+        auto pick = [&](auto hg) {
+            constexpr int HG = decltype(hg)::value;
+            return fmt == DSA_KV_BF16 ? dsa_mla_fwd_pair_kernel<DSA_KV_BF16, HG>
+                   : fmt == DSA_KV_FP8_656 ? dsa_mla_fwd_pair_kernel<DSA_KV_FP8_656, HG>
+                   : fmt == DSA_KV_MXFP8 ? dsa_mla_fwd_pair_kernel<DSA_KV_MXFP8, HG>
+                   : fmt == DSA_KV_MXFP8_V4 ? dsa_mla_fwd_pair_kernel<DSA_KV_MXFP8_V4, HG>
+                                            : dsa_mla_fwd_pair_kernel<DSA_KV_BF16_D512, HG>;
+        };
+        auto fn = kern == PAIR64 ? pick(std::integral_constant<int, 64>{}) : pick(std::integral_constant<int, 32>{});
         hipLaunchKernelGGL(fn, grid, block, 0, st, fp);
     } else if (kern == NARROW) {
         auto fn = fmt == DSA_KV_BF16 ? dsa_mla_fwd_narrow_kernel<DSA_KV_BF16>
@@ -3937,7 +4061,8 @@ int csr_plan_build(const int32_t* kv_indptr, int B, int s_q, int H, int max_len,
 int csr_plan_launch(FwdParams& fp, int fmt, int max_len, void* ws, bool build, hipStream_t st) {
     // 32-head workgroups for up to 64 heads (the plan's rows are a device matter:
     // its items number about 256 or more, so PAIR)
-    const Kern kern = narrow_path(fmt, (int64_t)fp.B * fp.s_q + PLAN_TARGET, fp.H, PLAN_TARGET) ? PAIR : WIDE;
+    const Kern kern = narrow_path(fmt, (int64_t)fp.B * fp.s_q + PLAN_TARGET, fp.H, PLAN_TARGET)
+                          ? pair_kern((int64_t)fp.B * fp.s_q, fp.H) : WIDE;
     fp.hgroups = groups_of(kern, fp.H);
     const CsrPlanLayout L = csr_plan_layout(fp.B, fp.s_q, fp.H, max_len);
     char* w = (char*)ws;
@@ -4050,7 +4175,7 @@ int prefill_plan(int fmt, int64_t N, int32_t H, int requested, int64_t max_list,
     *kern = WIDE;
     if (!narrow_path(fmt, N, H, wide)) return wide;
     const int ns = requested > 0 ? requested : narrow_splits(fmt, N * narrow_groups(H), max_list, PREFILL_MIN);
-    *kern = narrow_kern(fmt, N * narrow_groups(H) * ns);
+    *kern = narrow_kern(fmt, N * ns, H);
     return ns;
 }
 size_t prefill_ws_bytes(int ns, int64_t N, int H) {
@@ -4299,7 +4424,7 @@ int dsa_mla_decode_csr(const dsa_mla_decode_csr_args* a, void* ws, size_t ws_byt
     // uniform splits (no work plan) of few query rows or few heads: 32-head workgroups
     const int64_t rows_q = (int64_t)a->B * a->s_q;
     const Kern kern = ns >= 1 && narrow_path(a->kv_format, rows_q, a->H, ns)
-                          ? narrow_kern(a->kv_format, rows_q * narrow_groups(a->H) * ns) : WIDE;
+                          ? narrow_kern(a->kv_format, rows_q * ns, a->H) : WIDE;
     FwdParams fp{};
     fp.H = a->H;
     fp.hgroups = groups_of(kern, a->H);
@@ -4344,7 +4469,8 @@ int dsa_mla_decode_mxfp8(const dsa_mla_decode_mxfp8_args* a, void* ws, size_t ws
     if (need && (!ws || ws_bytes < need || ((uintptr_t)ws & 15))) return DSA_ERR_WORKSPACE;
     if (a->B == 0) return DSA_OK;
     hipStream_t st = (hipStream_t)stream;
-    const Kern kern = ns >= 1 && narrow_path(DSA_KV_MXFP8, (int64_t)a->B * a->s_q, a->H, ns) ? PAIR : WIDE;
+    const Kern kern = ns >= 1 && narrow_path(DSA_KV_MXFP8, (int64_t)a->B * a->s_q, a->H, ns)
+                          ? pair_kern((int64_t)a->B * a->s_q * ns, a->H) : WIDE;
     FwdParams fp{};
     fp.H = a->H;
     fp.hgroups = groups_of(kern, a->H);
