@@ -1409,8 +1409,8 @@ def c5_leg(args, dev, res):
                                    "kernel_avg_us": round(pk_ms * 1e3, 1)}}
     defer_cpu(args, "CPU baseline (oracle) on a c5 sample", res["prefill"],
               lambda: cpu_baseline_prefill(p, args.cpu_prefill_sample, pV))
-    # The c5 lists with fewer heads (the first H heads of c5's Q): H <= 64 runs on 32-head
-    # workgroups, H = 64 on 128-head ones; the fraction is of useful flops (H heads).
+    # The c5 lists with fewer heads (the first H heads of c5's Q), on 32- and (H = 64) 64-head
+    # workgroups, two to a CU; the fraction is of useful flops (H heads).
     import torch
     from opfoundry_amd import dsa
     res["prefill_heads"] = {}
