@@ -74,6 +74,7 @@ struct IxParams {
     float* scores;
     int64_t s_stride;
     int32_t s_q, n_cols, causal, tgroups;
+    int32_t parts;               // > 0: workgroups per group (one sequence); 0: an even deal of all chunks
 };
 
 // Positions j of token t of sequence b: j < min(len(b, t), n_cols).
@@ -170,39 +171,53 @@ dsa_indexer_kernel(const IxParams p) {
         const int g = (int)g64, b = seq_of(g), t0 = (g - b * p.tgroups) * TPW;
         return (uint32_t)((ix_len(p, p.seq_lens[b], min(t0 + TPW, p.s_q) - 1) + IX_CHUNK - 1) / IX_CHUNK);
     };
-    uint64_t all = 0;
-    uint32_t n0 = 0, end0 = 0;                 // of groups 0 .. IX_NTHR - 1
-    for (int64_t g0 = 0; g0 < p.groups; g0 += IX_NTHR) {
-        const uint32_t n = group_chunks(g0 + tid);
-        uint32_t tot;
-        const uint32_t end = ix_scan(n, s_part, &tot);
-        if (g0 == 0) { n0 = n; end0 = end; }
-        all += tot;
-    }
     const uint32_t G = gridDim.x, x = blockIdx.x;
-    const uint64_t each = all >> 32 ? all / G : (uint64_t)((uint32_t)all / G);
-    const uint32_t more = (uint32_t)(all - each * G);       // the first `more` workgroups take one chunk more
-    const uint64_t first = each * x + min(x, more);
-    int64_t left = (int64_t)(each + (x < more ? 1 : 0));
-    if (left <= 0) return;
-    {
-        // the group holding chunk `first`: exactly one thread finds it
-        const bool once = p.groups <= IX_NTHR;
-        uint64_t base = 0;
-        for (int64_t g0 = 0; g0 < p.groups && base <= first; g0 += IX_NTHR) {
-            const uint32_t n = once ? n0 : group_chunks(g0 + tid);
-            uint32_t tot = 0;
-            const uint64_t end = base + (once ? end0 : ix_scan(n, s_part, &tot));
-            if (end > first && end - n <= first) {
-                s_at[0] = (int)(g0 + tid);
-                s_at[1] = (int)(first - (end - n));
-            }
-            base += tot;
+    int g, c0;
+    int64_t left;
+    if (p.parts) {
+        // one sequence: its groups' lists differ by less than s_q positions, so
+        // that workgroups of one group each are as even, start once instead of
+        // up to twice and need no scan
+        g = (int)(x / (uint32_t)p.parts);
+        const uint32_t part = x - (uint32_t)g * (uint32_t)p.parts, n = group_chunks(g);
+        const uint32_t each = n / (uint32_t)p.parts, more = n - each * (uint32_t)p.parts;
+        c0 = (int)(each * part + min(part, more));
+        left = each + (part < more ? 1 : 0);
+        if (left <= 0) return;
+    } else {
+        uint64_t all = 0;
+        uint32_t n0 = 0, end0 = 0;                 // of groups 0 .. IX_NTHR - 1
+        for (int64_t g0 = 0; g0 < p.groups; g0 += IX_NTHR) {
+            const uint32_t n = group_chunks(g0 + tid);
+            uint32_t tot;
+            const uint32_t end = ix_scan(n, s_part, &tot);
+            if (g0 == 0) { n0 = n; end0 = end; }
+            all += tot;
         }
-        __syncthreads();
+        const uint64_t each = all >> 32 ? all / G : (uint64_t)((uint32_t)all / G);
+        const uint32_t more = (uint32_t)(all - each * G);       // the first `more` workgroups take one chunk more
+        const uint64_t first = each * x + min(x, more);
+        left = (int64_t)(each + (x < more ? 1 : 0));
+        if (left <= 0) return;
+        {
+            // the group holding chunk `first`: exactly one thread finds it
+            const bool once = p.groups <= IX_NTHR;
+            uint64_t base = 0;
+            for (int64_t g0 = 0; g0 < p.groups && base <= first; g0 += IX_NTHR) {
+                const uint32_t n = once ? n0 : group_chunks(g0 + tid);
+                uint32_t tot = 0;
+                const uint64_t end = base + (once ? end0 : ix_scan(n, s_part, &tot));
+                if (end > first && end - n <= first) {
+                    s_at[0] = (int)(g0 + tid);
+                    s_at[1] = (int)(first - (end - n));
+                }
+                base += tot;
+            }
+            __syncthreads();
+        }
+        g = __builtin_amdgcn_readfirstlane(s_at[0]);
+        c0 = __builtin_amdgcn_readfirstlane(s_at[1]);
     }
-    int g = __builtin_amdgcn_readfirstlane(s_at[0]);
-    int c0 = __builtin_amdgcn_readfirstlane(s_at[1]);
 
     const lds_ptr ring = (lds_ptr)s_k + wave * 2 * IX_SLOT;
     LDS_AS int32_t* const ents = (LDS_AS int32_t*)s_ent + wave * IX_LOOK * 64;
@@ -375,7 +390,15 @@ int launch_ix(IxParams& p, int B, hipStream_t st) {
     // two workgroups per CU, but no more than the chunks the lists can hold
     const int64_t most = (p.n_cols + (int64_t)IX_CHUNK - 1) / IX_CHUNK;
     const bool once = p.tgroups == 1;          // (always for NB < 4: chosen by s_q)
-    const int64_t wgs = p.groups >= IX_WGS || most >= IX_WGS ? IX_WGS : std::min<int64_t>(p.groups * most, IX_WGS);
+    int64_t wgs = p.groups >= IX_WGS || most >= IX_WGS ? IX_WGS : std::min<int64_t>(p.groups * most, IX_WGS);
+    // One sequence, and whole workgroups per group that fill at least 7/8 of the
+    // grid an even deal would have: 512 tokens of 32 heads x 8000 positions 48.5 us
+    // (about 53 by an even deal, whose workgroups mostly span two groups); at worst 7/8 of
+    // the places are used, where a second start costs about as much.
+    if (B == 1 && wgs / p.groups * p.groups >= wgs - wgs / 8) {
+        p.parts = (int32_t)(wgs / p.groups);
+        wgs = p.parts * p.groups;
+    }
     if (once) hipLaunchKernelGGL((dsa_indexer_kernel<HI, NB, true>), dim3((unsigned)wgs), dim3(IX_NTHR), 0, st, p);
     else if constexpr (NB == 4)
         hipLaunchKernelGGL((dsa_indexer_kernel<HI, NB, false>), dim3((unsigned)wgs), dim3(IX_NTHR), 0, st, p);

@@ -28,6 +28,21 @@ def test_row_blocks(dev, H_I, s_q):
     check(got, q, w, k, ref, f"indexer blocks H_I={H_I} s_q={s_q}")
 
 
+@pytest.mark.parametrize("H_I,s_q,n", [(64, 1, 70001), (64, 9, 300), (32, 17, 4500), (64, 130, 1100), (128, 600, 260)])
+def test_one_sequence(dev, H_I, s_q, n):
+    """One sequence: whole workgroups per token group (one group; as many as chunks; parts that
+    do not divide a list's chunks), and 600 groups, which are dealt out evenly."""
+    rng = np.random.default_rng(440 + s_q)
+    seq = np.array([n], np.int32)
+    q, w, k, bt = paged(rng, 1, seq, 64, H_I, s_q)
+    print(f"[case] indexer one sequence H_I={H_I} s_q={s_q} n={n}", flush=True)
+    ref = oracle.indexer_scores(q, w, k, seq, block_table=bt, block_size=64, causal=True, n_cols=n)
+    got = dsa.indexer_scores(t16(q, dev), torch.from_numpy(w).to(dev), t16(k, dev), torch.from_numpy(seq).to(dev),
+                             block_table=torch.from_numpy(bt).to(dev), block_size=64, causal=True, n_cols=n)
+    torch.cuda.synchronize()
+    check(got, q, w, k, ref, f"indexer one sequence s_q={s_q}")
+
+
 def test_nan_row_scores_zero(dev):
     """max(NaN, 0) is 0: a cache row of NaNs scores 0, its neighbours are untouched."""
     rng = np.random.default_rng(450)
