@@ -3919,16 +3919,47 @@ int one_round_splits(int64_t wgs, int64_t max_list, int64_t min_entries, int rou
     const int64_t by_len = std::max<int64_t>(1, max_list / min_entries);
     return (int)std::min<int64_t>(std::min<int64_t>(round / wgs, by_len), DSA_MLA_MAX_SPLITS);
 }
-// The same for 32-head workgroups, of which two fit a CU.  656-B rows fill both
-// places (a workgroup waits through its conversions): 130 tokens of 16 heads 68
-// us in 3 splits, 108 unsplit; 74 tokens 42 against 50 in 3.  bf16 rows gain
-// less from a second workgroup than its partials cost (40 tokens of 32 heads 34
-// us in 6 splits, 42 in 12), except where one round of CUs would leave the call
-// unsplit and a third of them idle (130 tokens of 16 heads 73 us in 3 splits, 84
-// unsplit; 200 tokens 104 in 2, 91 unsplit).
-int narrow_splits(int fmt, int64_t wgs, int64_t max_list, int64_t min_entries, bool one_per_cu = false) {
-    const bool two = one_per_cu ? false : fmt == DSA_KV_FP8_656 || fmt == DSA_KV_MXFP8_V4 || (wgs > 128 && wgs <= 512 / 3);
-    return one_round_splits(wgs, max_list, min_entries, two ? 512 : 256);
+// The same for 32- and 64-head workgroups, of which two fit a CU (units: query
+// tokens).  656-B rows fill both places (a workgroup waits through its
+// conversions): 130 tokens of 16 heads 68 us in 3 splits, 108 unsplit; 74 tokens
+// 42 against 50 in 3.  bf16 rows of up to 32 heads gain less from a second
+// workgroup than its partials cost (64 tokens of 32 heads x 2048 rows 37 us in 4
+// splits, 40 in 8), except where one round of CUs would leave the call unsplit and a
+// third of them idle (150 tokens 68 us in 3 splits, 81 unsplit; 200 tokens 85 in
+// 2, 83 unsplit), from 320 entries a split on (150 tokens x 512 rows 34 us in 3,
+// 27 unsplit).  At 33 to 64 heads, bf16, both places pay
+//   from 64 workgroups of 32 heads on: 43 tokens of 40 heads x 2048 rows 39 us in
+//   5 splits, 50 in 2; 64 tokens 44 in 4, 54 in 2
+//   beyond 170 of them, as 64-head workgroups, for 2048 entries or more: 100, 150
+//   and 200 tokens of 64 heads 65, 88 and 104 us in 5, 3 and 2 splits, 81, 108 and
+//   113 unsplit (250 tokens 121 in 2, 112 unsplit: past 5/6 of the CUs the second
+//   place is not worth the partials); for 1024 entries the partials cost what the
+//   second place gives (150 tokens 59 in 3, 57 unsplit)
+// 656-B rows at 33 to 64 heads as 64-head workgroups in as many splits as both
+// places hold, 64 heads x 2048 entries: 100, 128, 150 and 200 tokens 69, 79, 99 and
+// 121 us, 87, 107, 141 and 142 in splits of 32-head workgroups or unsplit; 1024
+// entries, 150 tokens 66 against 77, 250 tokens 88 against 79; 512 entries never
+// (100 tokens 40 in 2, 36 unsplit).
+int narrow_splits(int fmt, int64_t units, int32_t H, int64_t max_list, int64_t min_entries, bool one_per_cu = false) {
+    constexpr int PLACES = 512, MOST_UNITS = 256 * 5 / 6;
+    const int64_t wgs = units * narrow_groups(H);
+    const int one = one_round_splits(wgs, max_list, min_entries);
+    if (one_per_cu) return one;
+    const bool two_groups = H > 32 && H <= 64;
+    auto at_least = [&](int64_t n) { return std::max<int64_t>(min_entries, n); };
+    if (fmt == DSA_KV_FP8_656 || fmt == DSA_KV_MXFP8_V4) {
+        if (fmt == DSA_KV_FP8_656 && two_groups && wgs > 128) {
+            if (max_list >= 2048 || (max_list >= 1024 && wgs > PLACES / 3 && units <= MOST_UNITS))
+                return one_round_splits(units, max_list, at_least(225), PLACES);
+            if (wgs > PLACES / 3) return 1;
+        }
+        return one_round_splits(wgs, max_list, min_entries, PLACES);
+    }
+    if (wgs <= PLACES / 3 && (wgs > 128 || (two_groups && wgs >= 64)))
+        return std::max(one, one_round_splits(wgs, max_list, at_least(320), PLACES));
+    if (two_groups && wgs > PLACES / 3 && units <= MOST_UNITS && max_list >= 2048)
+        return one_round_splits(units, max_list, at_least(400), PLACES);
+    return one;
 }
 // decode: at least 4 tiles per split (at top-k 2048 and B = 2 or 4: 16 splits
 // measured 11 % faster than 8 and 6 % faster than 32)
@@ -3939,12 +3970,12 @@ int auto_splits(int64_t wgs, int topk) { return one_round_splits(wgs, (int64_t)t
 // automatic one for the kernel narrow_path picks.
 // one_per_cu: no more splits than one workgroup per CU asks for (fewer partials).
 int decode_splits(const dsa_mla_decode_args* a, Kern* kern, bool one_per_cu = false) {
-    const int64_t tokens = (int64_t)a->B * a->s_q, groups = narrow_groups(a->H);
+    const int64_t tokens = (int64_t)a->B * a->s_q;
     const int wide = a->num_splits ? a->num_splits : auto_splits(tokens * head_groups(a->H), a->topk);
     *kern = WIDE;
     if (!narrow_path(a->kv_format, tokens, a->H, wide)) return wide;
     const int ns = a->num_splits ? a->num_splits
-                                 : narrow_splits(a->kv_format, tokens * groups, (int64_t)a->topk + DECODE_MIN - 1, DECODE_MIN,
+                                 : narrow_splits(a->kv_format, tokens, a->H, (int64_t)a->topk + DECODE_MIN - 1, DECODE_MIN,
                                                one_per_cu);
     *kern = narrow_kern(a->kv_format, tokens * ns, a->H);
     return ns;
@@ -4174,7 +4205,7 @@ int prefill_plan(int fmt, int64_t N, int32_t H, int requested, int64_t max_list,
     const int wide = requested > 0 ? requested : one_round_splits(N * head_groups(H), max_list, PREFILL_MIN);
     *kern = WIDE;
     if (!narrow_path(fmt, N, H, wide)) return wide;
-    const int ns = requested > 0 ? requested : narrow_splits(fmt, N * narrow_groups(H), max_list, PREFILL_MIN);
+    const int ns = requested > 0 ? requested : narrow_splits(fmt, N, H, max_list, PREFILL_MIN);
     *kern = narrow_kern(fmt, N * ns, H);
     return ns;
 }
