@@ -3915,14 +3915,17 @@ Kern narrow_kern(int fmt, int64_t units, int32_t H) {
 // the one round shorter for any F > 0.  74 query tokens of 16 heads (656-B rows,
 // 2048 entries): 3 splits 49.9 us against 4 splits (296 workgroups) 73.5 us.
 int one_round_splits(int64_t wgs, int64_t max_list, int64_t min_entries, int round = 256) {
-    if (wgs <= 0 || wgs >= 256) return 1;
+    if (wgs <= 0 || wgs >= round) return 1;
     const int64_t by_len = std::max<int64_t>(1, max_list / min_entries);
     return (int)std::min<int64_t>(std::min<int64_t>(round / wgs, by_len), DSA_MLA_MAX_SPLITS);
 }
 // The same for 32- and 64-head workgroups, of which two fit a CU (units: query
 // tokens).  656-B rows fill both places (a workgroup waits through its
 // conversions): 130 tokens of 16 heads 68 us in 3 splits, 108 unsplit; 74 tokens
-// 42 against 50 in 3.  bf16 rows of up to 32 heads gain less from a second
+// 42 against 50 in 3; two splits (more than 170 workgroups) from 400 entries a
+// split on: 256 tokens x 2048 rows of 16 and 32 heads 86 and 93 us, 106 and 107
+// unsplit, 256 x 1024 52.5 and 60 (58.8 and 60.3), but 190 x 512 36.2 and 39.5 in
+// two (36.2 and 35.2).  bf16 rows of up to 32 heads gain less from a second
 // workgroup than its partials cost (64 tokens of 32 heads x 2048 rows 37 us in 4
 // splits, 40 in 8), except where one round of CUs would leave the call unsplit and a
 // third of them idle (150 tokens 68 us in 3 splits, 81 unsplit; 200 tokens 85 in
@@ -3953,7 +3956,8 @@ int narrow_splits(int fmt, int64_t units, int32_t H, int64_t max_list, int64_t m
                 return one_round_splits(units, max_list, at_least(225), PLACES);
             if (wgs > PLACES / 3) return 1;
         }
-        return one_round_splits(wgs, max_list, min_entries, PLACES);
+        if (fmt == DSA_KV_MXFP8_V4 && wgs >= 256) return 1;
+        return one_round_splits(wgs, max_list, wgs > PLACES / 3 ? at_least(400) : min_entries, PLACES);
     }
     if (wgs <= PLACES / 3 && (wgs > 128 || (two_groups && wgs >= 64)))
         return std::max(one, one_round_splits(wgs, max_list, at_least(320), PLACES));
