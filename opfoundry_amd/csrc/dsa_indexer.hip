@@ -11,10 +11,11 @@
 // a ReLU and a weighted sum over the index heads fused into its epilogue:
 // - a group is up to 128 (token, index head) rows of one sequence, so that the
 //   MTP tokens of a sequence (H_I = 64: two tokens) read each k row once.  The
-//   chunks of 128 positions of all groups are dealt out evenly to at most 512
-//   workgroups (two per CU), each taking one run of them: whatever the lengths
-//   are, the CUs finish together, a workgroup's start (Q, lengths, first rows)
-//   is paid once or twice, and a short call still spreads over the chip.  With
+//   chunks of 128 positions of all groups are dealt out to at most 512 workgroups
+//   (two per CU), each taking one run of them that counts what a group's start
+//   (Q, lengths, first rows) costs (dsa_deal.h): whatever the lengths are, the
+//   CUs finish together, and a short call still spreads over the chip.  Short
+//   lists get whole workgroups per group instead (launch_ix).  With
 //   a workgroup per 2048 positions the starts and the last, partly filled round
 //   took a quarter of the time (2 tokens x 32 sequences of 35 K to 100 K
 //   positions, 570 MB: 158 us, wave-private rings below alone 154 us; 512- and
@@ -42,6 +43,7 @@
 #include <algorithm>
 
 #include "../../include/dsa_indexer.h"
+#include "dsa_deal.h"
 #include "dsa_lds.h"
 
 namespace {
@@ -51,6 +53,8 @@ constexpr int IX_NTHR = 256;
 constexpr int IX_NW = IX_NTHR / 64;
 constexpr int IX_CHUNK = 128;              // positions per chunk (32 per wave)
 constexpr int IX_WGS = 512;                // workgroups of a full grid: two per CU
+constexpr int IX_TINY = 4, IX_SHORT = 16;  // chunks of the longest list that a call may hold
+constexpr int IX_MOST_WGS = 1 << 20;       // workgroups of a grid of one per group (a grid has a limit, the even deal none)
 constexpr int IX_LOOK = 4;                 // steps whose entries and rows a wave holds in LDS
 constexpr int IX_KS = IX_D / 16;           // k-steps of 16
 constexpr int IX_ROW = IX_D * 2;           // bytes of a k row (in LDS too: swizzled, unpadded)
@@ -74,7 +78,7 @@ struct IxParams {
     float* scores;
     int64_t s_stride;
     int32_t s_q, n_cols, causal, tgroups;
-    int32_t parts;               // > 0: workgroups per group (one sequence); 0: an even deal of all chunks
+    int32_t parts;               // > 0: workgroups per group; 0: an even deal of all chunks
 };
 
 // Positions j of token t of sequence b: j < min(len(b, t), n_cols).
@@ -83,25 +87,44 @@ __device__ __forceinline__ int64_t ix_len(const IxParams& p, int64_t L, int t) {
     return min(max(len, (int64_t)0), (int64_t)p.n_cols);
 }
 
-// Inclusive sum over the workgroup of one value per thread; *total gets the sum.
-__device__ __forceinline__ uint32_t ix_scan(uint32_t v, LDS_AS uint32_t* part, uint32_t* total) {
+// Inclusive prefix sum over the 64 lanes of a wave: within rows of 16 lanes by DPP
+// row shifts, then the row totals by the row broadcasts of lanes 15 and 31.
+__device__ __forceinline__ uint32_t ix_wave_scan(uint32_t x) {
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);  // row_shr:1
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);  // row_shr:2
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);  // row_shr:4
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);  // row_shr:8
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return x;
+}
+
+// Inclusive sums over the workgroup, of one value per thread (*sum) and of the
+// values that are not 0 (*some), and their totals.
+__device__ __forceinline__ void ix_scan(uint32_t v, LDS_AS uint32_t* part, uint32_t* sum, uint32_t* some,
+                                        uint32_t* all, uint32_t* all_some) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t u = __shfl_up(v, d, 64);
-        if (lane >= d) v += u;
+    const uint64_t any = __builtin_amdgcn_ballot_w64(v != 0);
+    uint32_t cn = (uint32_t)__builtin_popcountll(any & (~0ull >> (63 - lane)));
+    v = ix_wave_scan(v);
+    if (lane == 63) {
+        part[2 * wave] = v;
+        part[2 * wave + 1] = cn;
     }
-    if (lane == 63) part[wave] = v;
     __syncthreads();
-    uint32_t before = 0, all = 0;
+    uint32_t a = 0, an = 0;
 #pragma unroll
     for (int w = 0; w < IX_NW; ++w) {
-        before += w < wave ? part[w] : 0u;
-        all += part[w];
+        v += w < wave ? part[2 * w] : 0u;
+        cn += w < wave ? part[2 * w + 1] : 0u;
+        a += part[2 * w];
+        an += part[2 * w + 1];
     }
     __syncthreads();
-    *total = all;
-    return v + before;
+    *sum = v;
+    *some = cn;
+    *all = a;
+    *all_some = an;
 }
 
 // max(x, 0), 0 for NaN, as the median of x, 0 and inf (an infinity that the
@@ -151,8 +174,8 @@ dsa_indexer_kernel(const IxParams p) {
     __shared__ __attribute__((aligned(16))) uint64_t s_off[IX_NW * IX_LOOK * 32];   // byte offsets of the k rows
     __shared__ int32_t s_bad[IX_NW * IX_LOOK * 32];                                 // 1: the row is outside the cache
     __shared__ __attribute__((aligned(16))) float s_w[QROWS];
-    __shared__ uint32_t s_part_arr[IX_NW];
-    __shared__ int s_at[2];                   // the workgroup's first group and chunk
+    __shared__ uint32_t s_part_arr[2 * IX_NW];
+    __shared__ uint32_t s_at[4];              // the workgroup's first group and chunk, its last group and the chunk it ends before
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -160,11 +183,11 @@ dsa_indexer_kernel(const IxParams p) {
     const bool any_rows = p.k_rows > 0;
     LDS_AS uint32_t* const s_part = (LDS_AS uint32_t*)s_part_arr;
 
-    // ---- this workgroup's chunks: an equal part of all groups' chunks, in
-    // (sequence, token group, position) order.  Group g's list is its last
-    // token's (the lists grow with t).  A group holds at most 2^24 chunks and a
-    // block of IX_NTHR groups fewer than 2^32; the total is 64 bits, divided in
-    // 32 where it fits (a 64-bit division takes about a microsecond) ----
+    // ---- this workgroup's chunks: a run of all groups' chunks, in (sequence,
+    // token group, position) order, or its part of one group (dsa_deal.h).  Group
+    // g's list is its last token's (the lists grow with t).  A group holds at most
+    // 2^24 chunks and a block of IX_NTHR groups fewer than 2^32; the totals are 64
+    // bits ----
     auto seq_of = [&](int g) -> int { return ONCE ? g : (int)((unsigned)g / (unsigned)p.tgroups); };
     auto group_chunks = [&](int64_t g64) -> uint32_t {
         if (g64 >= p.groups) return 0u;
@@ -172,51 +195,53 @@ dsa_indexer_kernel(const IxParams p) {
         return (uint32_t)((ix_len(p, p.seq_lens[b], min(t0 + TPW, p.s_q) - 1) + IX_CHUNK - 1) / IX_CHUNK);
     };
     const uint32_t G = gridDim.x, x = blockIdx.x;
-    int g, c0;
-    int64_t left;
+    int g, g_last;
+    uint32_t c_first, c_last;                      // first chunk of group g; end of group g_last's
     if (p.parts) {
-        // one sequence: its groups' lists differ by less than s_q positions, so
-        // that workgroups of one group each are as even, start once instead of
-        // up to twice and need no scan
-        g = (int)(x / (uint32_t)p.parts);
-        const uint32_t part = x - (uint32_t)g * (uint32_t)p.parts, n = group_chunks(g);
-        const uint32_t each = n / (uint32_t)p.parts, more = n - each * (uint32_t)p.parts;
-        c0 = (int)(each * part + min(part, more));
-        left = each + (part < more ? 1 : 0);
-        if (left <= 0) return;
+        // whole workgroups per group
+        g = g_last = (int)(x / (uint32_t)p.parts);
+        dsa_deal::part_of(group_chunks(g), (uint32_t)p.parts, x - (uint32_t)g * (uint32_t)p.parts, &c_first, &c_last);
+        if (c_first >= c_last) return;
     } else {
-        uint64_t all = 0;
-        uint32_t n0 = 0, end0 = 0;                 // of groups 0 .. IX_NTHR - 1
+        uint64_t all = 0, some = 0;
+        uint32_t n0 = 0, sum0 = 0, some0 = 0;      // of groups 0 .. IX_NTHR - 1
         for (int64_t g0 = 0; g0 < p.groups; g0 += IX_NTHR) {
             const uint32_t n = group_chunks(g0 + tid);
-            uint32_t tot;
-            const uint32_t end = ix_scan(n, s_part, &tot);
-            if (g0 == 0) { n0 = n; end0 = end; }
+            uint32_t sum, cnt, tot, tot_n;
+            ix_scan(n, s_part, &sum, &cnt, &tot, &tot_n);
+            if (g0 == 0) { n0 = n; sum0 = sum; some0 = cnt; }
             all += tot;
+            some += tot_n;
         }
-        const uint64_t each = all >> 32 ? all / G : (uint64_t)((uint32_t)all / G);
-        const uint32_t more = (uint32_t)(all - each * G);       // the first `more` workgroups take one chunk more
-        const uint64_t first = each * x + min(x, more);
-        left = (int64_t)(each + (x < more ? 1 : 0));
-        if (left <= 0) return;
-        {
-            // the group holding chunk `first`: exactly one thread finds it
-            const bool once = p.groups <= IX_NTHR;
-            uint64_t base = 0;
-            for (int64_t g0 = 0; g0 < p.groups && base <= first; g0 += IX_NTHR) {
-                const uint32_t n = once ? n0 : group_chunks(g0 + tid);
-                uint32_t tot = 0;
-                const uint64_t end = base + (once ? end0 : ix_scan(n, s_part, &tot));
-                if (end > first && end - n <= first) {
-                    s_at[0] = (int)(g0 + tid);
-                    s_at[1] = (int)(first - (end - n));
-                }
-                base += tot;
+        const dsa_deal::Deal deal = dsa_deal::deal_of(all, some, G, ONCE ? dsa_deal::START_ONCE : dsa_deal::START);
+        uint64_t first, last;
+        dsa_deal::run_of(deal, x, &first, &last);
+        if (first >= last) return;
+        // the groups holding units `first` and `last - 1`: exactly one thread finds each
+        const bool once = p.groups <= IX_NTHR;
+        uint64_t base = 0;
+        for (int64_t g0 = 0; g0 < p.groups && base < last; g0 += IX_NTHR) {
+            uint32_t n = n0, sum = sum0, cnt = some0, tot = 0, tot_n = 0;
+            if (!once) {
+                n = group_chunks(g0 + tid);
+                ix_scan(n, s_part, &sum, &cnt, &tot, &tot_n);
             }
-            __syncthreads();
+            const uint64_t end = base + sum + (uint64_t)deal.start * cnt, begin = end - dsa_deal::units(deal, n);
+            if (begin <= first && first < end) {
+                s_at[0] = (uint32_t)(g0 + tid);
+                s_at[1] = dsa_deal::chunks_before(deal, first - begin);
+            }
+            if (begin < last && last <= end) {
+                s_at[2] = (uint32_t)(g0 + tid);
+                s_at[3] = dsa_deal::chunks_before(deal, last - begin);
+            }
+            base += tot + (uint64_t)deal.start * tot_n;
         }
-        g = __builtin_amdgcn_readfirstlane(s_at[0]);
-        c0 = __builtin_amdgcn_readfirstlane(s_at[1]);
+        __syncthreads();
+        g = __builtin_amdgcn_readfirstlane((int)s_at[0]);
+        c_first = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_at[1]);
+        g_last = __builtin_amdgcn_readfirstlane((int)s_at[2]);
+        c_last = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_at[3]);
     }
 
     const lds_ptr ring = (lds_ptr)s_k + wave * 2 * IX_SLOT;
@@ -226,15 +251,15 @@ dsa_indexer_kernel(const IxParams p) {
 
     float inf = INFINITY;
     asm volatile("" : "+s"(inf));
-    for (; left > 0; ++g, c0 = 0) {
+    for (; g <= g_last; ++g, c_first = 0) {
         const int b = seq_of(g);
         const int t0 = (g - b * p.tgroups) * TPW;
         const int ntok = min(TPW, p.s_q - t0);
         const int64_t L = p.seq_lens[b];
         const int32_t lmax = (int32_t)ix_len(p, L, t0 + ntok - 1);
-        const int m = (int)min(left, (lmax + (IX_CHUNK - 1ll)) / IX_CHUNK - c0);   // chunks of this group
-        if (m <= 0) continue;                  // (an empty list)
-        left -= m;
+        const uint32_t c_end = g == g_last ? c_last : (uint32_t)((lmax + (IX_CHUNK - 1ll)) / IX_CHUNK);
+        if (c_first >= c_end) continue;        // (an empty list, or the run ends in its start units)
+        const int c0 = (int)c_first, m = (int)(c_end - c_first);
 
         // ---- Q (A operand): lane (r32, hi) holds rows 32qb + r32, dims 16ks + 8hi .. +7 ----
         u32x4 qf[NB][IX_KS];
@@ -391,13 +416,30 @@ int launch_ix(IxParams& p, int B, hipStream_t st) {
     const int64_t most = (p.n_cols + (int64_t)IX_CHUNK - 1) / IX_CHUNK;
     const bool once = p.tgroups == 1;          // (always for NB < 4: chosen by s_q)
     int64_t wgs = p.groups >= IX_WGS || most >= IX_WGS ? IX_WGS : std::min<int64_t>(p.groups * most, IX_WGS);
-    // One sequence, and whole workgroups per group that fill at least 7/8 of the
-    // grid an even deal would have: 512 tokens of 32 heads x 8000 positions 48.5 us
-    // (about 53 by an even deal, whose workgroups mostly span two groups); at worst 7/8 of
-    // the places are used, where a second start costs about as much.
-    if (B == 1 && wgs / p.groups * p.groups >= wgs - wgs / 8) {
-        p.parts = (int32_t)(wgs / p.groups);
+    // Whole workgroups per group, which start once and need no scan of the lengths
+    // (about a microsecond):
+    // - lists of up to IX_TINY chunks, in as many workgroups per group as one per CU
+    //   gives: a second one there splits too few chunks to be worth its start (200
+    //   sequences x 3 tokens x 300 positions of 64 heads 17.2 us, 20.9 dealt out; 128
+    //   x 2 10.2 and 13.8);
+    // - one sequence, or lists of up to IX_SHORT chunks, where they fill at least 7/8
+    //   of the even deal's places: 1024 positions, 256 sequences x 2 tokens of 64
+    //   heads 21.8 us, 26.3 dealt out.  One sequence's groups are as even as its
+    //   lists are; several sequences' lists may differ by up to IX_SHORT chunks;
+    // - lists of up to IX_SHORT chunks in two or more rounds of workgroups, one per
+    //   group: the hardware hands them out as others end (causal, 2048 tokens x 2048
+    //   positions of 128 heads 102 us, 119 dealt out; with 600 groups the second
+    //   round is mostly empty, 51 and 46).
+    const int64_t parts = wgs / p.groups;
+    if (most <= IX_TINY && p.groups <= IX_MOST_WGS) {
+        p.parts = (int32_t)std::max<int64_t>(1, std::min<int64_t>(IX_WGS / 2 / p.groups, most));
         wgs = p.parts * p.groups;
+    } else if ((B == 1 || most <= IX_SHORT) && parts * p.groups >= wgs - wgs / 8) {
+        p.parts = (int32_t)parts;
+        wgs = parts * p.groups;
+    } else if (most <= IX_SHORT && p.groups >= 2 * IX_WGS && p.groups <= IX_MOST_WGS) {
+        p.parts = 1;
+        wgs = p.groups;
     }
     if (once) hipLaunchKernelGGL((dsa_indexer_kernel<HI, NB, true>), dim3((unsigned)wgs), dim3(IX_NTHR), 0, st, p);
     else if constexpr (NB == 4)

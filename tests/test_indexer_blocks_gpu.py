@@ -58,3 +58,22 @@ def test_nan_row_scores_zero(dev):
     torch.cuda.synchronize()
     assert (got[0, :, 71].cpu().numpy() == 0.0).all()
     check(got, q, w, k, ref, "indexer NaN row")
+
+
+@pytest.mark.parametrize("H_I,s_q,lens", [(64, 2, [500, 3, 128, 129] * 10), (64, 2, [2000, 700, 1, 1025] * 16),
+                                          (128, 40, [700, 90, 513] * 10), (32, 2, [1] * 260 + [3001] * 11),
+                                          (128, 3, [30] * 60 + [9000] * 3), (64, 5, [129] * 100 + [2500] * 12)])
+def test_deals(dev, H_I, s_q, lens):
+    """Whole workgroups per group (up to 4 chunks, up to 16, and 1200 groups in several rounds), and
+    even deals whose runs count the groups' starts (chunks read once, and by several groups; more
+    than 256 groups, in one block of the scan and two)."""
+    rng = np.random.default_rng(460 + len(lens) + s_q)
+    seq = np.array(lens, np.int32)
+    q, w, k, bt = paged(rng, len(seq), seq, 64, H_I, s_q, bad_blocks=3)
+    n = int(seq.max())
+    print(f"[case] indexer deal H_I={H_I} s_q={s_q} B={len(seq)} n={n}", flush=True)
+    ref = oracle.indexer_scores(q, w, k, seq, block_table=bt, block_size=64, causal=True, n_cols=n)
+    got = dsa.indexer_scores(t16(q, dev), torch.from_numpy(w).to(dev), t16(k, dev), torch.from_numpy(seq).to(dev),
+                             block_table=torch.from_numpy(bt).to(dev), block_size=64, causal=True, n_cols=n)
+    torch.cuda.synchronize()
+    check(got, q, w, k, ref, f"indexer deal H_I={H_I} s_q={s_q}")
