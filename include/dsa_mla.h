@@ -185,9 +185,17 @@ int dsa_mla_decode(const dsa_mla_decode_args* args, void* workspace, size_t work
  * GPU for the life of the process (DSA_MLA_NOALLOC_SCRATCH_BYTES; its address
  * is looked up on a device's first call).  A call whose partials need more
  * (dsa_mla_decode_workspace_size) returns DSA_ERR_SCRATCH_LIMIT before any
- * launch; unsplit calls need none.  Calls that overlap on one GPU share its
- * scratch and race: serialise them (one stream, or events).  Results equal
- * dsa_mla_decode's on the same arguments.
+ * launch, with one exception; unsplit calls need none.  The exception: with
+ * num_splits = 0 in workgroups of 32 or 64 heads, where the automatic count may
+ * run two to a CU, a call whose partials need too much runs instead with the
+ * fewest splits that give each of 256 CUs a workgroup,
+ *   max(1, min(ceil(256 / (B s_q g)), ceil(topk / 128), DSA_MLA_MAX_SPLITS)),
+ *   g = 1 up to 64 heads, ceil(H / 32) beyond,
+ * if those partials fit.  Calls that overlap on one GPU share its scratch and
+ * race: serialise them (one stream, or events).  Results equal
+ * dsa_mla_decode's on the same arguments, in the exception with that
+ * num_splits (dsa_mla_decode_num_splits reports the automatic count; another
+ * split count sums in another order and may change the last bits).
  */
 #define DSA_MLA_NOALLOC_SCRATCH_BYTES (16u << 20)
 int dsa_mla_decode_noalloc(const dsa_mla_decode_args* args, void* stream);

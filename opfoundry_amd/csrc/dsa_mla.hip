@@ -3819,7 +3819,8 @@ dsa_kv_quantize_kernel(const __bf16* __restrict__ src, int64_t src_stride, int64
 
 // ------------------------------------------------------------------- host
 
-int decode_launch(const dsa_mla_decode_args* a, int ns, int chunk, void* ws, hipStream_t st);
+struct DecodePlan;
+int decode_launch(const dsa_mla_decode_args* a, const DecodePlan& plan, void* ws, hipStream_t st);
 
 // Device scratch of dsa_mla_decode_noalloc: the split partials (fp32 O and
 // LSE) of a call live here instead of in a caller workspace.  Every GPU the
@@ -3943,11 +3944,10 @@ int one_round_splits(int64_t wgs, int64_t max_list, int64_t min_entries, int rou
 // 121 us, 87, 107, 141 and 142 in splits of 32-head workgroups or unsplit; 1024
 // entries, 150 tokens 66 against 77, 250 tokens 88 against 79; 512 entries never
 // (100 tokens 40 in 2, 36 unsplit).
-int narrow_splits(int fmt, int64_t units, int32_t H, int64_t max_list, int64_t min_entries, bool one_per_cu = false) {
+int narrow_splits(int fmt, int64_t units, int32_t H, int64_t max_list, int64_t min_entries) {
     constexpr int PLACES = 512, MOST_UNITS = 256 * 5 / 6;
     const int64_t wgs = units * narrow_groups(H);
     const int one = one_round_splits(wgs, max_list, min_entries);
-    if (one_per_cu) return one;
     const bool two_groups = H > 32 && H <= 64;
     auto at_least = [&](int64_t n) { return std::max<int64_t>(min_entries, n); };
     if (fmt == DSA_KV_FP8_656 || fmt == DSA_KV_MXFP8_V4) {
@@ -3970,22 +3970,34 @@ int narrow_splits(int fmt, int64_t units, int32_t H, int64_t max_list, int64_t m
 constexpr int DECODE_MIN = 128;
 int auto_splits(int64_t wgs, int topk) { return one_round_splits(wgs, (int64_t)topk + DECODE_MIN - 1, DECODE_MIN); }
 
-// Split count and kernel of a top-k decode call: the caller's count, or the
-// automatic one for the kernel narrow_path picks.
-// one_per_cu: no more splits than one workgroup per CU asks for (fewer partials).
-int decode_splits(const dsa_mla_decode_args* a, Kern* kern, bool one_per_cu = false) {
+// A top-k decode call: its split count (the caller's, or the automatic one for the
+// kernel narrow_path picks), the entries of a split, and the kernel.
+struct DecodePlan {
+    int ns, chunk;
+    Kern kern;
+};
+DecodePlan decode_plan(const dsa_mla_decode_args* a) {
     const int64_t tokens = (int64_t)a->B * a->s_q;
-    const int wide = a->num_splits ? a->num_splits : auto_splits(tokens * head_groups(a->H), a->topk);
-    *kern = WIDE;
-    if (!narrow_path(a->kv_format, tokens, a->H, wide)) return wide;
-    const int ns = a->num_splits ? a->num_splits
-                                 : narrow_splits(a->kv_format, tokens, a->H, (int64_t)a->topk + DECODE_MIN - 1, DECODE_MIN,
-                                               one_per_cu);
-    *kern = narrow_kern(a->kv_format, tokens * ns, a->H);
-    return ns;
+    DecodePlan p{a->num_splits ? a->num_splits : auto_splits(tokens * head_groups(a->H), a->topk), 0, WIDE};
+    if (narrow_path(a->kv_format, tokens, a->H, p.ns)) {
+        if (!a->num_splits)
+            p.ns = narrow_splits(a->kv_format, tokens, a->H, (int64_t)a->topk + DECODE_MIN - 1, DECODE_MIN);
+        p.kern = narrow_kern(a->kv_format, tokens * p.ns, a->H);
+    }
+    p.chunk = a->topk == 0 ? 0 : (a->topk + p.ns - 1) / p.ns;
+    return p;
+}
+// The split count of a no-allocation call whose automatic partials do not fit the
+// scratch (two 32- or 64-head workgroups to a CU): the fewest splits, of at least
+// DECODE_MIN entries, that give every CU a workgroup, with all of a token's heads
+// in one up to 64 heads, 32 in each beyond.
+int noalloc_splits(const dsa_mla_decode_args* a) {
+    const int64_t wgs = (int64_t)a->B * a->s_q * (a->H <= 64 ? 1 : narrow_groups(a->H));
+    const int64_t by_len = std::max<int64_t>(1, ((int64_t)a->topk + DECODE_MIN - 1) / DECODE_MIN);
+    return (int)std::min<int64_t>(std::min<int64_t>((256 + wgs - 1) / wgs, by_len), DSA_MLA_MAX_SPLITS);
 }
 
-int validate_decode(const dsa_mla_decode_args* a, int* ns_out, int* chunk_out, bool one_per_cu = false) {
+int validate_decode(const dsa_mla_decode_args* a, DecodePlan* plan) {
     if (!a) return DSA_ERR_NULL_POINTER;
     if (a->B < 0 || a->s_q <= 0 || a->topk < 0 || a->topk > MAX_LIST) return DSA_ERR_BAD_SHAPE;
     if (!heads_ok(a->H, a->B)) return DSA_ERR_BAD_SHAPE;
@@ -3994,9 +4006,6 @@ int validate_decode(const dsa_mla_decode_args* a, int* ns_out, int* chunk_out, b
     if (a->block_table && a->block_size <= 0) return DSA_ERR_BAD_SHAPE;
     if (row_stride_bytes(a->kv_format, a->kv_stride_row) < 0) return DSA_ERR_BAD_STRIDE;
     if (a->num_splits < 0 || a->num_splits > DSA_MLA_MAX_SPLITS) return DSA_ERR_BAD_SPLITS;
-    Kern kern;
-    const int ns = decode_splits(a, &kern, one_per_cu);
-    const int chunk = a->topk == 0 ? 0 : (a->topk + ns - 1) / ns;
     if (a->B > 0 && a->topk > 0) {
         if (!a->q || !a->kv_cache || !a->seq_lens || !a->indices || !a->out) return DSA_ERR_NULL_POINTER;
         if ((a->q_stride_h % 8) != 0 || (a->q_stride_t % 8) != 0 || (a->q_stride_b % 8) != 0)
@@ -4008,8 +4017,7 @@ int validate_decode(const dsa_mla_decode_args* a, int* ns_out, int* chunk_out, b
     }
     // the kernel reads Q even when no entry is valid: q is needed whenever B > 0
     if (a->B > 0 && a->topk == 0 && (!a->out || !a->q)) return DSA_ERR_NULL_POINTER;
-    *ns_out = ns;
-    *chunk_out = chunk;
+    *plan = decode_plan(a);
     return DSA_OK;
 }
 
@@ -4336,63 +4344,62 @@ const char* dsa_mla_strerror(int code) {
 
 int dsa_mla_decode_num_splits(const dsa_mla_decode_args* a, int32_t* num_splits) {
     if (!num_splits) return DSA_ERR_NULL_POINTER;
-    int ns, chunk;
-    const int rc = validate_decode(a, &ns, &chunk);
+    DecodePlan plan;
+    const int rc = validate_decode(a, &plan);
     if (rc) return rc;
-    *num_splits = ns;
+    *num_splits = plan.ns;
     return DSA_OK;
 }
 
 int dsa_mla_decode_workspace_size(const dsa_mla_decode_args* a, size_t* bytes) {
     if (!bytes) return DSA_ERR_NULL_POINTER;
-    int ns, chunk;
-    const int rc = validate_decode(a, &ns, &chunk);
+    DecodePlan plan;
+    const int rc = validate_decode(a, &plan);
     if (rc) return rc;
-    *bytes = decode_ws_bytes(a, ns);
+    *bytes = decode_ws_bytes(a, plan.ns);
     return DSA_OK;
 }
 
 int dsa_mla_decode(const dsa_mla_decode_args* a, void* ws, size_t ws_bytes, void* stream) {
-    int ns, chunk;
-    const int rc = validate_decode(a, &ns, &chunk);
+    DecodePlan plan;
+    const int rc = validate_decode(a, &plan);
     if (rc) return rc;
-    const size_t need = decode_ws_bytes(a, ns);
+    const size_t need = decode_ws_bytes(a, plan.ns);
     if (need && (!ws || ws_bytes < need || ((uintptr_t)ws & 15))) return DSA_ERR_WORKSPACE;
     if (a->B == 0) return DSA_OK;
-    return decode_launch(a, ns, chunk, ws, (hipStream_t)stream);
+    return decode_launch(a, plan, ws, (hipStream_t)stream);
 }
 
 int dsa_mla_decode_noalloc(const dsa_mla_decode_args* a, void* stream) {
-    int ns, chunk;
-    const int rc = validate_decode(a, &ns, &chunk);
+    DecodePlan plan;
+    const int rc = validate_decode(a, &plan);
     if (rc) return rc;
-    size_t need = decode_ws_bytes(a, ns);
-    if (need > DSA_MLA_NOALLOC_SCRATCH_BYTES) {
-        // fewer splits, where the automatic count can do with fewer
-        validate_decode(a, &ns, &chunk, true);
-        need = decode_ws_bytes(a, ns);
+    if (a->B == 0) return DSA_OK;
+    size_t need = decode_ws_bytes(a, plan.ns);
+    if (need > DSA_MLA_NOALLOC_SCRATCH_BYTES && !a->num_splits && plan.kern != WIDE) {
+        dsa_mla_decode_args fewer = *a;
+        fewer.num_splits = noalloc_splits(a);
+        plan = decode_plan(&fewer);
+        need = decode_ws_bytes(a, plan.ns);
     }
     if (need > DSA_MLA_NOALLOC_SCRATCH_BYTES) return DSA_ERR_SCRATCH_LIMIT;
-    if (a->B == 0) return DSA_OK;
     void* ws = nullptr;
     if (need) {
         const int rs = device_scratch(&ws);
         if (rs) return rs;
     }
-    return decode_launch(a, ns, chunk, ws, (hipStream_t)stream);
+    return decode_launch(a, plan, ws, (hipStream_t)stream);
 }
 
 }  // extern "C"
 
 namespace {
 
-int decode_launch(const dsa_mla_decode_args* a, int ns, int chunk, void* ws, hipStream_t st) {
-    // the kernel of this split count (the automatic one, or fewer)
-    Kern kern;
-    if (decode_splits(a, &kern) != ns) decode_splits(a, &kern, true);
+int decode_launch(const dsa_mla_decode_args* a, const DecodePlan& plan, void* ws, hipStream_t st) {
+    const int ns = plan.ns;
     FwdParams fp{};
     fp.H = a->H;
-    fp.hgroups = groups_of(kern, a->H);
+    fp.hgroups = groups_of(plan.kern, a->H);
     fp.q = (const __bf16*)a->q;
     fp.q_sb = a->q_stride_b; fp.q_st = a->q_stride_t; fp.q_sh = a->q_stride_h;
     fp.kv = (const unsigned char*)a->kv_cache;
@@ -4410,7 +4417,7 @@ int decode_launch(const dsa_mla_decode_args* a, int ns, int chunk, void* ws, hip
     fp.out = (__bf16*)a->out;
     fp.o_sb = a->o_stride_b; fp.o_st = a->o_stride_t; fp.o_sh = a->o_stride_h;
     fp.lse = a->lse;
-    fp.B = a->B; fp.s_q = a->s_q; fp.topk = a->topk; fp.chunk = chunk;
+    fp.B = a->B; fp.s_q = a->s_q; fp.topk = a->topk; fp.chunk = plan.chunk;
     fp.causal = a->causal ? 1 : 0;
     fp.causal_offset = 0;
     fp.scale_log2 = a->sm_scale * LOG2E;
@@ -4419,7 +4426,7 @@ int decode_launch(const dsa_mla_decode_args* a, int ns, int chunk, void* ws, hip
         fp.part_o = (float*)ws;
         fp.part_lse = (float*)((char*)ws + (size_t)ns * rows * D_VO * sizeof(float));
     }
-    int r = launch_fwd(fp, a->kv_format, a->B, a->s_q, ns, st, kern);
+    int r = launch_fwd(fp, a->kv_format, a->B, a->s_q, ns, st, plan.kern);
     if (r || ns == 1) return r;
     return launch_combine(fp.part_o, fp.part_lse, ns, a->B * a->s_q, a->H, a->s_q, a->out, a->o_stride_b,
                           a->o_stride_t, a->o_stride_h, a->lse, st);

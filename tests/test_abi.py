@@ -174,6 +174,9 @@ def test_decode_rejects_missing_workspace(lib):
     (dict(topk=2 ** 31 - 1), -2),
     # 64 splits of 2 x 128 rows: 33.6 MB of partials, beyond the 16 MiB scratch
     (dict(B=2, num_splits=64), -9),
+    # automatic counts: 100 tokens of 32 heads (5 splits, 33 MB; at one workgroup per CU 3, 20 MB),
+    # and 128-head workgroups (8 tokens of 72 heads, 16 splits, 19 MB)
+    (dict(B=100, H=32, topk=2048, kv_format=abi.KV_FP8_656), -9), (dict(B=8, H=72, topk=2048), -9),
 ])
 def test_decode_noalloc_rejects_before_launch(lib, kw, code):
     a = _decode_args(**kw)

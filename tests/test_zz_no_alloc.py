@@ -66,6 +66,40 @@ def test_noalloc_matches_workspace_entry(dev, fp8):
         assert not np.isnan(l_na).all()
 
 
+@pytest.mark.parametrize("fp8,B,H,splits", [(True, 128, 16, 2), (True, 64, 16, 4), (True, 256, 32, 1),
+                                            (False, 300, 40, 1), (True, 7, 80, 13)])
+def test_noalloc_at_one_workgroup_per_cu(dev, fp8, B, H, splits):
+    """An automatic split count for two workgroups per CU whose partials exceed the scratch: the
+    call runs with the documented count, and gives dsa_mla_decode's bits at that count.  (Where
+    the automatic partials fit, the automatic count's.)"""
+    c = paged_case(seed=80 + B + H, B=B, s_q=1, H=H, seq_len=2112, topk=2048, fp8=fp8, varlen=True)
+    lib = abi.load_library()
+    q, kv = t16(c.q, dev), kv_tensor(c.kv, dev)
+    idx, sl, bt = (torch.from_numpy(x).to(dev) for x in (c.indices, c.seq_lens, c.block_table))
+
+    def run(num_splits, noalloc):
+        out = torch.full((B, 1, H, 512), float("nan"), dtype=torch.bfloat16, device=dev)
+        lse = torch.full((B, 1, H), float("nan"), dtype=torch.float32, device=dev)
+        a = dsa.make_decode_args(q, kv, idx, c.sm_scale, out, lse, seq_lens=sl, block_table=bt,
+                                 block_size=c.block_size, causal=c.causal, num_splits=num_splits)
+        size = dsa.decode_workspace_size(a)
+        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        if noalloc:
+            rc = lib.dsa_mla_decode_noalloc(ctypes.byref(a), stream)
+        else:
+            ws = torch.empty(max(size, 1), dtype=torch.uint8, device=dev)
+            rc = lib.dsa_mla_decode(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()), size, stream)
+        assert rc == 0, abi.ERRORS.get(rc, rc)
+        torch.cuda.synchronize()
+        return size, out.cpu().view(torch.int16).numpy(), lse.cpu().numpy()
+
+    print(f"[case] noalloc one per CU fp8={fp8} B={B} H={H}", flush=True)
+    size, o, l = run(0, True)
+    _, o_ref, l_ref = run(splits if size > abi.NOALLOC_SCRATCH_BYTES else 0, False)
+    assert np.array_equal(o, o_ref) and np.array_equal(l, l_ref, equal_nan=True)
+    assert not np.isnan(l).all()
+
+
 def test_noalloc_scratch_limit(dev):
     """A call whose partials exceed the scratch is refused before any launch; the outputs
     are left untouched."""
