@@ -45,17 +45,15 @@ FLOP_PER_PAIR = 2 * H * (D_QK + D_VO)
 
 
 def _fwd_kernel(name, tokens, splits, heads):
-    """The library's rule: workgroups of 32 heads (of 64 for 33 to 64 heads of more tokens x
-    splits than CUs) when heads <= 64 or when the 128-head kernel would run fewer than 128
-    workgroups, two to a CU (pair) when they outnumber the CUs, else one (narrow); else
-    128-head workgroups.  (splits: the split count the call runs with.)"""
-    groups = (heads + 31) // 32
-    if heads <= 64 or tokens * ((heads + 127) // 128) * splits < 128:
-        if 32 < heads <= 64 and tokens * splits > 256:
-            return f"dsa_mla_fwd_pair_kernel<{name}, 64>"
-        return (f"dsa_mla_fwd_pair_kernel<{name}, 32>" if tokens * groups * splits > 256
-                else f"dsa_mla_fwd_narrow_kernel<{name}>")
-    return f"dsa_mla_fwd_kernel<{name}>"
+    """The kernel the library runs: beyond 64 heads 128-head workgroups, or 32-head ones when those
+    would be fewer than 128 (one to a CU, or two when they outnumber the CUs); up to 64 heads its
+    choice of the least expected time.  (splits: the split count the call runs with.)"""
+    if heads <= 64:
+        return f"dsa_mla_fwd_narrow_kernel<{name}> or dsa_mla_fwd_pair_kernel<{name}, .>"
+    if tokens * ((heads + 127) // 128) * splits >= 128:
+        return f"dsa_mla_fwd_kernel<{name}>"
+    return (f"dsa_mla_fwd_pair_kernel<{name}, 32>" if tokens * ((heads + 31) // 32) * splits > 256
+            else f"dsa_mla_fwd_narrow_kernel<{name}>")
 
 
 def bf16_fwd_kernel(tokens, splits, heads=H, d512=False):

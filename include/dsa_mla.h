@@ -37,13 +37,17 @@
  *
  * Heads.  Every entry takes any head count H >= 1 (H <= 0 is
  * DSA_ERR_BAD_SHAPE).  A query token runs in ceil(H / 128) workgroups of 128
- * heads, or in workgroups of 32 or 64 heads at H <= 64 and, of 32, for bf16 and
- * 656-B fp8 rows when 128-head workgroups would be too few to occupy the GPU
- * (the summation order of the scores then differs, within the same bounds); the
- * last group computes its heads past H on a copy of head H-1 and stores nothing
- * for them, so outputs, LSEs and partials are written for heads
- * 0..H-1 only.  The kernel choice changes dsa_mla_decode_num_splits and the
- * workspace sizes, which report the split count of the kernel that runs.
+ * heads, or in workgroups of 32 or 64 heads: at H <= 64 where those are
+ * expected to take less time, and, of 32, for bf16 and 656-B fp8 rows when
+ * 128-head workgroups would be too few to occupy the GPU.  The last group
+ * computes its heads past H on a copy of head H-1 and stores nothing for them,
+ * so outputs, LSEs and partials are written for heads 0..H-1 only.  The kernel
+ * choice changes dsa_mla_decode_num_splits and the workspace sizes, which
+ * report the split count of the kernel that runs.  Both choices depend on the
+ * call's sizes alone.  Another kernel or split count sums in another order and
+ * rounds probabilities against another reference, so the last bits of O and LSE
+ * may differ between calls of different sizes or num_splits, within the same
+ * bounds; one call repeats its bits.
  *
  * Numerics.  Scores s = (q . k) * sm_scale in fp32; softmax probabilities are
  * rounded to the P.V product's 16-bit type before it (bf16 for bf16 and MXFP8

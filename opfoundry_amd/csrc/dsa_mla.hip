@@ -31,6 +31,7 @@
 #include <stdint.h>
 #include <float.h>
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 
@@ -3871,25 +3872,14 @@ bool heads_ok(int32_t H, int64_t tokens) {
     return H >= 1 && tokens * head_groups(H) <= INT32_MAX;
 }
 
-// Forward kernel of a call of `tokens` query tokens (work items) and H heads.
+// Forward kernels of a call:
 //   WIDE    128 heads per workgroup, one per CU (dsa_mla_fwd_kernel)
 //   NARROW  32 heads, one workgroup per CU (dsa_mla_fwd_narrow_kernel)
 //   PAIR    32 heads, two workgroups per CU (dsa_mla_fwd_pair_kernel<., 32>)
 //   PAIR64  64 heads, two workgroups per CU (dsa_mla_fwd_pair_kernel<., 64>)
-// The three small ones where the 128-head kernel would compute at least 2x padding
-// heads (H <= 64), or could not occupy half the GPU even with its splits (fewer
-// than 128 workgroups at wide_splits splits).  Splits are counted for 32-head
-// workgroups (narrow_splits); given them, `units` query tokens (or plan items)
-// x splits run
-//   PAIR64  at 33..64 heads when the units alone outnumber the CUs: below that
-//           each would have a CU to itself, and twice as many workgroups of 32
-//           heads are faster (MXFP8, 256 units, 92.3 against 93.3 us, 100 tokens
-//           with their plan 41.8 against 43.3; above, 300 units at H = 64 136 us
-//           against 226 on WIDE)
-//   PAIR    when 32-head workgroups outnumber the CUs, so that a second one on a
-//           CU has something to fill (4096 queries x 2048 rows, H = 16, bf16:
-//           747 us, NARROW 1226), and for the formats without a narrow kernel
-//   NARROW  otherwise
+// The three small ones are considered where the 128-head kernel would compute at
+// least 2x padding heads (H <= 64), or could not occupy half the GPU even with its
+// splits (fewer than 128 workgroups at wide_splits splits).
 enum Kern { WIDE, NARROW, PAIR, PAIR64 };
 int narrow_groups(int32_t H) { return (H + NARROW_HEADS - 1) / NARROW_HEADS; }
 int groups_of(Kern k, int32_t H) {
@@ -3901,91 +3891,124 @@ bool narrow_path(int fmt, int64_t tokens, int32_t H, int wide_splits) {
     if (H <= 64) return true;
     return has_narrow(fmt) && tokens * head_groups(H) * wide_splits < 128;
 }
+// Work plans and MXFP8 lists, whose lengths the host does not know: PAIR64 at 33..64
+// heads when the units (rows, or tokens x splits) alone outnumber the CUs: below that
+// each would have a CU to itself, and twice as many workgroups of 32 heads are faster
+// (MXFP8, 256 units, 92.3 against 93.3 us, 100 tokens with their plan 41.8 against
+// 43.3; above, 300 units at H = 64 136 us against 226 on WIDE).
 Kern pair_kern(int64_t units, int32_t H) {
     return H > 32 && H <= 64 && units > 256 ? PAIR64 : PAIR;
 }
-Kern narrow_kern(int fmt, int64_t units, int32_t H) {
-    return !has_narrow(fmt) || units * narrow_groups(H) > 256 ? pair_kern(units, H) : NARROW;
+
+// Splits of a call whose `wgs` unsplit workgroups would leave places idle: as many
+// as fit one round of `round` places, of at least 1 / by_len of the list each.  A
+// second, mostly empty round costs another workgroup's fixed time (its Q load, first
+// gathers and output) and its share of the list: 2 (F + L / ceil) against F + L /
+// floor, and ceil <= floor + 1 makes the one round shorter for any F > 0.  74 query
+// tokens of 16 heads (656-B rows, 2048 entries, one workgroup per CU): 3 splits 49.9
+// us against 4 splits (296 workgroups) 73.5 us.
+constexpr int CUS = 256;
+int one_round_splits(int64_t wgs, int64_t by_len, int round = CUS) {
+    if (wgs <= 0 || wgs >= round) return 1;
+    return (int)std::min<int64_t>(std::min<int64_t>(round / wgs, std::max<int64_t>(by_len, 1)), DSA_MLA_MAX_SPLITS);
 }
 
-// Splits of a call whose `wgs` unsplit workgroups would leave CUs idle: as many
-// as fit one round of the 256 CUs (a workgroup takes a whole CU), with at least
-// min_entries list entries each.  A second, mostly empty round costs another
-// workgroup's fixed time (its Q load, first gathers and output) and its share of
-// the list: 2 (F + L / ceil) against F + L / floor, and ceil <= floor + 1 makes
-// the one round shorter for any F > 0.  74 query tokens of 16 heads (656-B rows,
-// 2048 entries): 3 splits 49.9 us against 4 splits (296 workgroups) 73.5 us.
-int one_round_splits(int64_t wgs, int64_t max_list, int64_t min_entries, int round = 256) {
-    if (wgs <= 0 || wgs >= round) return 1;
-    const int64_t by_len = std::max<int64_t>(1, max_list / min_entries);
-    return (int)std::min<int64_t>(std::min<int64_t>(round / wgs, by_len), DSA_MLA_MAX_SPLITS);
-}
-// The same for 32- and 64-head workgroups, of which two fit a CU (units: query
-// tokens).  656-B rows fill both places (a workgroup waits through its
-// conversions): 130 tokens of 16 heads 68 us in 3 splits, 108 unsplit; 74 tokens
-// 42 against 50 in 3; two splits (more than 170 workgroups) from 400 entries a
-// split on: 256 tokens x 2048 rows of 16 and 32 heads 86 and 93 us, 106 and 107
-// unsplit, 256 x 1024 52.5 and 60 (58.8 and 60.3), but 190 x 512 36.2 and 39.5 in
-// two (36.2 and 35.2).  bf16 rows of up to 32 heads gain less from a second
-// workgroup than its partials cost (64 tokens of 32 heads x 2048 rows 37 us in 4
-// splits, 40 in 8), except where one round of CUs would leave the call unsplit and a
-// third of them idle (150 tokens 68 us in 3 splits, 81 unsplit; 200 tokens 85 in
-// 2, 83 unsplit), from 320 entries a split on (150 tokens x 512 rows 34 us in 3,
-// 27 unsplit).  At 33 to 64 heads, bf16, both places pay
-//   from 64 workgroups of 32 heads on: 43 tokens of 40 heads x 2048 rows 39 us in
-//   5 splits, 50 in 2; 64 tokens 44 in 4, 54 in 2
-//   beyond 170 of them, as 64-head workgroups, for 2048 entries or more: 100, 150
-//   and 200 tokens of 64 heads 65, 88 and 104 us in 5, 3 and 2 splits, 81, 108 and
-//   113 unsplit (250 tokens 121 in 2, 112 unsplit: past 5/6 of the CUs the second
-//   place is not worth the partials); for 1024 entries the partials cost what the
-//   second place gives (150 tokens 59 in 3, 57 unsplit)
-// 656-B rows at 33 to 64 heads as 64-head workgroups in as many splits as both
-// places hold, 64 heads x 2048 entries: 100, 128, 150 and 200 tokens 69, 79, 99 and
-// 121 us, 87, 107, 141 and 142 in splits of 32-head workgroups or unsplit; 1024
-// entries, 150 tokens 66 against 77, 250 tokens 88 against 79; 512 entries never
-// (100 tokens 40 in 2, 36 unsplit).
-int narrow_splits(int fmt, int64_t units, int32_t H, int64_t max_list, int64_t min_entries) {
-    constexpr int PLACES = 512, MOST_UNITS = 256 * 5 / 6;
-    const int64_t wgs = units * narrow_groups(H);
-    const int one = one_round_splits(wgs, max_list, min_entries);
-    const bool two_groups = H > 32 && H <= 64;
-    auto at_least = [&](int64_t n) { return std::max<int64_t>(min_entries, n); };
-    if (fmt == DSA_KV_FP8_656 || fmt == DSA_KV_MXFP8_V4) {
-        if (fmt == DSA_KV_FP8_656 && two_groups && wgs > 128) {
-            if (max_list >= 2048 || (max_list >= 1024 && wgs > PLACES / 3 && units <= MOST_UNITS))
-                return one_round_splits(units, max_list, at_least(225), PLACES);
-            if (wgs > PLACES / 3) return 1;
-        }
-        if (fmt == DSA_KV_MXFP8_V4 && wgs >= 256) return 1;
-        return one_round_splits(wgs, max_list, wgs > PLACES / 3 ? at_least(400) : min_entries, PLACES);
+// What a call costs, in us:
+//   work   rounds of workgroups, each `start` and `tile` per 32 rows of its list; of
+//          the pair kernels, CUs that hold two take start2 and tile2
+//   bytes  the rows' bytes, `bytes` per MB
+//   t = (work^4 + bytes^4)^(1/4), and for ns > 1 the combine: `split`, and `part` per
+//       MB of partials
+// Constants fitted to measured times of every kernel at every split count (4 to 2048
+// query tokens of 8 to 64 heads, lists of 200 to 16384 entries; mean error 2 to 3 %,
+// 95 % below 9 %), then moved by up to 8 % each to where the choices cost least.
+// 656-B and V4 fp8 rows are not bound by the rows' bytes.
+struct KernTime { float start, tile, start2, tile2, split, part, bytes; };
+constexpr KernTime KERN_TIME[][4] = {
+    // DSA_KV_BF16: WIDE, NARROW, PAIR, PAIR64
+    {{13.5f, 1.49f, 0, 0, 3.2f, 0.38f, 0.185f}, {10.3f, 1.13f, 0, 0, 2.3f, 0.48f, 0.123f},
+     {8.3f, 1.06f, 11.3f, 1.43f, 2.6f, 0.39f, 0.162f}, {9.1f, 1.54f, 10.9f, 2.10f, 3.3f, 0.30f, 0.154f}},
+    // DSA_KV_FP8_656
+    {{16.0f, 2.02f, 0, 0, 3.0f, 0.40f, 0}, {10.3f, 1.56f, 0, 0, 2.6f, 0.40f, 0},
+     {9.5f, 1.59f, 10.9f, 2.12f, 3.0f, 0.39f, 0}, {10.2f, 2.15f, 11.3f, 2.94f, 3.3f, 0.31f, 0}},
+    // DSA_KV_BF16_D512
+    {{13.1f, 1.56f, 0, 0, 3.0f, 0.39f, 0.190f}, {10.2f, 1.06f, 0, 0, 1.5f, 0.47f, 0.128f},
+     {9.8f, 1.02f, 10.9f, 1.37f, 1.8f, 0.37f, 0.157f}, {11.7f, 1.39f, 10.8f, 2.15f, 1.7f, 0.36f, 0.146f}},
+    // DSA_KV_MXFP8 (its kernel is pair_kern's)
+    {},
+    // DSA_KV_MXFP8_V4 (no NARROW kernel)
+    {{13.9f, 2.28f, 0, 0, 2.6f, 0.39f, 0}, {},
+     {10.6f, 2.04f, 12.4f, 2.53f, 1.5f, 0.36f, 0}, {11.6f, 2.54f, 12.3f, 3.37f, 2.0f, 0.31f, 0}},
+};
+double kern_time(int fmt, Kern k, int64_t tokens, int32_t H, int64_t list, int ns) {
+    const KernTime& c = KERN_TIME[fmt][k];
+    const int64_t wgs = tokens * groups_of(k, H) * ns, tiles = ((list + ns - 1) / ns + TILE - 1) / TILE;
+    int64_t once = (wgs + CUS - 1) / CUS, twice = 0;    // rounds of one and of two workgroups per CU
+    if (k == PAIR || k == PAIR64) {
+        const int64_t rest = wgs % (2 * CUS);
+        once = rest > 0 && rest <= CUS ? 1 : 0;
+        twice = wgs / (2 * CUS) + (rest > CUS ? 1 : 0);
     }
-    if (wgs <= PLACES / 3 && (wgs > 128 || (two_groups && wgs >= 64)))
-        return std::max(one, one_round_splits(wgs, max_list, at_least(320), PLACES));
-    if (two_groups && wgs > PLACES / 3 && units <= MOST_UNITS && max_list >= 2048)
-        return one_round_splits(units, max_list, at_least(400), PLACES);
-    return one;
+    const double work = once * (c.start + (double)tiles * c.tile) + twice * (c.start2 + (double)tiles * c.tile2);
+    const double row = fmt == DSA_KV_BF16 ? BF16_ROW : 2 * D_VO;
+    const double bytes = (double)tokens * list * row * 1e-6 * c.bytes;
+    double t = std::sqrt(std::sqrt(work * work * work * work + bytes * bytes * bytes * bytes));
+    if (ns > 1) t += c.split + c.part * 1e-6 * ns * tokens * H * (D_VO + 1) * sizeof(float);
+    return t;
+}
+
+// Kernel and split count (`requested`, or 0: automatic, of at most by_len) of a call
+// of `tokens` query tokens over lists of up to `list` entries: the least expected time
+// of the kernels that it can run, unsplit, in one round of CUs, and (pair kernels) in
+// both places of every CU.  Of 3400 calls measured with every kernel and count, the
+// choice is within 0.2 % of the fastest such one on average and 5 % at most; 128-head
+// workgroups win where their one round just fills the GPU (V4 fp8 rows, 256 tokens of
+// 64 heads x 640 rows 60.6 us, 66.0 and 63.1 in 32 and 64 heads) and 64-head ones, in
+// splits, on either side of it (x 1664 122.6 us in two splits, 132.4 on WIDE).
+// NARROW is for one round at most: past it, a second workgroup per CU covers the first
+// one's waits.  Beyond 64 heads PAIR is only for what NARROW cannot hold in a round
+// (its head groups lie 8 apart, which costs where splits of 8 or 16 tokens meet on an
+// XCD: 16 tokens of 128 heads x 1024 656-B rows 37.3 us, NARROW 32.1).
+struct Choice {
+    Kern kern;
+    int ns;
+};
+Choice choose_kern(int fmt, int64_t tokens, int32_t H, int64_t list, int requested, int64_t by_len) {
+    Choice best{WIDE, requested > 0 ? requested : one_round_splits(tokens * head_groups(H), by_len)};
+    if (tokens <= 0 || !narrow_path(fmt, tokens, H, best.ns)) return best;
+    double least = -1.0;
+    for (Kern k : {WIDE, NARROW, PAIR, PAIR64}) {
+        if ((k == WIDE && H > 64) || (k == NARROW && !has_narrow(fmt)) || (k == PAIR64 && (H <= 32 || H > 64)))
+            continue;
+        const bool pair = k == PAIR || k == PAIR64;
+        const int64_t wgs = tokens * groups_of(k, H);
+        const int counts[] = {1, one_round_splits(wgs, by_len), one_round_splits(wgs, by_len, pair ? 2 * CUS : CUS)};
+        for (int ns : counts) {
+            if (requested > 0) ns = requested;
+            if (k == NARROW && wgs * ns > CUS) continue;
+            if (k == PAIR && H > 64 && wgs * ns <= CUS) continue;
+            const double t = kern_time(fmt, k, tokens, H, list, ns);
+            if (least >= 0 && t >= least) continue;
+            least = t;
+            best = Choice{k, ns};
+        }
+    }
+    return best;
 }
 // decode: at least 4 tiles per split (at top-k 2048 and B = 2 or 4: 16 splits
 // measured 11 % faster than 8 and 6 % faster than 32)
 constexpr int DECODE_MIN = 128;
-int auto_splits(int64_t wgs, int topk) { return one_round_splits(wgs, (int64_t)topk + DECODE_MIN - 1, DECODE_MIN); }
+int64_t decode_by_len(int64_t list) { return (list + DECODE_MIN - 1) / DECODE_MIN; }
 
-// A top-k decode call: its split count (the caller's, or the automatic one for the
-// kernel narrow_path picks), the entries of a split, and the kernel.
+// A top-k decode call: its split count, the entries of a split, and the kernel.
 struct DecodePlan {
     int ns, chunk;
     Kern kern;
 };
 DecodePlan decode_plan(const dsa_mla_decode_args* a) {
-    const int64_t tokens = (int64_t)a->B * a->s_q;
-    DecodePlan p{a->num_splits ? a->num_splits : auto_splits(tokens * head_groups(a->H), a->topk), 0, WIDE};
-    if (narrow_path(a->kv_format, tokens, a->H, p.ns)) {
-        if (!a->num_splits)
-            p.ns = narrow_splits(a->kv_format, tokens, a->H, (int64_t)a->topk + DECODE_MIN - 1, DECODE_MIN);
-        p.kern = narrow_kern(a->kv_format, tokens * p.ns, a->H);
-    }
-    p.chunk = a->topk == 0 ? 0 : (a->topk + p.ns - 1) / p.ns;
-    return p;
+    const Choice c = choose_kern(a->kv_format, (int64_t)a->B * a->s_q, a->H, a->topk, a->num_splits,
+                                 decode_by_len(a->topk));
+    return DecodePlan{c.ns, a->topk == 0 ? 0 : (a->topk + c.ns - 1) / c.ns, c.kern};
 }
 // The split count of a no-allocation call whose automatic partials do not fit the
 // scratch (two 32- or 64-head workgroups to a CU): the fewest splits, of at least
@@ -3993,8 +4016,8 @@ DecodePlan decode_plan(const dsa_mla_decode_args* a) {
 // in one up to 64 heads, 32 in each beyond.
 int noalloc_splits(const dsa_mla_decode_args* a) {
     const int64_t wgs = (int64_t)a->B * a->s_q * (a->H <= 64 ? 1 : narrow_groups(a->H));
-    const int64_t by_len = std::max<int64_t>(1, ((int64_t)a->topk + DECODE_MIN - 1) / DECODE_MIN);
-    return (int)std::min<int64_t>(std::min<int64_t>((256 + wgs - 1) / wgs, by_len), DSA_MLA_MAX_SPLITS);
+    const int64_t by_len = std::max<int64_t>(1, decode_by_len(a->topk));
+    return (int)std::min<int64_t>(std::min<int64_t>((CUS + wgs - 1) / wgs, by_len), DSA_MLA_MAX_SPLITS);
 }
 
 int validate_decode(const dsa_mla_decode_args* a, DecodePlan* plan) {
@@ -4213,13 +4236,8 @@ size_t mx_ws_bytes(const dsa_mla_decode_mxfp8_args* a, int ns) {
 // Split count and kernel of a prefill call (N query tokens, lists of at most
 // max_list entries).
 constexpr int PREFILL_MIN = 256;
-int prefill_plan(int fmt, int64_t N, int32_t H, int requested, int64_t max_list, Kern* kern) {
-    const int wide = requested > 0 ? requested : one_round_splits(N * head_groups(H), max_list, PREFILL_MIN);
-    *kern = WIDE;
-    if (!narrow_path(fmt, N, H, wide)) return wide;
-    const int ns = requested > 0 ? requested : narrow_splits(fmt, N, H, max_list, PREFILL_MIN);
-    *kern = narrow_kern(fmt, N * ns, H);
-    return ns;
+Choice prefill_plan(int fmt, int64_t N, int32_t H, int requested, int64_t max_list) {
+    return choose_kern(fmt, N, H, max_list, requested, max_list / PREFILL_MIN);
 }
 size_t prefill_ws_bytes(int ns, int64_t N, int H) {
     return ns <= 1 || N == 0 ? 0 : (size_t)ns * N * H * (D_VO + 1) * sizeof(float) + 256;
@@ -4250,8 +4268,7 @@ int validate_prefill(const dsa_mla_prefill_args* a, int* ns_out) {
     if (row_stride_bytes(a->kv_format, a->kv_stride_row) < 0) return DSA_ERR_BAD_STRIDE;
     if (a->topk > MAX_LIST) return DSA_ERR_BAD_SHAPE;
     if (a->num_splits < 0 || a->num_splits > DSA_MLA_MAX_SPLITS) return DSA_ERR_BAD_SPLITS;
-    Kern kern;
-    *ns_out = prefill_plan(a->kv_format, a->N, a->H, a->num_splits, a->topk, &kern);
+    *ns_out = prefill_plan(a->kv_format, a->N, a->H, a->num_splits, a->topk).ns;
     if (a->N == 0) return DSA_OK;
     if (!a->q || !a->out || (a->topk > 0 && (!a->kv || !a->indices))) return DSA_ERR_NULL_POINTER;
     if ((a->q_stride_n % 8) || (a->q_stride_h % 8) || (a->o_stride_n % 4) || (a->o_stride_h % 4))
@@ -4270,8 +4287,7 @@ int validate_v4(const dsa_mla_prefill_v4_args* a, int* ns_out) {
     if (!heads_ok(a->H, a->N)) return DSA_ERR_BAD_SHAPE;
     if (a->D != DSA_MLA_D_V4) return DSA_ERR_UNSUPPORTED;
     if (a->num_splits < 0 || a->num_splits > DSA_MLA_MAX_SPLITS) return DSA_ERR_BAD_SPLITS;
-    Kern kern;
-    *ns_out = prefill_plan(DSA_KV_BF16_D512, a->N, a->H, a->num_splits, a->max_rows, &kern);
+    *ns_out = prefill_plan(DSA_KV_BF16_D512, a->N, a->H, a->num_splits, a->max_rows).ns;
     if (a->N == 0) return DSA_OK;
     if (!a->q || !a->out || !a->kv_indptr_prefix || !a->kv_indices_prefix || !a->kv_indptr_extend ||
         !a->kv_indices_extend)
@@ -4294,8 +4310,7 @@ int validate_v4fp8(const dsa_mla_prefill_v4_fp8_args* a, int* ns_out) {
     if (a->max_rows > MAX_LIST) return DSA_ERR_BAD_SHAPE;
     if (!heads_ok(a->H, a->N)) return DSA_ERR_BAD_SHAPE;
     if (a->num_splits < 0 || a->num_splits > DSA_MLA_MAX_SPLITS) return DSA_ERR_BAD_SPLITS;
-    Kern kern;
-    *ns_out = prefill_plan(DSA_KV_MXFP8_V4, a->N, a->H, a->num_splits, a->max_rows, &kern);
+    *ns_out = prefill_plan(DSA_KV_MXFP8_V4, a->N, a->H, a->num_splits, a->max_rows).ns;
     if (a->N == 0) return DSA_OK;
     if (!a->q_nope || !a->q_rope || !a->out || !a->kv_indptr_prefix || !a->kv_indices_prefix ||
         !a->kv_indptr_extend || !a->kv_indices_extend)
@@ -4463,10 +4478,9 @@ int dsa_mla_decode_csr(const dsa_mla_decode_csr_args* a, void* ws, size_t ws_byt
     if (need && (!ws || ws_bytes < need || ((uintptr_t)ws & 15))) return DSA_ERR_WORKSPACE;
     if (a->B == 0) return DSA_OK;
     hipStream_t st = (hipStream_t)stream;
-    // uniform splits (no work plan) of few query rows or few heads: 32-head workgroups
+    // (a work plan's kernel is csr_plan_launch's)
     const int64_t rows_q = (int64_t)a->B * a->s_q;
-    const Kern kern = ns >= 1 && narrow_path(a->kv_format, rows_q, a->H, ns)
-                          ? narrow_kern(a->kv_format, rows_q * ns, a->H) : WIDE;
+    const Kern kern = ns >= 1 ? choose_kern(a->kv_format, rows_q, a->H, a->max_kv_len, ns, 0).kern : WIDE;
     FwdParams fp{};
     fp.H = a->H;
     fp.hgroups = groups_of(kern, a->H);
@@ -4576,8 +4590,7 @@ int dsa_mla_prefill(const dsa_mla_prefill_args* a, void* ws, size_t ws_bytes, vo
     const size_t need = prefill_ws_bytes(ns, a->N, a->H);
     if (need && (!ws || ws_bytes < need || ((uintptr_t)ws & 15))) return DSA_ERR_WORKSPACE;
     if (a->N == 0) return DSA_OK;
-    Kern kern;
-    prefill_plan(a->kv_format, a->N, a->H, a->num_splits, a->topk, &kern);
+    const Kern kern = prefill_plan(a->kv_format, a->N, a->H, a->num_splits, a->topk).kern;
     FwdParams fp{};
     fp.H = a->H;
     fp.hgroups = groups_of(kern, a->H);
@@ -4622,8 +4635,7 @@ int dsa_mla_prefill_v4(const dsa_mla_prefill_v4_args* a, void* ws, size_t ws_byt
     const size_t need = prefill_ws_bytes(ns, a->N, a->H);
     if (need && (!ws || ws_bytes < need || ((uintptr_t)ws & 15))) return DSA_ERR_WORKSPACE;
     if (a->N == 0) return DSA_OK;
-    Kern kern;
-    prefill_plan(DSA_KV_BF16_D512, a->N, a->H, a->num_splits, a->max_rows, &kern);
+    const Kern kern = prefill_plan(DSA_KV_BF16_D512, a->N, a->H, a->num_splits, a->max_rows).kern;
     FwdParams fp{};
     fp.H = a->H;
     fp.hgroups = groups_of(kern, a->H);
@@ -4661,8 +4673,7 @@ int dsa_mla_prefill_v4_fp8(const dsa_mla_prefill_v4_fp8_args* a, void* ws, size_
     const size_t need = prefill_ws_bytes(ns, a->N, a->H);
     if (need && (!ws || ws_bytes < need || ((uintptr_t)ws & 15))) return DSA_ERR_WORKSPACE;
     if (a->N == 0) return DSA_OK;
-    Kern kern;
-    prefill_plan(DSA_KV_MXFP8_V4, a->N, a->H, a->num_splits, a->max_rows, &kern);
+    const Kern kern = prefill_plan(DSA_KV_MXFP8_V4, a->N, a->H, a->num_splits, a->max_rows).kern;
     FwdParams fp{};
     fp.H = a->H;
     fp.hgroups = groups_of(kern, a->H);

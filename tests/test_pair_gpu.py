@@ -151,7 +151,8 @@ def test_v4_bf16(dev, H, topk, splits):
     assert_parity(bits(out), lse.cpu().numpy(), o_ref, l_ref, f"pair V4 bf16 H={H}")
 
 
-@pytest.mark.parametrize("H,N,topk", [(16, 300, 1100), (32, 40, 300), (40, 260, 1100), (64, 140, 700), (33, 300, 20)])
+@pytest.mark.parametrize("H,N,topk", [(16, 300, 1100), (32, 40, 300), (40, 260, 1100), (64, 140, 700), (33, 300, 20),
+                                      (40, 256, 500)])      # the last: one round of 128-head workgroups
 def test_v4_fp8(dev, H, N, topk):
     print(f"[case] pair V4 fp8 H={H} N={N}", flush=True)
     q, ukv, xkv, sink, lists = v4fp8_inputs(560 + H, N=N, total_pages=4096, topk=topk)

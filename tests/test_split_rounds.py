@@ -1,10 +1,22 @@
 """Automatic split counts: the workgroups of a split call fit one round of the GPU (256 CUs,
-each holding one 128-head workgroup or up to two 32-head ones)."""
+each holding one 128-head workgroup or up to two smaller ones), the counts are among the fastest
+measured, and neighbouring calls get neighbouring counts."""
 import ctypes
 
 import pytest
 
 from opfoundry_amd import abi
+
+
+def num_splits(fmt, B, H, topk):
+    a = abi.DecodeArgs()
+    for f in ("q", "kv_cache", "block_table", "seq_lens", "indices", "out", "lse"):
+        setattr(a, f, 0x1000)
+    a.kv_format, a.kv_total_rows, a.block_size, a.block_table_stride = fmt, 1 << 20, 64, 1024
+    a.B, a.s_q, a.H, a.topk, a.sm_scale = B, 1, H, topk, 0.07
+    ns = ctypes.c_int32(0)
+    assert abi.load_library().dsa_mla_decode_num_splits(ctypes.byref(a), ctypes.byref(ns)) == 0
+    return ns.value
 
 
 @pytest.mark.parametrize("fmt", [abi.KV_BF16, abi.KV_FP8_656])
@@ -18,33 +30,32 @@ from opfoundry_amd import abi
                                       (100, 64, 512), (213, 16, 512), (214, 16, 512), (256, 16, 2048), (257, 16, 2048),
                                       (256, 64, 2048)])
 def test_splits_fit_one_round(fmt, B, H, topk):
-    a = abi.DecodeArgs()
-    for f in ("q", "kv_cache", "block_table", "seq_lens", "indices", "out", "lse"):
-        setattr(a, f, 0x1000)
-    a.kv_format, a.kv_total_rows, a.block_size, a.block_table_stride = fmt, 1 << 20, 64, 1024
-    a.B, a.s_q, a.H, a.topk, a.sm_scale = B, 1, H, topk, 0.07
-    ns = ctypes.c_int32(0)
-    assert abi.load_library().dsa_mla_decode_num_splits(ctypes.byref(a), ctypes.byref(ns)) == 0
-    cap = max(1, (topk + 127) // 128)
-    wide_wgs = B * ((H + 127) // 128)
-    wide = 1 if wide_wgs >= 256 else min(256 // wide_wgs, cap, 64)
-    if H <= 64 or wide_wgs * wide < 128:       # 32-head workgroups
-        wgs = B * ((H + 31) // 32)
-        two, longest = 32 < H <= 64, topk + 127
-        if two and fmt == abi.KV_FP8_656 and (longest >= 2048 and wgs > 128 or longest >= 1024 and 170 < wgs <= 2 * 213):
-            wgs, round_, cap = B, 512, longest // 225            # 64-head workgroups
-        elif two and fmt == abi.KV_FP8_656 and wgs > 170:
-            cap, round_ = 1, 512
-        elif two and fmt == abi.KV_BF16 and wgs > 170 and B <= 213 and longest >= 2048:
-            wgs, round_, cap = B, 512, longest // 400            # 64-head workgroups
-        elif fmt == abi.KV_BF16 and (128 < wgs <= 170 or two and 64 <= wgs <= 170):
-            one = max(1, min(256 // wgs, cap))
-            round_, cap = 512, max(one, longest // 320)
-        else:
-            round_ = 512 if fmt == abi.KV_FP8_656 else 256
-            if fmt == abi.KV_FP8_656 and wgs > 170:
-                cap = longest // 400
-    else:
-        wgs, round_ = wide_wgs, 256
-    assert ns.value == (1 if wgs >= round_ else max(1, min(round_ // wgs, cap, 64)))
-    assert wgs >= round_ or wgs * ns.value <= round_
+    """A split call's workgroups fit the GPU's places (256 CUs: one 128-head workgroup each, or two
+    of 32 or 64 heads), and a split keeps at least four tiles of the list."""
+    ns = num_splits(fmt, B, H, topk)
+    wide = max(1, min(256 // min(256, B * ((H + 127) // 128)), -(-topk // 128)))
+    small = H <= 64 or B * ((H + 127) // 128) * wide < 128       # 32- or 64-head workgroups
+    wgs = B * ((H + 63) // 64 if 32 < H <= 64 else (H + 31) // 32 if small else (H + 127) // 128)
+    assert ns == 1 or wgs * ns <= (512 if small else 256)
+    assert 1 <= ns <= max(1, -(-topk // 128))
+
+
+# the split counts within 6 % of the fastest measured kernel and count
+@pytest.mark.parametrize("fmt,H,topk,B,fast", [
+    (abi.KV_BF16, 40, 1920, 128, (2, 3, 4)), (abi.KV_BF16, 64, 1920, 128, (2, 3)), (abi.KV_BF16, 64, 1024, 128, (1,)),
+    (abi.KV_BF16, 64, 2048, 100, (4, 5)), (abi.KV_BF16, 64, 1920, 100, (2, 4, 5)), (abi.KV_BF16, 40, 512, 43, (2, 4)),
+    (abi.KV_BF16, 64, 1024, 213, (1,)), (abi.KV_BF16, 16, 2048, 75, (3, 4, 5, 6)), (abi.KV_BF16, 24, 256, 86, (1,)),
+    (abi.KV_FP8_656, 32, 1024, 64, (4,)), (abi.KV_FP8_656, 32, 1536, 32, (7, 8)), (abi.KV_FP8_656, 32, 2048, 32, (8,)),
+    (abi.KV_FP8_656, 32, 512, 128, (2,)), (abi.KV_FP8_656, 16, 2048, 75, (5, 6)), (abi.KV_FP8_656, 16, 2048, 256, (2,)),
+    (abi.KV_FP8_656, 64, 2048, 150, (3,)), (abi.KV_FP8_656, 64, 1024, 150, (3,)), (abi.KV_FP8_656, 64, 512, 100, (1,)),
+    (abi.KV_FP8_656, 128, 2048, 5, (8, 10, 12)), (abi.KV_FP8_656, 128, 2048, 6, (8, 10)),
+    (abi.KV_FP8_656, 96, 2048, 7, (8, 10, 12))])
+def test_counts_against_measured_times(fmt, H, topk, B, fast):
+    assert num_splits(fmt, B, H, topk) in fast
+
+
+@pytest.mark.parametrize("fmt,B,H", [(abi.KV_BF16, 100, 64), (abi.KV_FP8_656, 100, 64), (abi.KV_FP8_656, 74, 16)])
+def test_no_cliff_between_neighbouring_lists(fmt, B, H):
+    """One entry more, of lists that differ by little, does not unsplit a call or split it many ways."""
+    ns = [num_splits(fmt, B, H, k) for k in range(1850, 2049)]
+    assert max(ns) - min(ns) <= 1
