@@ -46,6 +46,14 @@ __device__ __forceinline__ void wait_vm() {
     __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 0xF) | ((N >> 4) << 14));
 }
 
+// The lane id anew, from no register that would have to be kept for it.
+__device__ __forceinline__ int fresh_lane() {
+    int v;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(v));
+    return v;
+}
+
+
 // Opaque copy: stops the compiler from hoisting per-lane address math out of
 // the tile loop (which would pin dozens of loop-invariant VGPRs).
 __device__ __forceinline__ int opaque(int v) {

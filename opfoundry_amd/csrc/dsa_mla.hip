@@ -220,13 +220,14 @@ __device__ __forceinline__ int32_t sload(const int32_t* ptr) {
     return *(const __attribute__((address_space(4))) int32_t*)(uintptr_t)ptr;
 }
 
-// Inclusive prefix sum over the wave's lanes of v (0 <= v < 16): from the
-// ballots of v's four bits, each counted below the lane (v_mbcnt), with no
-// LDS round trip.
+// Inclusive prefix sum over the wave's lanes of v (0 <= v < 2^BITS): from the
+// ballots of v's bits, each counted below the lane (v_mbcnt), with no LDS round
+// trip.
+template <int BITS = 4>
 __device__ __forceinline__ int wave_incl_sum16(int v) {
     int excl = 0;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < BITS; ++k) {
         const uint64_t m = __builtin_amdgcn_ballot_w64(((v >> k) & 1) != 0);
         excl += (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u)) << k;
     }
@@ -2473,7 +2474,7 @@ dsa_mla_fwd_narrow_kernel(const FwdParams p_arg) {
 // 86; V4 fp8 rows, 2048 queries x 1152, H = 16, 389 instead of 701.  H = 64, 2048
 // queries, 128-head workgroups / two of HG = 32 / HG = 64: bf16 rows x 2048
 // 939 / 759 / 585 us, 656-B rows 1136 / 1089 / 755, V4 bf16 x 1152 561 / 473 /
-// 368, V4 fp8 714 / 763 / 484.
+// 368, V4 fp8 714 / 763 / 484 (before its last spills went: 4 % less now).
 // grid = (tokens or plan items x ceil(H / HG), s_q, num_splits), block = 256.
 // ---------------------------------------------------------------------------
 template <int NF, int HG>
@@ -2513,6 +2514,7 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
     using L = PairLay<NF, HG>;
     constexpr int QB = HG / 32;                   // 16-row blocks of a wave's QK^T, 32-head blocks of its PV
     constexpr bool D512 = L::D512, F16 = L::F16, RAW = L::RAW;
+    constexpr bool CSR = NF == DSA_KV_MXFP8;      // (MXFP8 lists have the CSR form alone)
     __shared__ __attribute__((aligned(1024))) unsigned char s_pool[L::BYTES];
     const lds_ptr POOL = (lds_ptr)s_pool;
     const lds_ptr PX = POOL + L::PXO;
@@ -2629,8 +2631,14 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
     // QK^T: 32 heads: row half and head half; 64 heads: both row halves, head quarter
     const int rb = HG == 64 ? 0 : wave & 1, hb = HG == 64 ? wave : wave >> 1;
     const int c16 = lane & 15, g4 = lane >> 4;    // 16x16 operand lanes
-    const int hi = lane >> 5, r32 = lane & 31;    // PV and epilogue lanes: head r32
     const int hq = 16 * hb + c16;                 // this lane's head in QK^T and the softmax
+    // The lane id outside the tile loop (64 heads: anew each time, so that none of the
+    // addresses formed from it is kept in a register across the loop: with Q and O
+    // there, that spilled up to 16)
+    auto lane_now = [&]() -> int {
+        if constexpr (HG == 64) return fresh_lane();
+        else return opaque(lane);
+    };
     // (heads past H: a copy of head H-1, never stored)
     if (tid == 0) {
         s_misc[NWAVE] = 0;
@@ -2655,7 +2663,7 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
         k0 = (int)min((int64_t)split * cb, n_b);
         k1 = (int)min((int64_t)k0 + cb, n_b);
         idx = p.idx_pre + pb;
-    } else if (p.kv_indptr) {
+    } else if (CSR || p.kv_indptr) {
         const int64_t kb = sload(p.kv_indptr + b);
         const int64_t count = (int64_t)sload(p.kv_indptr + b + 1) - kb - (p.s_q - 1 - t);
         k1 = (int)min(p.plan_items ? (int64_t)item_k1 : (int64_t)k0 + p.chunk, count);
@@ -2672,7 +2680,7 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
     const int nchunks = k1 > k0 ? (k1 - k0 + MC - 1) / MC : 1;
     // the entries of chunk c (-1 past the split's end); V4: entry k is an
     // extend entry from k = v4_np on
-    auto load_entries = [&](int c, int32_t (&jv)[PER_T]) {
+    auto load_entries = [&](int c, int tid, int32_t (&jv)[PER_T]) {
         const int kc0 = k0 + c * MC;
         const int kc1 = min(kc0 + MC, k1);
 #pragma unroll
@@ -2685,9 +2693,9 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
     // chunk 0's entries, and a paged list's block-table reads for them, before Q:
     // vmcnt counts in order, so waiting for them does not wait for Q
     int32_t jv0[PER_T], ent0[PER_T];
-    load_entries(0, jv0);
+    load_entries(0, tid, jv0);
     int64_t jmax = 0;
-    const bool topk_form = !D512 && !p.kv_indptr;
+    const bool topk_form = !D512 && !CSR && !p.kv_indptr;
     if (topk_form) {
         const int64_t Lq = p.seq_lens ? (int64_t)sload(p.seq_lens + b) : p.seq_len_default;
         jmax = Lq;
@@ -2722,9 +2730,15 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
     // with the head's power-of-two prescale (see dsa_mla_fwd_narrow_kernel)
     auto convert_q = [&]() {
         if constexpr (L::MX) {
+            // (copies the compiler cannot look through: it would unpack all scales
+            // ahead of the chunk loop, in registers that Q and O need)
+            unsigned qs[4] = {q_scales[0], q_scales[1], q_scales[2], q_scales[3]};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if constexpr (CSR && HG == 64) qs[i] = (unsigned)opaque_here((int)qs[i]);
 #pragma unroll
             for (int ks = 0; ks < L::Q8_KS; ++ks)
-                qf[ks] = mx_to_bf16(qf[ks][0], qf[ks][1], (q_scales[ks >> 2] >> (8 * (ks & 3))) & 0xFFu);
+                qf[ks] = mx_to_bf16(qf[ks][0], qf[ks][1], (qs[ks >> 2] >> (8 * (ks & 3))) & 0xFFu);
         } else if constexpr (F16) {
             typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
             u16x2 amax = {0, 0};
@@ -2755,6 +2769,8 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
     int n_valid = 0, ntiles = 0;
     bool any_rows = false;
     auto resolve_chunk = [&](int c, bool preloaded) {
+        const int lane = HG == 64 ? lane_now() : (int)(threadIdx.x & 63);
+        const int tid = HG == 64 ? 64 * wave + lane : (int)threadIdx.x;
         int32_t rows_local[PER_T];
         int cnt = 0;
         {
@@ -2763,7 +2779,7 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
 #pragma unroll
                 for (int e = 0; e < PER_T; ++e) jv[e] = jv0[e];
             } else {
-                load_entries(c, jv);
+                load_entries(c, tid, jv);
             }
             if constexpr (D512) {
                 const int kc0 = k0 + c * MC;
@@ -2771,23 +2787,27 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
                 for (int e = 0; e < PER_T; ++e)
                     rows_local[e] = kc0 + tid * PER_T + e >= v4_np ? dsa_rows::v4_extend_row(jv[e], p.kv2_rows)
                                                                    : dsa_rows::v4_prefix_row(jv[e], p.kv_total_rows);
-            } else if (p.kv_indptr) {
+            } else if (CSR || p.kv_indptr) {
 #pragma unroll
                 for (int e = 0; e < PER_T; ++e) rows_local[e] = dsa_rows::csr_row(jv[e], p.kv_total_rows);
             } else {
+                // (64 heads: a page size the compiler cannot look through, whose
+                // reciprocal it would keep in a register across the tile loop)
+                FwdParams pc = p;
+                if constexpr (HG == 64) asm volatile("" : "+s"(pc.block_size));
                 int32_t ent[PER_T];
                 if (preloaded && topk_paged) {
 #pragma unroll
                     for (int e = 0; e < PER_T; ++e) ent[e] = ent0[e];
                 } else {
-                    topk_ents(p, b, jmax, jv, ent);
+                    topk_ents(pc, b, jmax, jv, ent);
                 }
-                topk_rows_of(p, b, jv, ent, rows_local);
+                topk_rows_of(pc, b, jv, ent, rows_local);
             }
 #pragma unroll
             for (int e = 0; e < PER_T; ++e) cnt += rows_local[e] >= 0 ? 1 : 0;
         }
-        const int incl = wave_incl_sum16(cnt);
+        const int incl = wave_incl_sum16<PER_T < 4 ? 2 : (PER_T < 8 ? 3 : 4)>(cnt);
         // (the barrier also ends every wave's use of the previous chunk's row
         // list, tile buffers and P)
         if (lane == 63) s_misc[wave] = incl;
@@ -3233,7 +3253,7 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
         tile_barrier();
         if constexpr (QB == 1) top = get_max(2);
         top *= c_s;
-        if (pass == 0 && __builtin_amdgcn_ballot_w64(top - m_ref > L::TAU) != 0 && lane == 0) s_misc[NWAVE] = 1;
+        if (pass == 0 && __builtin_amdgcn_ballot_w64(top - m_ref > L::TAU) != 0 && lane_now() == 0) s_misc[NWAVE] = 1;
         tile_barrier();
         if (pass != 0 || s_misc[NWAVE] == 0) break;
         m_ref = fmaxf(m_ref, top);
@@ -3245,9 +3265,10 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
         if (rb == 0 && g4 == 0) s_red[8 * NARROW_HEADS + hq] = m_ref;
     } else {
         const float l_all = red4_sum(l_lane);
-        if (g4 == 0) {
-            s_red[hq] = l_all;
-            s_red[HG + hq] = m_ref;
+        const int el = lane_now();
+        if (el < 16) {
+            s_red[16 * hb + el] = l_all;
+            s_red[HG + 16 * hb + el] = m_ref;
         }
     }
     if (F16 && range_bad) s_misc[NWAVE + 1] = 1;
@@ -3256,6 +3277,8 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
     // NaN outputs, never a silently truncated or wrong attention.
     const bool nan_out = truncated || (F16 && s_misc[NWAVE + 1] != 0);
     const bool has = any_rows;
+    const int ol = HG == 64 ? lane_now() : lane;
+    const int hi = ol >> 5, r32 = ol & 31;        // epilogue lanes: head r32
     float inv[QB], lse_v[QB];                     // of heads hbase + 32 h + r32
 #pragma unroll
     for (int h = 0; h < QB; ++h) {
@@ -3292,7 +3315,7 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
     // 32 h + r32.  Staged through LDS, 32 heads at a time, each wave in its own region
     // (its LDS accesses run in order: no barrier), so that the global stores write
     // whole row pieces of the wave's 128 dims.
-    const int ln = opaque(lane);
+    const int ln = lane_now();
     constexpr int OST = 2 * 128 + 16;               // staged head row: 128 bf16 + pad
     constexpr int PST = 4 * 128 + 16;               // 128 floats + pad
     static_assert(NWAVE * 32 * OST <= L::STAGE, "O stage fits below P");
@@ -3892,10 +3915,11 @@ bool narrow_path(int fmt, int64_t tokens, int32_t H, int wide_splits) {
     return has_narrow(fmt) && tokens * head_groups(H) * wide_splits < 128;
 }
 // Work plans and MXFP8 lists, whose lengths the host does not know: PAIR64 at 33..64
-// heads when the units (rows, or tokens x splits) alone outnumber the CUs: below that
-// each would have a CU to itself, and twice as many workgroups of 32 heads are faster
-// (MXFP8, 256 units, 92.3 against 93.3 us, 100 tokens with their plan 41.8 against
-// 43.3; above, 300 units at H = 64 136 us against 226 on WIDE).
+// heads when the units (rows, or tokens x splits) alone outnumber the CUs.  With a plan,
+// 64 heads x 2048 entries, PAIR and PAIR64: 300 rows of bf16 196 and 157 us, MXFP8 242 and
+// 191; up to 256 rows, in about 256 items, the two are within 5 % of each other (256
+// rows 128 and 133, 151 and 144), and fewer items are faster in 32 heads (8 rows x 512
+// 17 and 20 us).
 Kern pair_kern(int64_t units, int32_t H) {
     return H > 32 && H <= 64 && units > 256 ? PAIR64 : PAIR;
 }
@@ -3937,8 +3961,8 @@ constexpr KernTime KERN_TIME[][4] = {
     // DSA_KV_MXFP8 (its kernel is pair_kern's)
     {},
     // DSA_KV_MXFP8_V4 (no NARROW kernel)
-    {{13.9f, 2.28f, 0, 0, 2.6f, 0.39f, 0}, {},
-     {10.6f, 2.04f, 12.4f, 2.53f, 1.5f, 0.36f, 0}, {11.6f, 2.54f, 12.3f, 3.37f, 2.0f, 0.31f, 0}},
+    {{13.8f, 2.23f, 0, 0, 2.7f, 0.40f, 0}, {},
+     {10.4f, 2.14f, 11.9f, 2.65f, 1.6f, 0.36f, 0}, {10.8f, 2.41f, 11.8f, 3.06f, 2.0f, 0.32f, 0}},
 };
 double kern_time(int fmt, Kern k, int64_t tokens, int32_t H, int64_t list, int ns) {
     const KernTime& c = KERN_TIME[fmt][k];
@@ -3960,11 +3984,10 @@ double kern_time(int fmt, Kern k, int64_t tokens, int32_t H, int64_t list, int n
 // Kernel and split count (`requested`, or 0: automatic, of at most by_len) of a call
 // of `tokens` query tokens over lists of up to `list` entries: the least expected time
 // of the kernels that it can run, unsplit, in one round of CUs, and (pair kernels) in
-// both places of every CU.  Of 3400 calls measured with every kernel and count, the
-// choice is within 0.2 % of the fastest such one on average and 5 % at most; 128-head
-// workgroups win where their one round just fills the GPU (V4 fp8 rows, 256 tokens of
-// 64 heads x 640 rows 60.6 us, 66.0 and 63.1 in 32 and 64 heads) and 64-head ones, in
-// splits, on either side of it (x 1664 122.6 us in two splits, 132.4 on WIDE).
+// both places of every CU.  Of 3600 calls measured with every kernel and count, the
+// choice is within 0.2 % of the fastest such one on average and 5 % at most.  At up to
+// 64 heads 128-head workgroups win where the count given leaves them in one round (V4
+// fp8 rows, 160 tokens of 64 heads x 2048 unsplit 153 us, 164 in 64 heads, 177 in 32).
 // NARROW is for one round at most: past it, a second workgroup per CU covers the first
 // one's waits.  Beyond 64 heads PAIR is only for what NARROW cannot hold in a round
 // (its head groups lie 8 apart, which costs where splits of 8 or 16 tokens meet on an
