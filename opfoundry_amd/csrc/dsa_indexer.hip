@@ -87,18 +87,6 @@ __device__ __forceinline__ int64_t ix_len(const IxParams& p, int64_t L, int t) {
     return min(max(len, (int64_t)0), (int64_t)p.n_cols);
 }
 
-// Inclusive prefix sum over the 64 lanes of a wave: within rows of 16 lanes by DPP
-// row shifts, then the row totals by the row broadcasts of lanes 15 and 31.
-__device__ __forceinline__ uint32_t ix_wave_scan(uint32_t x) {
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);  // row_shr:1
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);  // row_shr:2
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);  // row_shr:4
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);  // row_shr:8
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // row_bcast:15
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // row_bcast:31
-    return x;
-}
-
 // Inclusive sums over the workgroup, of one value per thread (*sum) and of the
 // values that are not 0 (*some), and their totals.
 __device__ __forceinline__ void ix_scan(uint32_t v, LDS_AS uint32_t* part, uint32_t* sum, uint32_t* some,
@@ -106,7 +94,7 @@ __device__ __forceinline__ void ix_scan(uint32_t v, LDS_AS uint32_t* part, uint3
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint64_t any = __builtin_amdgcn_ballot_w64(v != 0);
     uint32_t cn = (uint32_t)__builtin_popcountll(any & (~0ull >> (63 - lane)));
-    v = ix_wave_scan(v);
+    v = wave_incl_scan(v);
     if (lane == 63) {
         part[2 * wave] = v;
         part[2 * wave + 1] = cn;

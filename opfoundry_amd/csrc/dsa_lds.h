@@ -53,6 +53,25 @@ __device__ __forceinline__ int fresh_lane() {
     return v;
 }
 
+// Inclusive prefix of a wave's 64 values under f (0 its neutral value): within rows
+// of 16 lanes by DPP row shifts (a lane whose source lies outside its row takes 0),
+// then the rows' totals by the row broadcasts of lanes 15 and 31.
+template <class F>
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t x, F f) {
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false));  // row_shr:1
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false));  // row_shr:2
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false));  // row_shr:4
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false));  // row_shr:8
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false));  // row_bcast:15
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false));  // row_bcast:31
+    return x;
+}
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
+    return wave_prefix(x, [](uint32_t a, uint32_t b) { return a + b; });
+}
+__device__ __forceinline__ uint32_t wave_incl_max(uint32_t x) {
+    return wave_prefix(x, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+}
 
 // Opaque copy: stops the compiler from hoisting per-lane address math out of
 // the tile loop (which would pin dozens of loop-invariant VGPRs).

@@ -3412,27 +3412,29 @@ dsa_mla_fwd_pair_kernel(const FwdParams p_arg) {
 // ---------------------------------------------------------------------------
 constexpr int PLAN_TARGET = 256;     // workgroups a plan aims at: one per CU
 constexpr int PLAN_MIN_CHUNK = 128;  // entries: at least four tiles per item
-constexpr int PLAN_THREADS = 512;
-constexpr int PLAN_BLOCK = 256;      // rows laid out at a time
+constexpr int PLAN_THREADS = 512;    // and rows laid out at a time
+constexpr int PLAN_ROW_ITEMS = 4;    // most items that a row's own thread writes
 
 // A call that builds its own plan waits for this kernel, one workgroup on one
 // CU: a chain of dependent steps, so it is the number of them that counts.  The
-// chunk is found by 8 waves testing 8 candidates per step (a bisection by one
-// candidate took 11 steps for a 65536-entry list, two barriers each), and the
-// items of a block of rows are written by all threads (one thread per row wrote
-// them in a loop).  8 lists of 5 to 65536 entries: 7.2 us, before 12.0.
+// chunk is found by 8 waves testing 8 candidates per step; sums over a wave are
+// DPP chains.  In a block of rows that have up to PLAN_ROW_ITEMS items each, a
+// row's own thread writes them; where one has more, all threads write the items,
+// which they find by a search behind one more barrier.  One list of 65536
+// entries 6.0 us (25.5 by a bisection and one thread per row), 8 of them 6.0
+// (10.0), 64 of up to 128 entries 3.3 (3.4; 4.1 when every block took the
+// search), 4096 rows 11.2 (25.9 with the search and blocks of 256 rows).
 __global__ void __launch_bounds__(PLAN_THREADS)
 dsa_csr_plan_kernel(const int32_t* __restrict__ indptr, int B, int s_q, int max_len, int4* __restrict__ items,
                     int4* __restrict__ splits, int32_t* __restrict__ hdr) {
     constexpr int NW = PLAN_THREADS / 64;
-    constexpr int RPL = PLAN_BLOCK / 64;      // rows per lane when every wave holds a block
+    constexpr int RPL = PLAN_TARGET / 64;     // rows per lane when every wave holds all of them
     __shared__ long long s_tot[NW];
-    __shared__ int s_len[PLAN_BLOCK];         // entries of the block's rows (-1: longer than max_len)
-    __shared__ int s_end[PLAN_BLOCK];         // items up to and with each row of the block
-    __shared__ int s_slot[PLAN_BLOCK];        // first partial slot of each row
+    __shared__ int s_len[PLAN_THREADS];       // entries of the block's rows (-1: longer than max_len)
+    __shared__ int s_end[PLAN_THREADS];       // items up to and with each row of the block
+    __shared__ int s_slot[PLAN_THREADS];      // first partial slot of each row
     __shared__ int s_cnt[2][NW];
-    __shared__ int s_scan[3][PLAN_BLOCK / 64];
-    __shared__ int s_long;
+    __shared__ int4 s_scan[2][NW];            // per wave: items, partial slots, split rows, `many`
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int rows = B * s_q;
     // entries of row q; -1 for a row longer than max_len
@@ -3442,9 +3444,8 @@ dsa_csr_plan_kernel(const int32_t* __restrict__ indptr, int B, int s_q, int max_
         return L > max_len ? -1 : (int)max(L, (int64_t)0);
     };
     auto items_of = [](int L, int c) -> int { return L <= c ? 1 : (int)((unsigned)L / (unsigned)c + ((unsigned)L % (unsigned)c != 0)); };
-    static_assert(PLAN_TARGET <= PLAN_BLOCK, "below PLAN_TARGET rows, one block holds every row");
+    static_assert(PLAN_TARGET <= PLAN_THREADS, "below PLAN_TARGET rows, one block holds every row");
     int chunk;
-    if (tid == 0) s_long = 0;
     if (rows >= PLAN_TARGET) {
         long long tot = 0;
         for (int q = tid; q < rows; q += PLAN_THREADS) tot += max(len_of(q), 0);
@@ -3473,8 +3474,7 @@ dsa_csr_plan_kernel(const int32_t* __restrict__ indptr, int B, int s_q, int max_
             Lr[i] = q < rows ? s_len[q] : -2;              // (-2: no row, no item)
             lmax = max(lmax, Lr[i]);
         }
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) lmax = max(lmax, __shfl_xor(lmax, off, 64));
+        lmax = __builtin_amdgcn_readlane((int)wave_incl_max(lmax), 63);
         int lo = PLAN_MIN_CHUNK / TILE, hi = max(lo, (lmax + TILE - 1) / TILE);   // in tiles
         for (int step = 0; lo < hi; step ^= 1) {
             // candidates lo + ((hi - lo) (w + 1)) / 9 of wave w, below hi, rising with w
@@ -3482,9 +3482,8 @@ dsa_csr_plan_kernel(const int32_t* __restrict__ indptr, int B, int s_q, int max_
             int n = 0;
 #pragma unroll
             for (int i = 0; i < RPL; ++i) n += Lr[i] == -2 ? 0 : items_of(Lr[i], c);
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) n += __shfl_xor(n, off, 64);
-            if (lane == 0) s_cnt[step][wave] = n;
+            n = (int)wave_incl_scan(n);
+            if (lane == 63) s_cnt[step][wave] = n;
             __syncthreads();
             // the first candidate that fits bounds the chunk from above, the last
             // that does not from below (the other buffer is written next: no barrier)
@@ -3496,55 +3495,50 @@ dsa_csr_plan_kernel(const int32_t* __restrict__ indptr, int B, int s_q, int max_
         }
         chunk = lo * TILE;
     }
-    auto wave_incl = [&](int v) {
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int u = __shfl_up(v, off, 64);
-            if (lane >= off) v += u;
-        }
-        return v;
-    };
-    int item_base = 0, slot_base = 0, split_base = 0;
-    for (int q0 = 0; q0 < rows; q0 += PLAN_BLOCK) {
-        // the block's rows, one per thread of the first waves: items, partial
-        // slots and split rows up to each
+    int item_base = 0, slot_base = 0, split_base = 0, any_many = 0;
+    for (int q0 = 0, buf = 0; q0 < rows; q0 += PLAN_THREADS, buf ^= 1) {
+        // the block's rows, one per thread: items, partial slots and split rows
+        // up to each
         const int q = q0 + tid;
-        const bool mine = tid < PLAN_BLOCK && q < rows;
+        const bool mine = q < rows;
         const int L = mine ? (rows < PLAN_TARGET ? s_len[tid] : len_of(q)) : 0;
         const int n = mine ? items_of(L, chunk) : 0;
         const int ns = n > 1 ? n : 0, sp = n > 1 ? 1 : 0;
-        const int ia = wave_incl(n), ic = wave_incl(ns), id = wave_incl(sp);
-        __syncthreads();    // the last block's items are written
-        if (lane == 63 && tid < PLAN_BLOCK) {
-            s_scan[0][wave] = ia;
-            s_scan[1][wave] = ic;
-            s_scan[2][wave] = id;
+        const int ia = (int)wave_incl_scan(n), ic = (int)wave_incl_scan(ns), id = (int)wave_incl_scan(sp);
+        const int many = (__any(n > PLAN_ROW_ITEMS) ? 1 : 0) | (__any(n > SMALL_SPLITS) ? 2 : 0);
+        if (lane == 63) s_scan[buf][wave] = make_int4(ia, ic, id, many);
+        __syncthreads();        // (and the last block's items are written)
+        int wa = 0, wc = 0, wd = 0, ta = 0, tc = 0, td = 0, tm = 0;
+        for (int w = 0; w < NW; ++w) {
+            const int4 x = s_scan[buf][w];
+            if (w < wave) { wa += x.x; wc += x.y; wd += x.z; }
+            ta += x.x; tc += x.y; td += x.z; tm |= x.w;
         }
-        __syncthreads();
-        int wa = 0, wc = 0, wd = 0, ta = 0, tc = 0, td = 0;
-        for (int w = 0; w < PLAN_BLOCK / 64; ++w) {
-            const int x = s_scan[0][w], y = s_scan[1][w], z = s_scan[2][w];
-            if (w < wave) { wa += x; wc += y; wd += z; }
-            ta += x; tc += y; td += z;
-        }
-        if (tid < PLAN_BLOCK) {
+        const int slot = slot_base + wc + ic - ns;
+        if (n > 1) splits[split_base + wd + id - sp] = make_int4(q, slot, n, 0);
+        any_many |= tm;
+        // item j of a row of L entries in n items
+        auto item = [&](int row, int L, int n, int slot, int j) {
+            const int e0 = L < 0 ? 0 : j * chunk;
+            const int e1 = L < 0 ? 0 : (int)min((int64_t)(j + 1) * chunk, (int64_t)L);
+            return make_int4(row, e0, e1, plan_item_w(n > 1 ? slot + j : -1, j == n - 1));
+        };
+        if (!(tm & 1)) {
+            for (int j = 0; j < n; ++j) items[item_base + wa + ia - n + j] = item(q, L, n, slot, j);
+        } else {
             s_len[tid] = L;
             s_end[tid] = wa + ia;
-            s_slot[tid] = slot_base + wc + ic - ns;
-            if (n > 1) splits[split_base + wd + id - sp] = make_int4(q, slot_base + wc + ic - ns, n, 0);
-            if (n > SMALL_SPLITS) s_long = 1;
-        }
-        __syncthreads();
-        // item i of the block belongs to the first row whose s_end exceeds i
-        for (int i = tid; i < ta; i += PLAN_THREADS) {
-            int r = 0;
+            s_slot[tid] = slot;
+            __syncthreads();
+            // item i of the block belongs to the first row whose s_end exceeds i
+            for (int i = tid; i < ta; i += PLAN_THREADS) {
+                int r = 0;
 #pragma unroll
-            for (int half = PLAN_BLOCK / 2; half >= 1; half >>= 1)
-                if (s_end[r + half - 1] <= i) r += half;
-            const int rl = s_len[r], rn = items_of(rl, chunk), j = i - (s_end[r] - rn);
-            const int e0 = rl < 0 ? 0 : j * chunk;
-            const int e1 = rl < 0 ? 0 : (int)min((int64_t)(j + 1) * chunk, (int64_t)rl);
-            items[item_base + i] = make_int4(q0 + r, e0, e1, plan_item_w(rn > 1 ? s_slot[r] + j : -1, j == rn - 1));
+                for (int half = PLAN_THREADS / 2; half >= 1; half >>= 1)
+                    if ((half < PLAN_TARGET || rows > PLAN_TARGET) && s_end[r + half - 1] <= i) r += half;
+                const int rl = s_len[r], rn = items_of(rl, chunk);
+                items[item_base + i] = item(q0 + r, rl, rn, s_slot[r], i - (s_end[r] - rn));
+            }
         }
         item_base += ta;
         slot_base += tc;
@@ -3557,7 +3551,7 @@ dsa_csr_plan_kernel(const int32_t* __restrict__ indptr, int B, int s_q, int max_
         hdr[PLAN_HDR_B] = B;
         hdr[PLAN_HDR_SQ] = s_q;
         hdr[PLAN_HDR_MAXLEN] = max_len;
-        hdr[PLAN_HDR_LONG] = s_long;           // (written before the last block's barrier)
+        hdr[PLAN_HDR_LONG] = any_many >> 1;    // 0 or 1
     }
 }
 
@@ -4133,9 +4127,10 @@ CsrPlanLayout csr_plan_layout(int B, int s_q, int H, int max_len) {
     L.total = align256(L.pl + (size_t)L.slots_max * H * sizeof(float));
     return L;
 }
-// the plan's grid: (rows + PLAN_TARGET) x head groups workgroups
+// the plan's grid: (rows + PLAN_TARGET) x head groups workgroups.  (So the plan
+// kernel's row counters, at most rows - 1 + PLAN_THREADS, fit too.)
 bool plan_grid_ok(int B, int s_q, int H) {
-    return ((int64_t)B * s_q + PLAN_TARGET) * head_groups(H) <= INT32_MAX - PLAN_THREADS;
+    return ((int64_t)B * s_q + PLAN_TARGET) * head_groups(H) <= INT32_MAX - 256;
 }
 // the plan kernel alone (into a workspace laid out by csr_plan_layout)
 int csr_plan_build(const int32_t* kv_indptr, int B, int s_q, int H, int max_len, void* ws, hipStream_t st) {

@@ -31,6 +31,7 @@
 #include <stdint.h>
 
 #include "dsa_topk.h"
+#include "dsa_lds.h"
 
 namespace {
 
@@ -395,19 +396,6 @@ __device__ __forceinline__ uint32_t order_key_sel(float x) {
 // workgroup barrier over LDS only: outstanding global loads stay in flight
 __device__ __forceinline__ void lds_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-// Inclusive prefix sum over the 64 lanes of a wave: Hillis-Steele within each
-// row of 16 lanes by DPP row shifts (a lane whose source lies outside its row
-// adds 0), then the row totals by the row broadcasts of lanes 15 and 31.
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);  // row_shr:1
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);  // row_shr:2
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);  // row_shr:4
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);  // row_shr:8
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // row_bcast:15 -> rows 1, 3
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // row_bcast:31 -> rows 2, 3
-    return x;
 }
 
 // Exclusive sum over the workgroup of one value per thread, *total the sum.  One

@@ -241,6 +241,9 @@ def test_csr_split_plan():
     assert rc == 0 and ws_big < 512 * row + (100_000 + 512) * 16 + (1 << 16)
     # one explicit split: no workspace
     assert _csr_ws(lib, _csr_args(num_splits=1)) == (0, 0)
+    # the most rows a plan takes: rows + 256 items in a grid below 2^31 - 256
+    assert _csr_ws(lib, _csr_args(B=2 ** 31 - 513, s_q=1, max_kv_len=128))[0] == 0
+    assert _csr_ws(lib, _csr_args(B=2 ** 31 - 512, s_q=1, max_kv_len=128))[0] == -2
 
 
 @pytest.mark.parametrize("kw,code", [

@@ -1,8 +1,9 @@
-"""The CSR work plan and its combine at their edges: row counts around a block of 256 and
-around the rule's 256, lengths that put the chunk search on its bounds, rows of more items
-than one wave merges at a time (16), and the plan's invariants (items in row order, each at
-most `chunk` long, the smallest such chunk whose items fit 256 workgroups).  Outputs against
-one workgroup per row (num_splits = 1): the same sums in another order.
+"""The CSR work plan and its combine at their edges: row counts around a block of 512 and
+around the rule's 256, lengths that put the chunk search on its bounds, rows of at most 4
+items beside rows of more, rows of just as many items as one wave merges (16) and of one
+more, and the plan's invariants (items in row order, each at most `chunk` long, the smallest
+such chunk whose items fit 256 workgroups; the split rows and where their items' results
+lie).  Outputs against one workgroup per row (num_splits = 1): the same sums in another order.
 """
 import numpy as np
 import pytest
@@ -19,17 +20,23 @@ def plan_of(dev, lens, s_q, H):
     longest = int(max(lens))
     ws = dsa.csr_plan(indptr, len(lens), s_q, H, longest)
     torch.cuda.synchronize()
-    hdr = ws[:24].cpu().numpy().view(np.int32)
-    items = ws[256:256 + 16 * int(hdr[0])].cpu().numpy().view(np.int32).reshape(-1, 4)
-    return indptr, longest, ws, hdr, items
+    hdr = ws[:28].cpu().numpy().view(np.int32)
+    records = lambda at, n: ws[at:at + 16 * n].cpu().numpy().view(np.int32).reshape(-1, 4)  # noqa: E731
+    items = records(256, int(hdr[0]))
+    # the split rows follow room for rows + 256 items, on a multiple of 256 bytes
+    split_rows = records(-(-(256 + 16 * (len(lens) * s_q + 256)) // 256) * 256, int(hdr[1]))
+    return hdr, items, split_rows
 
 
 @pytest.mark.parametrize("lens,s_q", [([1] * 255, 1), ([1] * 256, 1), ([1] * 257, 1), ([129] * 300, 2), ([4097], 1),
                                       ([128] * 5 + [70001], 1), ([65536, 5, 0, 33000], 2), ([200000], 3),
-                                      (list(range(1, 250)), 1), ([2048] * 130, 1), ([100003] + [31] * 700, 1)])
+                                      (list(range(1, 250)), 1), ([2048] * 130, 1), ([100003] + [31] * 700, 1),
+                                      ([600] * 200, 1), ([512, 513] * 3, 1), ([640, 641], 1), ([2048, 7], 1),
+                                      ([2049, 7], 1), ([16384] * 2, 1), ([31] * 511, 1), ([300] * 512, 1),
+                                      ([31] * 513 + [9000] * 3, 1), ([1, 20000, 2] * 400, 1), ([40] * 1023 + [5000], 1)])
 def test_plan_rule(dev, lens, s_q):
     print(f"[case] plan of {len(lens)} lists, s_q={s_q}", flush=True)
-    _, _, _, hdr, items = plan_of(dev, lens, s_q, 16)
+    hdr, items, split_rows = plan_of(dev, lens, s_q, 16)
     L = np.maximum(np.repeat(np.array(lens, np.int64), s_q) - np.tile(np.arange(s_q)[::-1], len(lens)), 0)
     chunk = int(hdr[2])
     count = lambda c: int(np.maximum(1, -(-L // c)).sum())  # noqa: E731
@@ -45,11 +52,21 @@ def test_plan_rule(dev, lens, s_q):
     slot = (items[:, 3] & ((1 << 30) - 1)) - 1
     assert (slot[n[row] == 1] == -1).all() and (slot[n[row] > 1] == np.arange((n[row] > 1).sum())).all()
     assert ((items[:, 3] >> 30 & 1) == (j == n[row] - 1)).all()
+    split = n > 1
+    first = np.cumsum(np.where(split, n, 0)) - n
+    want = np.stack([np.flatnonzero(split), first[split], n[split], np.zeros(split.sum(), np.int64)], 1)
+    assert int(hdr[1]) == split.sum() and (split_rows == want).all()
+    assert list(hdr[3:6]) == [len(lens), s_q, max(lens)]
+    assert hdr[6] == int((n > 16).any())
 
 
-@pytest.mark.parametrize("lens", [[2100, 40], [2200, 40], [8000, 0, 130], [16400, 16400]])
-def test_combine_of_many_items(dev, lens):
-    """16, 17, ~60 and 128 items per row (chunks of 128)."""
+@pytest.mark.parametrize("lens,counts", [([2048, 40], [16, 1]), ([2049, 40], [17, 1]), ([2048, 2049], [16, 17]),
+                                         ([8000, 0, 130], [63, 1, 2]), ([16384, 16384], [128, 128])])
+def test_combine_of_many_items(dev, lens, counts):
+    """Rows of as many items as one wave merges (16), of one more, and up to the 128 that two
+    rows can have, all of 128 entries but the last."""
+    _, items, _ = plan_of(dev, lens, 1, 128)
+    assert np.bincount(items[:, 0]).tolist() == counts
     rng = np.random.default_rng(sum(lens))
     B, H, rows = len(lens), 128, 4096
     t = lambda a: torch.from_numpy(a.view(np.int16)).view(torch.bfloat16).to(dev)  # noqa: E731
