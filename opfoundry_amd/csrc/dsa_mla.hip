@@ -374,9 +374,16 @@ __device__ __forceinline__ void add_sink(float l_rows, float m, float sink2, flo
 // ---------------------------------------------------------------------------
 // Fused sparse-MLA forward: one workgroup per (query token, split).
 // grid = (B, s_q, num_splits), block = 256.
+// Its 47 to 67 KB of code are about what the instruction cache of two CUs holds, so
+// where they lie counts: the same code 8.5 KB further down ran 24 tokens x 2048
+// 656-B rows in 52.5 us instead of 51.5, 119 MXFP8 tokens in 60.0 instead of 58.7.
+// At a multiple of 64 KB, with the combine kernels that follow a split call at one of
+// 16 KB, neither moves with the code before it.  (Of five such pairs the one with no
+// slow format: over 75 calls none more than 0.8 % above the better of two former
+// places; 16 KB and 8 KB left 656-B rows 1.6 % slower in places.)
 // ---------------------------------------------------------------------------
 template <int FMT>
-__global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(1, 1)))
+__global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(1, 1), aligned(65536)))
 dsa_mla_fwd_kernel(const FwdParams p) {
     using L = Lay<FMT>;
     constexpr bool FP8 = L::FP8;
@@ -2457,7 +2464,9 @@ dsa_mla_fwd_narrow_kernel(const FwdParams p_arg) {
 //   row list      512 to 2048 entries at a time, as the format leaves room
 // Tile rows are 1040 bytes apart (a 16-byte pad: 16 rows start at 16 distinct
 // 16-byte bank groups), and a row's 16-byte chunk c sits at c ^ 4 (r & 3), so
-// that the transposed V reads (4 rows x 4 chunks) are spread as well.
+// that the transposed V reads (4 rows x 4 chunks) are spread as well.  (Counted,
+// bank conflicts are still 31 % of the LDS-active cycles for 656-B rows and 39 %
+// for V4 fp8, raw-row reads and conversion stores included.)
 // Formats: those of the narrow kernel, MXFP8 split streams and V4 fp8 rows (both
 // converted exactly to bf16); index forms: top-k, CSR with uniform splits or a
 // work plan, V4.  Arithmetic per tile as in dsa_mla_fwd_narrow_kernel.
@@ -2466,8 +2475,10 @@ dsa_mla_fwd_narrow_kernel(const FwdParams p_arg) {
 // which leaves few for reads ahead: row ids are read when they are needed, K
 // two k-steps ahead instead of six, fp8 rows converted four at a time.  Rows are
 // gathered, converted and read for PV once instead of once per 32 heads.
-// Bound by the LDS and VALU work of both workgroups.  HG = 32 against the narrow
-// kernel:
+// No unit is near full (V4 fp8 rows, HG = 64: VALU issues 41 % of the cycles, LDS
+// active 42 %, MFMA busy 22 %; 656-B rows of 16 heads 26, 27 and 10): it is bound by
+// the order of a workgroup's phases and their barriers, which the CU's other
+// workgroup covers in part.  HG = 32 against the narrow kernel:
 // 4096 queries x 2048 bf16 rows, H = 16, 747 us instead of 1226; 2048 queries of
 // 656-B rows, H = 32, 549 instead of 835.  Against 128-head workgroups (the other
 // 64 or more heads padding): MXFP8, 128 tokens x 2048 rows, H = 16, 67 instead of
@@ -3657,7 +3668,7 @@ constexpr int COMBINE_MAX_Y = 65535;     // the grid's y extent (HIP's limit is 
 // CU (four heads per workgroup put C1's 256 (row, head) pairs on 64 CUs, each
 // pulling 128 KB of partials through its own memory path).  Past
 // COMBINE_MAX_Y heads a workgroup takes every gridDim.y-th head.
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(64) __attribute__((aligned(16384)))
 dsa_mla_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ part_lse, int ns,
                        int rows, int H, int s_q, __bf16* __restrict__ out, int64_t o_sb, int64_t o_st,
                        int64_t o_sh, float* __restrict__ lse, const float* __restrict__ sink) {
@@ -3739,7 +3750,7 @@ __device__ __forceinline__ void combine_head_wide(const float* __restrict__ part
 // partials at 4.9 TB/s, against 15.2 with a wave per head; 2 rows of 128 items of
 // 64 heads, where few waves hide their round trips: the whole call 44.5 us
 // against 61.6.
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256) __attribute__((aligned(16384)))
 dsa_mla_combine_plan_kernel(const float* __restrict__ part_o, const float* __restrict__ part_lse, int B, int H,
                             int s_q, int max_len, __bf16* __restrict__ out, int64_t o_sb, int64_t o_st,
                             int64_t o_sh, float* __restrict__ lse, const int4* __restrict__ map,
