@@ -30,7 +30,7 @@
 //   its token's rows (16 accumulator registers and one cross-half exchange per
 //   row block).  A slot is refilled as soon as its last fragment is in
 //   registers, before the epilogue; no barrier ties the waves together;
-// - HBM bounds it when each k row is read once: 117 us for those 570 MB (4.9
+// - HBM bounds it when each k row is read once: 114 us for those 570 MB (5.0
 //   TB/s, a plain copy moves 5.1), 131 us without the non-temporal mark on rows
 //   that a single group reads.  Many tokens on one sequence (512 tokens x 16 K
 //   positions) are bound by the MFMAs and the epilogue's two VALU instructions

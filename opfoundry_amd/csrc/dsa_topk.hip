@@ -602,7 +602,8 @@ __device__ __forceinline__ void emit_flags(TopkLds& s, uint32_t* flags, int D, b
 // positions took 69 us when they were counted into one bin).
 // What bounds it: 256 rows of 65,536 (67 MB) are loaded in about 17 us, with the
 // keys and the histogram under the loads; the threshold, the flags and the
-// output then run with the memory idle: 24.5 us in all.  Ranking every key
+// output then run with the memory idle: 24.1 to 24.8 us in all (three score sets in
+// turn; 26 with five, 320 MB, more than the MALL holds).  Ranking every key
 // against ballots, prefix tables and a slot per key took 35.2 us; flags cost two
 // to three instructions per key, and only taken positions pay for a slot.
 // ---------------------------------------------------------------------------
