@@ -63,6 +63,13 @@ def test_every_chunk_once_and_even(lib, chunks, G):
         assert taken.max() <= -(-chunks.sum() // G)
 
 
+@pytest.mark.parametrize("groups,chunks,G", [(4, 512, 512), (128, 128, 512), (128, 24, 512), (512, 17, 512), (1, 2048, 512)])
+def test_equal_groups_in_equal_runs(lib, groups, chunks, G):
+    """Equal groups that divide into as many equal runs each are cut that way, no run across two."""
+    seen, taken, begun = walk(lib, [chunks] * groups, G)
+    assert (seen == 1).all() and (taken == groups * chunks // G).all() and (begun == 1).all()
+
+
 def test_random_deals(lib):
     rng = np.random.default_rng(5)
     for i in range(400):
