@@ -3992,8 +3992,9 @@ double kern_time(int fmt, Kern k, int64_t tokens, int32_t H, int64_t list, int n
 // both places of every CU.  Of 3556 calls measured with every kernel and count, the
 // choice is 0.1 % slower than the fastest such one on average, more than 3 % in 45 and
 // 7 % at most (bf16, 40 to 64 heads, 70 to 85 tokens x 1700 to 2048: 64 heads in 3
-// splits, 32 heads in 3 are 3 to 4 % faster).  At up to 64 heads 128-head workgroups win where the count given leaves them in one round (V4
-// fp8 rows, 160 tokens of 64 heads x 2048 unsplit 153 us, 164 in 64 heads, 177 in 32).
+// splits, 32 heads in 3 are 3 to 4 % faster).  At up to 64 heads 128-head workgroups
+// win where the count given leaves them in one round (V4 fp8 rows, 160 tokens of 64
+// heads x 2048 unsplit 153 us, 164 in 64 heads, 177 in 32).
 // NARROW is for one round at most: past it, a second workgroup per CU covers the first
 // one's waits.  Beyond 64 heads PAIR is only for what NARROW cannot hold in a round
 // (its head groups lie 8 apart, which costs where splits of 8 or 16 tokens meet on an
