@@ -75,6 +75,23 @@ def test_decode_edges_and_restart(dev, H, fp8, spike):
     assert_parity(o, l, o_ref, l_ref, f"pair decode H={H} fp8={fp8} spike={spike}")
 
 
+@pytest.mark.parametrize("H,tokens,fp8", [(96, 7, False), (100, 5, True), (128, 5, False), (128, 6, True)])
+def test_three_and_four_head_groups(dev, H, tokens, fp8):
+    """Beyond 64 heads a split call of few tokens runs 32-head workgroups, two per CU where one
+    round does not hold them (16 splits here: 320 workgroups and more)."""
+    print(f"[case] pair decode of {tokens} tokens H={H} fp8={fp8}", flush=True)
+    q, kv, idx, sl = (x[:tokens] if i != 1 else x for i, x in enumerate(shared_case(570 + H, H, fp8)))
+    for b, n in enumerate([2048, 0, 1999, 33, 769, 16, 1537][:tokens]):
+        idx[b, 0, :n] = np.random.default_rng(b).permutation(4096)[:n]
+        idx[b, 0, n:] = -1
+    kvt = torch.from_numpy(kv).to(dev) if fp8 else t16(kv, dev)
+    out, lse = dsa.mla_decode(t16(q, dev), kvt, torch.from_numpy(idx).to(dev), SM_SCALE,
+                              seq_lens=torch.from_numpy(sl).to(dev), num_splits=16)
+    torch.cuda.synchronize()
+    o_ref, l_ref = oracle.mla_decode(q, kv, idx, sl, SM_SCALE)
+    assert_parity(bits(out), lse.cpu().numpy(), o_ref, l_ref, f"pair decode of {tokens} tokens H={H} fp8={fp8}")
+
+
 def test_bad_scale_is_nan(dev):
     print("[case] pair fp8 bad scale", flush=True)
     q, kv, idx, sl = shared_case(520, 16, True)
